@@ -263,7 +263,7 @@ __global__ __launch_bounds__(256) void sl_accumulate_kernel(
       double c1, s1;
       planar_angle(x, y, c1, s1);
       if (h == 0) {
-        SLCell cell = sl_locate(r, g.cmap, g.scale, g.xi, g.numr, g.idxi);
+        SLCell cell = sl_locate(r, g.cmap, g.scale, g.xi, g.numr, g.idxi, g.xi0, g.xin);
         const double P0 = cell.x1 * g.p0[cell.i] + cell.x2 * g.p0[cell.i + 1];
         s_i[qp] = cell.i;
         s_w1[qp] = live ? (float)(cell.x1 * P0) : 0.f;
@@ -789,7 +789,7 @@ __device__ __forceinline__ void sl_deposit_body(
         const double costh = z / r;
         double c1, s1v;
         planar_angle(x, y, c1, s1v);
-        const SLCell cell = sl_locate(r, g.cmap, g.scale, g.xi, g.numr, g.idxi);
+        const SLCell cell = sl_locate(r, g.cmap, g.scale, g.xi, g.numr, g.idxi, g.xi0, g.xin);
         const double P0 = cell.x1 * g.p0[cell.i] + cell.x2 * g.p0[cell.i + 1];
         ci = cell.i;
         w1 = live ? (float)(cell.x1 * P0) : 0.f;
@@ -1046,7 +1046,7 @@ __global__ __launch_bounds__(256) void sl_mfma_kernel(
         double c1, s1v;
         planar_angle(x, y, c1, s1v);
         if (h == 0) {
-          SLCell cell = sl_locate(r, g.cmap, g.scale, g.xi, g.numr, g.idxi);
+          SLCell cell = sl_locate(r, g.cmap, g.scale, g.xi, g.numr, g.idxi, g.xi0, g.xin);
           const double P0 = cell.x1 * g.p0[cell.i] + cell.x2 * g.p0[cell.i + 1];
           s_i[qp] = cell.i;
           s_w1[qp] = live ? (float)(cell.x1 * P0) : 0.f;

@@ -270,6 +270,11 @@ extern "C" int bfe_sl_tables_set(bfe_ctx* h, int lmax, int nmax, int numr, int c
       lmc[kLmcNB + lm] = l - 2 >= m ? lmc[kLmcB + lm] * y / lmc[kLmcY + lm_index(l - 2, m)] : 0.0;
     }
   }
+  for (int m = 0, p = 0; m <= kMaxL; ++m)
+    for (int l = m; l <= kMaxL; ++l, ++p) {
+      lmc[kLmcAB + 2 * p] = lmc[kLmcA + lm_index(l, m)];
+      lmc[kLmcAB + 2 * p + 1] = lmc[kLmcB + lm_index(l, m)];
+    }
   int rc;
   if ((rc = dev_upload(c, &c->sl_lmc, lmc.data(), lmc.size()))) return rc;
   if ((rc = dev_upload(c, &c->sl_xi, xi, numr))) return rc;
@@ -387,6 +392,9 @@ extern "C" int bfe_set_tuning(bfe_ctx* h, const char* name, int64_t value) {
   } else if (!strcmp(name, "order_min")) {
     if (value < 0) return set_error(c, BFE_EINVAL, "order_min < 0");
     c->order_min = value;
+  } else if (!strcmp(name, "split_max") || !strcmp(name, "split_eval_max")) {
+    if (value < 0) return set_error(c, BFE_EINVAL, "%s < 0", name);
+    (name[5] == '_' && name[6] == 'm' ? c->split_max : c->split_eval_max) = value;
   } else if (!strcmp(name, "kernel_timing")) {
     c->kernel_timing = value != 0;
   } else if (!strcmp(name, "sl_acc_path")) {
@@ -418,6 +426,8 @@ extern "C" int bfe_get_tuning(const bfe_ctx* h, const char* name, int64_t* value
   else if (!strcmp(name, "eof_seg_tiles")) *value = c->eof_seg_tiles;
   else if (!strcmp(name, "sl_seg_tiles")) *value = c->sl_seg_tiles;
   else if (!strcmp(name, "order_min")) *value = c->order_min;
+  else if (!strcmp(name, "split_max")) *value = c->split_max;
+  else if (!strcmp(name, "split_eval_max")) *value = c->split_eval_max;
   else if (!strcmp(name, "kernel_timing")) *value = c->kernel_timing ? 1 : 0;
   else if (!strcmp(name, "sl_acc_path")) *value = c->sl_acc_path;
   else if (!strcmp(name, "eof_dep_shape")) *value = c->eof_dep_shape;

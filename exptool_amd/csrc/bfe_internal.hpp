@@ -30,11 +30,13 @@ constexpr int kMaxLM = (kMaxL + 1) * (kMaxL + 2) / 2;
 //   [kLmcNA + lm], [kLmcNB + lm]  the same recurrence for Q_l^m = -4 pi N_lm
 //                 P_l^m:  Q_l^m = x A N_lm/N_{l-1,m} Q_{l-1}^m
 //                                 - B N_lm/N_{l-2,m} Q_{l-2}^m
+//   [kLmcAB + 2 p] A, B of pair p in m-major order (m = 0..kMaxL, l = m..kMaxL)
 //   [kLmcN0 + m]  -4 pi N_mm (-1)^m (2m - 1)!!   Q_m^m = N0_m (1 - x^2)^{m/2}
 constexpr int kLmcY = 0, kLmcA = kMaxLM, kLmcB = 2 * kMaxLM, kLmcD = 3 * kMaxLM;
 constexpr int kLmcL = 3 * kMaxLM + kMaxL + 1, kLmcS = kLmcL + kMaxLM;
 constexpr int kLmcNA = kLmcS + kMaxLM, kLmcNB = kLmcNA + kMaxLM, kLmcN0 = kLmcNB + kMaxLM;
-constexpr int kLmcSize = kLmcN0 + kMaxL + 1;
+constexpr int kLmcAB = (kLmcN0 + kMaxL + 2) / 2 * 2;   // 16-byte aligned
+constexpr int kLmcSize = kLmcAB + 2 * kMaxLM;
 
 // Row length of the padded deposit tables: radial orders rounded up to a
 // multiple of 48, so that for every chunk length of the lane shapes (2, 4, 8,
@@ -159,7 +161,10 @@ struct Context {
   int64_t sl_acc_blocks_beside = 1024;
   int64_t eof_seg_tiles = 0;       // batch accumulate: tiles per segment, 0 = from the budget
   int64_t sl_seg_tiles = 0;
-  int64_t order_min = 65536;       // evaluate in cell order from this many points
+  int64_t order_min = 65536;       // accumulate in cell order from this many particles,
+                                   // evaluate in it from twice as many points
+  int64_t split_max = 36864;       // orbits up to which the split integrators run
+  int64_t split_eval_max = 131072; // points up to which the split evaluation runs
   int64_t sl_acc_path = 0;         // SL accumulate: 0 auto (vector ALU), 1 MFMA, 2 vector ALU
   int64_t eof_dep_shape = -1;      // cell-ordered EOF accumulate lane shape (index), -1 auto
   int64_t sl_dep_shape = -1;       // cell-ordered SL accumulate lane shape (index), -1 auto
@@ -200,6 +205,7 @@ struct SLGeom {
   int numr, cmap, lmax, nmax;
   double scale;
   const double* lmc;   // Context::sl_lmc
+  double xi0, xin;     // xi[0], xi[numr - 1]
   double idxi;         // 1 / (xi[1] - xi[0])
   double dfac;         // cmap 1: 0.5 / (scale (xi[1] - xi[0])), d xi/d r over the step
 };
@@ -231,7 +237,8 @@ __host__ __device__ inline int eof_edge_index(int X, int Y, int numx, int numy) 
 inline SLGeom sl_geom(const Context* c) {
   const double dxi = c->h_xi.size() >= 2 ? c->h_xi[1] - c->h_xi[0] : 1.0;
   return SLGeom{c->sl_xi, c->sl_p0, c->sl_d0, c->numr, c->cmap, c->lmax, c->nmax, c->scale,
-                c->sl_lmc, 1.0 / dxi, 0.5 / (c->scale * dxi)};
+                c->sl_lmc, c->h_xi.empty() ? 0.0 : c->h_xi.front(),
+                c->h_xi.empty() ? 0.0 : c->h_xi.back(), 1.0 / dxi, 0.5 / (c->scale * dxi)};
 }
 inline EOFGeom eof_geom(const Context* c) {
   return EOFGeom{c->ecmap, c->numx, c->numy, c->mmax, c->norder, c->ascale, c->hscale,
@@ -281,6 +288,8 @@ int sl_accumulate_one(Context* c, const float* x, const float* y, const float* z
 // float64 per-point scratch in the ordering buffer (n entries), valid after
 // order_points for the same n.
 double* order_energy_buffer(Context* c, int64_t n);
+// Sizes the ordering buffer for n points (for order_energy_buffer without a sort).
+int order_reserve(Context* c, int64_t n);
 // Release the ordering buffer (bfe_destroy).
 void order_free(Context* c);
 // Release the batched-field buffers (bfe_destroy).

@@ -183,6 +183,100 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void l
   }
 }
 
+// The same steps with the field evaluated by split blocks (field_eval_split:
+// 64 orbits, eight waves sharing the orders) for orbit counts that leave the
+// one-lane kernel latency-bound (up to split_max: one orbit 7.9 -> 2.8 us a
+// step, 12 800 orbits 14.6 -> 4.5, 36k orbits 12.4 and 12.4; RK4 of 20 000
+// orbits 15.5 -> 8.4 us an evaluation).  A block's eight waves fill a CU at
+// 156 registers; at four waves per SIMD (128, 120 B spilled) one orbit took
+// 3.3 us.  Every wave carries the state of the block's
+// orbits and advances it alike; wave w writes component w of the records.
+// init: step k0 first (initial acceleration, energy and record 0), in place
+// of leapfrog_init_kernel.  perm NULL: orbit j in lane j.
+template <bool PER_ORBIT, int LM, int MM>
+__global__ __launch_bounds__(kSplitThreads) __attribute__((amdgpu_waves_per_eu(2))) void leapfrog_split_kernel(
+    float* __restrict__ x, float* __restrict__ y, float* __restrict__ z, float* __restrict__ vx,
+    float* __restrict__ vy, float* __restrict__ vz, const int* __restrict__ perm, FieldTables T,
+    LeapArgs a, int init, OrbitAux* __restrict__ aux, double* __restrict__ ebuf,
+    float* __restrict__ traj) {
+  extern __shared__ __align__(16) double split_sm[];
+  const SplitWave w = split_wave();
+  const int64_t j = xcd_block(a.nblocks) * kSplitPts + w.lane;
+  if (j - w.lane >= a.n) return;   // whole block past the end (XCD mapping)
+  const bool live = j < a.n;
+  const int64_t i = live ? (perm ? (int64_t)perm[j] : j) : 0;
+  float px = 1.f, py = 0, pz = 0, ux = 0, uy = 0, uz = 0, ax = 0, ay = 0, az = 0;
+  double dtd = a.dt;
+  if (live) {
+    px = x[i]; py = y[i]; pz = z[i];
+    ux = vx[i]; uy = vy[i]; uz = vz[i];
+    if (!init) {
+      const float4 acc = *reinterpret_cast<const float4*>(&aux[i].ax);
+      ax = acc.x; ay = acc.y; az = acc.z;
+    }
+    if (PER_ORBIT) dtd = a.dtv[i];
+  }
+  const float dt = (float)dtd;
+  const float hdt2 = 0.5f * dt * dt;
+  const float hdt = 0.5f * dt;
+  float pot = 0.f;
+  double e0 = 0.0;
+  const size_t n = (size_t)a.n;
+  for (int64_t k = init ? a.k0 : a.k0 + 1; k <= a.k1; ++k) {
+    const bool first = k == a.k0;
+    if (live && !first) {
+      // integrate.py:129-143
+      px = px + ux * dt + ax * hdt2;
+      py = py + uy * dt + ay * hdt2;
+      pz = pz + uz * dt + az * hdt2;
+    }
+    rot_of(a, dtd, k, T);
+    double cv[8];
+    field_eval_split<LM, MM>(T, px, py, pz, w, split_sm, cv);
+    const float nx = (float)(cv[0] + cv[1]), ny = (float)(cv[2] + cv[3]), nz = (float)(cv[4] + cv[5]);
+    pot = (float)(cv[6] + cv[7]);
+    if (live && !first) {
+      ux = ux + (ax + nx) * hdt;
+      uy = uy + (ay + ny) * hdt;
+      uz = uz + (az + nz) * hdt;
+    }
+    ax = nx; ay = ny; az = nz;
+    if (first) e0 = 0.5 * ((double)ux * ux + (double)uy * uy + (double)uz * uz) + (double)pot;
+    if (live && traj && (first || (a.record_every > 0 && (k % a.record_every) == 0))) {
+      float* t = traj + (size_t)(first ? 0 : k / a.record_every) * 7 * n + i;
+      if (w.wave == 0) t[0] = px;
+      if (w.wave == 1) t[n] = py;
+      if (w.wave == 2) t[2 * n] = pz;
+      if (w.wave == 3) t[3 * n] = ux;
+      if (w.wave == 4) t[4 * n] = uy;
+      if (w.wave == 5) t[5 * n] = uz;
+      if (w.wave == 6) t[6 * n] = pot;
+    }
+  }
+  __syncthreads();   // every wave has read its state before wave 0 rewrites it
+  if (live && w.wave == 0) {
+    x[i] = px; y[i] = py; z[i] = pz;
+    vx[i] = ux; vy[i] = uy; vz[i] = uz;
+    OrbitAux o;
+    if (init) {
+      o.pad = 0.f;
+      o.e0 = e0;
+      o.drift = 0.0;
+      if (ebuf && a.k1 == a.k0) ebuf[i] = e0;
+    } else {
+      o = aux[i];
+    }
+    o.ax = ax; o.ay = ay; o.az = az;
+    if (a.energy_every > 0 && a.k1 > a.k0) {
+      const double e = 0.5 * ((double)ux * ux + (double)uy * uy + (double)uz * uz) + (double)pot;
+      const double rel = fabs(e - o.e0) / fabs(o.e0);
+      if (rel > o.drift || !(rel == rel)) o.drift = rel;
+      if (ebuf) ebuf[i] = e;
+    }
+    aux[i] = o;
+  }
+}
+
 // Block sums of the checkpoint energies over 256 consecutive orbits (input
 // order), fixed tree: partE[check * nblocks + b].
 __global__ __launch_bounds__(256) void energy_block_kernel(const double* __restrict__ ebuf,
@@ -256,8 +350,9 @@ __device__ __forceinline__ void rk4_frame(const RK4Args& a, float px, float py, 
                                           float& fx, float& fy) {
   if (a.omegab == 0.0) return;
   const float w = (float)a.omegab, s = (float)a.frame_sign;
-  fx += s * (w * w * px + 2.0f * w * uy);
-  fy += s * (w * w * py - 2.0f * w * ux);
+  const float w2 = w * w, tw = 2.0f * w;
+  fx = fmaf(s, fmaf(w2, px, tw * uy), fx);
+  fy = fmaf(s, fmaf(w2, py, -(tw * ux)), fy);
 }
 
 // Three waves per SIMD (168 registers, about 300 B per lane spilled):
@@ -320,6 +415,76 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void r
   }
 }
 
+// RK4 with the field evaluated by split blocks (as leapfrog_split_kernel).
+template <int LM, int MM>
+__global__ __launch_bounds__(kSplitThreads) __attribute__((amdgpu_waves_per_eu(2))) void rk4_split_kernel(
+    float* __restrict__ x, float* __restrict__ y, float* __restrict__ z, float* __restrict__ vx,
+    float* __restrict__ vy, float* __restrict__ vz, const int* __restrict__ perm, FieldTables T,
+    RK4Args a, float* __restrict__ traj) {
+  extern __shared__ __align__(16) double split_sm[];
+  const SplitWave w = split_wave();
+  const int64_t j = xcd_block(a.nblocks) * kSplitPts + w.lane;
+  if (j - w.lane >= a.n) return;   // whole block past the end (XCD mapping)
+  const bool live = j < a.n;
+  const int64_t i = live ? (perm ? (int64_t)perm[j] : j) : 0;
+  float px = 1.f, py = 0, pz = 0, ux = 0, uy = 0, uz = 0;
+  if (live) {
+    px = x[i]; py = y[i]; pz = z[i];
+    ux = vx[i]; uy = vy[i]; uz = vz[i];
+  }
+  const float h = (float)a.dt, hh = 0.5f * h, h6 = h / 6.0f;
+  const size_t n = (size_t)a.n;
+  for (int64_t k = a.k0 + 1; k <= a.k1; ++k) {
+    // rk4.py:48-60, one stage at a time: stage 0 at x, 1 and 2 at the half
+    // steps, 3 at the full step; the weighted sums grow stage by stage
+    float qx = px, qy = py, qz = pz, rx = ux, ry = uy, rz = uz;
+    float sfx = 0, sfy = 0, sfz = 0, srx = 0, sry = 0, srz = 0;
+#pragma unroll 1
+    for (int g = 0; g < 4; ++g) {
+      double cv[8];
+      field_eval_split<LM, MM>(T, qx, qy, qz, w, split_sm, cv);
+      float fx = (float)(cv[0] + cv[1]), fy = (float)(cv[2] + cv[3]);
+      const float fz = (float)(cv[4] + cv[5]);
+      rk4_frame(a, qx, qy, rx, ry, fx, fy);
+      if (g == 0) {
+        sfx = fx; sfy = fy; sfz = fz;
+        srx = rx; sry = ry; srz = rz;
+      } else if (g < 3) {
+        sfx = sfx + 2.0f * fx; sfy = sfy + 2.0f * fy; sfz = sfz + 2.0f * fz;
+        srx = srx + 2.0f * rx; sry = sry + 2.0f * ry; srz = srz + 2.0f * rz;
+      } else {
+        sfx = sfx + fx; sfy = sfy + fy; sfz = sfz + fz;
+        srx = srx + rx; sry = sry + ry; srz = srz + rz;
+      }
+      if (g < 3) {
+        const float hg = g < 2 ? hh : h;
+        qx = px + rx * hg; qy = py + ry * hg; qz = pz + rz * hg;
+        rx = ux + fx * hg; ry = uy + fy * hg; rz = uz + fz * hg;
+      }
+    }
+    if (live) {
+      px = px + h6 * srx;
+      py = py + h6 * sry;
+      pz = pz + h6 * srz;
+      ux = ux + h6 * sfx; uy = uy + h6 * sfy; uz = uz + h6 * sfz;
+      if (traj && a.record_every > 0 && (k % a.record_every) == 0) {
+        float* t = traj + (size_t)(k / a.record_every) * 6 * n + i;
+        if (w.wave == 0) t[0] = px;
+        if (w.wave == 1) t[n] = py;
+        if (w.wave == 2) t[2 * n] = pz;
+        if (w.wave == 3) t[3 * n] = ux;
+        if (w.wave == 4) t[4 * n] = uy;
+        if (w.wave == 5) t[5 * n] = uz;
+      }
+    }
+  }
+  __syncthreads();   // every wave has read its state before wave 0 rewrites it
+  if (live && w.wave == 0) {
+    x[i] = px; y[i] = py; z[i] = pz;
+    vx[i] = ux; vy[i] = uy; vz[i] = uz;
+  }
+}
+
 // Record 0 of an RK4 trajectory: the initial state.
 __global__ void rk4_record0_kernel(const float* __restrict__ x, const float* __restrict__ y,
                                    const float* __restrict__ z, const float* __restrict__ vx,
@@ -331,6 +496,12 @@ __global__ void rk4_record0_kernel(const float* __restrict__ x, const float* __r
     traj[3 * n + i] = vx[i]; traj[4 * n + i] = vy[i]; traj[5 * n + i] = vz[i];
   }
 }
+
+// Steps between the re-orderings of a split integration (their six launches
+// cost as much as ten steps), and the orbits from which it is ordered at all:
+// below, the blocks are fewer than 32 and share no cells worth sorting for.
+constexpr int kSplitChunkSteps = 400;
+constexpr int64_t kSplitOrderMin = 2048;
 
 }  // namespace bfe
 
@@ -357,7 +528,9 @@ static int leapfrog_run(bfe_ctx* h, float* x, float* y, float* z, float* vx, flo
   BFE_HIP(c, hipSetDevice(c->device));
   hipStream_t s = (hipStream_t)stream;
   const int nb = (int)((n + 255) / 256);
-  const int chunk = energy_every > 0 ? energy_every : (int)std::min<int64_t>(nsteps > 0 ? nsteps : 1, 100);
+  const bool split = n <= c->split_max && split_ok(T);
+  const int64_t plain = split ? kSplitChunkSteps : 100;
+  const int chunk = energy_every > 0 ? energy_every : (int)std::min<int64_t>(nsteps > 0 ? nsteps : 1, plain);
   const int nchecks = energy_every > 0 ? (int)(nsteps / energy_every) + 1 : 1;
   const size_t aux_bytes = (size_t)n * sizeof(OrbitAux);
   const size_t part_bytes = (size_t)nchecks * nb * sizeof(double);
@@ -368,10 +541,17 @@ static int leapfrog_run(bfe_ctx* h, float* x, float* y, float* z, float* vx, flo
   // cell order of the initial positions, rebuilt from the current positions
   // before every chunk
   const int* perm = nullptr;
-  rc = order_points(c, T, x, y, z, n, s, &perm);
+  const bool ordered = !split || n >= kSplitOrderMin;
+  if (ordered) {
+    rc = order_points(c, T, x, y, z, n, s, &perm);
+  } else if (energy_log) {
+    rc = order_reserve(c, n);   // the energy buffer only
+  }
   if (rc) return rc;
   double* ebuf = energy_log ? order_energy_buffer(c, n) : nullptr;
-  const unsigned grid = xcd_grid(nb);
+  const int sb = (int)((n + kSplitPts - 1) / kSplitPts);
+  const unsigned grid = xcd_grid(split ? sb : nb);
+  const size_t slds = (size_t)split_lds_doubles(c->mmax, c->lmax) * sizeof(double);
   LeapArgs a;
   a.dt = dt;
   a.dtv = dtv;
@@ -383,9 +563,27 @@ static int leapfrog_run(bfe_ctx* h, float* x, float* y, float* z, float* vx, flo
   a.energy_every = energy_every;
   a.check0 = 0;
   a.record_every = record_every;
-  a.nblocks = nb;
-  hipLaunchKernelGGL(leapfrog_init_kernel, dim3(grid), dim3(256), 0, s, x, y, z, vx, vy, vz, perm,
-                     T, a, aux, ebuf, traj);
+  a.nblocks = split ? sb : nb;
+  // the split form takes step 0 with its first chunk unless the energies of
+  // step 0 are wanted by themselves
+  const bool merged = split && !ebuf;
+  auto launch_split = [&](const LeapArgs& b, int init, double* eb) {
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(grid), dim3(kSplitThreads), slds, s, x, y, z, vx, vy, vz, perm,
+                         T, b, init, aux, eb, traj);
+    };
+    const bool fixed = c->lmax == 6 && c->mmax == 6;
+    if (dtv && fixed) go(leapfrog_split_kernel<true, 6, 6>);
+    else if (dtv) go(leapfrog_split_kernel<true, -1, -1>);
+    else if (fixed) go(leapfrog_split_kernel<false, 6, 6>);
+    else go(leapfrog_split_kernel<false, -1, -1>);
+  };
+  if (split) {
+    if (!merged || nsteps == 0) launch_split(a, 1, ebuf);
+  } else {
+    hipLaunchKernelGGL(leapfrog_init_kernel, dim3(grid), dim3(256), 0, s, x, y, z, vx, vy, vz, perm,
+                       T, a, aux, ebuf, traj);
+  }
   if (ebuf)
     hipLaunchKernelGGL(energy_block_kernel, dim3(nb), dim3(256), 0, s, ebuf, n, partE);
   BFE_HIP(c, hipGetLastError());
@@ -406,7 +604,7 @@ static int leapfrog_run(bfe_ctx* h, float* x, float* y, float* z, float* vx, flo
   for (const LeapArgs& b : chunks) {
     // re-sort by the current cells between chunks (the sort allocates
     // nothing here: the buffer was sized by the first sort, before any capture)
-    if (b.k0 > 0) {
+    if (b.k0 > 0 && ordered) {
       rc = order_points(c, T, x, y, z, n, s, &perm);
       if (rc) {
         // leave the caller's stream out of capture mode
@@ -416,7 +614,9 @@ static int leapfrog_run(bfe_ctx* h, float* x, float* y, float* z, float* vx, flo
       }
     }
     const bool check = ebuf && b.energy_every > 0;
-    if (dtv)
+    if (split)
+      launch_split(b, merged && b.k0 == 0, check ? ebuf : nullptr);
+    else if (dtv)
       hipLaunchKernelGGL(leapfrog_chunk_kernel<true>, dim3(grid), dim3(256), 0, s, x, y, z, vx, vy,
                          vz, perm, T, b, aux, check ? ebuf : nullptr, traj);
     else
@@ -487,8 +687,12 @@ extern "C" int bfe_rk4(bfe_ctx* h, float* x, float* y, float* z, float* vx, floa
   if (n == 0) return 0;
   BFE_HIP(c, hipSetDevice(c->device));
   hipStream_t s = (hipStream_t)stream;
+  const bool split = n <= c->split_max && split_ok(T);
+  const bool ordered = !split || n >= kSplitOrderMin;
   const int nb = (int)((n + 255) / 256);
-  const unsigned grid = xcd_grid(nb);
+  const int sb = (int)((n + kSplitPts - 1) / kSplitPts);
+  const unsigned grid = xcd_grid(split ? sb : nb);
+  const size_t slds = (size_t)split_lds_doubles(c->mmax, c->lmax) * sizeof(double);
   if (traj)
     hipLaunchKernelGGL(rk4_record0_kernel, dim3(nb), dim3(256), 0, s, x, y, z, vx, vy, vz, n, traj);
   RK4Args a;
@@ -497,16 +701,25 @@ extern "C" int bfe_rk4(bfe_ctx* h, float* x, float* y, float* z, float* vx, floa
   a.frame_sign = (flags & BFE_COMPAT_RK4_FRAME) ? -1 : 1;
   a.n = n;
   a.record_every = record_every;
-  a.nblocks = nb;
+  a.nblocks = split ? sb : nb;
   // chunks of 25 steps (100 field evaluations), re-sorted by cell in between
-  const int64_t chunk = 25;
+  const int64_t chunk = split ? kSplitChunkSteps / 4 : 25;
   for (int64_t k0 = 0; k0 < nsteps; k0 += chunk) {
     const int* perm = nullptr;
-    rc = order_points(c, T, x, y, z, n, s, &perm);
-    if (rc) return rc;
+    if (ordered) {
+      rc = order_points(c, T, x, y, z, n, s, &perm);
+      if (rc) return rc;
+    }
     a.k0 = k0;
     a.k1 = std::min<int64_t>(nsteps, k0 + chunk);
-    hipLaunchKernelGGL(rk4_chunk_kernel, dim3(grid), dim3(256), 0, s, x, y, z, vx, vy, vz, perm, T,
+    if (split && c->lmax == 6 && c->mmax == 6)
+      hipLaunchKernelGGL((rk4_split_kernel<6, 6>), dim3(grid), dim3(kSplitThreads), slds, s, x, y, z,
+                         vx, vy, vz, perm, T, a, traj);
+    else if (split)
+      hipLaunchKernelGGL((rk4_split_kernel<-1, -1>), dim3(grid), dim3(kSplitThreads), slds, s, x, y, z,
+                         vx, vy, vz, perm, T, a, traj);
+    else
+      hipLaunchKernelGGL(rk4_chunk_kernel, dim3(grid), dim3(256), 0, s, x, y, z, vx, vy, vz, perm, T,
                        a, traj);
   }
   BFE_HIP(c, hipGetLastError());

@@ -201,9 +201,11 @@ struct SLCell {
   double x1, x2;
 };
 
-// idxi = 1 / (xi[1] - xi[0]).
-BFE_HD SLCell sl_locate(double r, int cmap, double scale, const double* xi, int numr,
-                        double idxi) {
+// The cell and the mapped coordinate without the weights, which need the
+// table: idxi = 1 / (xi[1] - xi[0]); xi0, xin: the first and last of xi (by
+// value, so that the cell index waits for no read).
+BFE_HD SLCell sl_cell_index(double r, int cmap, double scale, int numr, double idxi, double xi0,
+                            double xin) {
   SLCell c;
   double x = r_to_xi(r, cmap, scale);
   if (cmap == 1) {
@@ -211,10 +213,10 @@ BFE_HD SLCell sl_locate(double r, int cmap, double scale, const double* xi, int 
     if (x >= 1.0) x = 1.0 - 1.0e-08;
   } else if (cmap == 2) {
     // intended semantics of spheresl.py:128-130 (NameError as written)
-    if (!(x >= xi[0])) x = xi[0];
-    if (x > xi[numr - 1]) x = xi[numr - 1];
+    if (!(x >= xi0)) x = xi0;
+    if (x > xin) x = xin;
   }
-  double f = floor((x - xi[0]) * idxi);
+  double f = floor((x - xi0) * idxi);
   int i;
   if (!(f == f)) i = 0;
   else if (f < 0.0) i = 0;
@@ -222,8 +224,17 @@ BFE_HD SLCell sl_locate(double r, int cmap, double scale, const double* xi, int 
   else i = (int)f;
   c.x = x;
   c.i = i;
-  c.x1 = (xi[i + 1] - x) * idxi;
-  c.x2 = (x - xi[i]) * idxi;
+  c.x1 = c.x2 = 0.0;
+  return c;
+}
+BFE_HD void sl_cell_weights(SLCell& c, const double* xi, double idxi) {
+  c.x1 = (xi[c.i + 1] - c.x) * idxi;
+  c.x2 = (c.x - xi[c.i]) * idxi;
+}
+BFE_HD SLCell sl_locate(double r, int cmap, double scale, const double* xi, int numr,
+                        double idxi, double xi0, double xin) {
+  SLCell c = sl_cell_index(r, cmap, scale, numr, idxi, xi0, xin);
+  sl_cell_weights(c, xi, idxi);
   return c;
 }
 

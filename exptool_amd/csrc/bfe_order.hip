@@ -676,6 +676,10 @@ double* order_energy_buffer(Context* c, int64_t n) {
   return (double*)((char*)c->order + order_layout(n, sort_tiles(n), 1).energy);
 }
 
+int order_reserve(Context* c, int64_t n) {
+  return ensure_order(c, order_layout(n, sort_tiles(n), 1).total);
+}
+
 void order_free(Context* c) {
   if (c->order) (void)hipFree(c->order);
   c->order = nullptr;

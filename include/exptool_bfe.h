@@ -290,9 +290,13 @@ int bfe_field_eval_batch(bfe_ctx* ctx, const float* x, const float* y, const flo
  * 0 = derived from the budget), "eof_dep_shape" (0..7), "sl_dep_shape" (0..6)
  * (lane shape of the cell-ordered accumulate kernels, -1 = automatic; a
  * shape that does not fit the tables falls back to the automatic one),
- * "order_min" (points from which evaluation runs in table-cell order, 65536).
- * Results do not depend on "order_min"; accumulate sums depend on the segment
- * plan and the lane shape only through the float32 partial sums. */
+ * "order_min" (particles from which the accumulates run in table-cell order,
+ * and half the points from which evaluation does, 65536), "split_max" and
+ * "split_eval_max" (orbits, unordered points up to which the field is
+ * evaluated by split blocks, several waves per 64 points; 36864, 131072).
+ * Evaluation and orbits do not depend on these; accumulate sums depend on
+ * "order_min", the segment plan and the lane shape only through the float32
+ * partial sums. */
 int bfe_set_tuning(bfe_ctx* ctx, const char* name, int64_t value);
 int bfe_get_tuning(const bfe_ctx* ctx, const char* name, int64_t* value);
 /* With tuning knob "kernel_timing" = 1, the main compute kernel of
