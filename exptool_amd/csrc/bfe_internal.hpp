@@ -70,7 +70,7 @@ constexpr int kMaxMN = 4;
 constexpr int kMLPBaseMax = 4 + 3 * kMaxMN;
 
 // MLP surrogate state (float32 masters, bf16 MFMA operand copies, Adam moments
-// and the per-batch training buffers).
+// and the partial sums of a gradient).
 struct MLPState {
   float* params = nullptr;
   float* grads = nullptr;
@@ -78,13 +78,10 @@ struct MLPState {
   float* v = nullptr;
   __bf16* Wp = nullptr;
   __bf16* Wt = nullptr;
-  float* feat = nullptr;
-  float* Z = nullptr;
-  float* gZ = nullptr;
-  float* gY = nullptr;
-  float* dwpart = nullptr;
-  double* loss_part = nullptr;
-  int64_t bcap = 0;
+  float* dwpart = nullptr;       // per 128-point tile: partial sums of dW1..dW3
+  float* small_wave = nullptr;   // per tile and wave: of the other gradients
+  double* small_part = nullptr;  // per training block: these and the loss
+  int64_t bcap = 0;              // tiles these hold
   int64_t step = 0;
   double cfg[11] = {1, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0};
   double base[kMLPBaseMax] = {0};   // no base: nmn 0, Mh 0, phi0 0

@@ -55,19 +55,13 @@ constexpr int kSmallFloats = kH * kNIn + 4 * kH + kNOut * kH + kNOut;  // W0, b0
 #endif
 constexpr int kNT = BFE_MLP_NT;                  // 16-point N-tiles per wave
 constexpr int kWaveTile = 16 * kNT;              // points per wave
-// Threads per block.  The inference and integrator kernels run 8 waves on
-// one copy of the LDS weights (two waves per SIMD hide the SiLU latency);
-// the training kernels keep 4 waves, whose stores of the intermediates need
-// the registers.
+// Threads per block of the inference and integrator kernels: 8 waves on one
+// copy of the LDS weights (two waves per SIMD hide the SiLU latency).
 constexpr int kBlockInf = BFE_MLP_BLOCK;
-constexpr int kBlockTrain = 256;
+constexpr int kInfPts = kWaveTile * kBlockInf / 64;   // points per block
 // The conservative-field kernels carry three tangent operand sets beside the
 // activations: four waves per block, one per SIMD, keep them in registers.
 constexpr int kBlockGrad = 256;
-template <bool TRAIN>
-constexpr int block_threads() { return TRAIN ? kBlockTrain : kBlockInf; }
-template <bool TRAIN>
-constexpr int block_points() { return kWaveTile * block_threads<TRAIN>() / 64; }
 // LDS copy of the three hidden weight matrices: rows of kH bf16 padded to
 // kLdsRow.  A lane reads 16 bytes of row 16 mt + c; unpadded (256-byte)
 // rows put the rows that one read cycle serves on the same four banks, with
@@ -158,19 +152,9 @@ struct MLPKArgs {
   const float* y;
   const float* z;
   int64_t n;
-  const float* target;   // [4][n] normalised targets (training)
-  const float* weight;   // [n] per-point loss weight or NULL
-  float* out;            // [4][n] physical outputs (inference)
-  float* feat;           // [3][bcap]
-  float* Z;              // [4][128][bcap] pre-activations of layers 1..4
-  float* gZ;             // [4][128][bcap]
-  float* gY;             // [4][bcap]
-  int64_t bcap;
+  float* out;            // [4][n] physical outputs
   const float* params;
   const __bf16* Wp;      // [3][128][128] forward A operands (K-permuted)
-  const __bf16* Wt;      // [3][128][128] backward A operands (transposed, K-permuted)
-  double* loss_part;     // [gridDim.x]
-  float inv_n;
   MLPCfg cfg;
 };
 
@@ -219,39 +203,29 @@ __device__ __forceinline__ void hidden_mfma(const __bf16* __restrict__ sW, const
   }
 }
 
-// SiLU of hidden layer `layer`'s pre-activations acc: into the next layer's
-// bf16 operands B, or (LAST) in place as float32 for the output layer.
-// With TRAIN the pre-activations are stored to Z for points with valid[nt].
-template <bool TRAIN, bool LAST>
-__device__ __forceinline__ void forward_activate(floatx4 (&acc)[8][kNT], bf16x8 (&B)[4][kNT],
-                                                 float* Z, int64_t bcap,
-                                                 const int64_t (&pid)[kNT],
-                                                 const bool (&valid)[kNT], int layer, int g) {
+// SiLU of a hidden layer's pre-activations acc: into the next layer's bf16
+// operands B, or (LAST) in place as float32 for the output layer.
+template <bool LAST>
+__device__ __forceinline__ void forward_activate(floatx4 (&acc)[8][kNT], bf16x8 (&B)[4][kNT]) {
 #pragma unroll
   for (int mt = 0; mt < 8; ++mt)
 #pragma unroll
     for (int nt = 0; nt < kNT; ++nt)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float zz = acc[mt][nt][i];
-        if (TRAIN && valid[nt])
-          Z[((size_t)(layer + 1) * kH + 16 * mt + 4 * g + i) * bcap + pid[nt]] = zz;
-        const float hh = silu(zz);
-        if (LAST) acc[mt][nt][i] = hh;   // H4 in place (Z4 is reloaded in backward)
+        const float hh = silu(acc[mt][nt][i]);
+        if (LAST) acc[mt][nt][i] = hh;
         else B[mt >> 1][nt][(mt & 1) * 4 + i] = (__bf16)hh;
       }
 }
 
 // Forward pass of one wave tile (kNT x 16 points, column c of lane group g):
 // features f -> normalised outputs yk (all four lane groups of a column end
-// with the same yk).  With TRAIN the pre-activations are stored to Z
-// ([4][128][bcap]) for points with valid[nt].
-template <bool TRAIN>
+// with the same yk).
 __device__ __forceinline__ void mlp_tile_forward(const __bf16* __restrict__ sW,
                                                  const float* __restrict__ sS,
                                                  const float (&f)[kNT][3], float (&yk)[kNT][4],
-                                                 int g, int c, float* Z, int64_t bcap,
-                                                 const int64_t (&pid)[kNT], const bool (&valid)[kNT]) {
+                                                 int g, int c) {
   const float* sW0 = sS;
   const float* sB0 = sS + kH * kNIn;
   const float* sBh = sS + kH * kNIn + kH;           // b1, b2, b3
@@ -268,7 +242,6 @@ __device__ __forceinline__ void mlp_tile_forward(const __bf16* __restrict__ sW,
 #pragma unroll
       for (int nt = 0; nt < kNT; ++nt) {
         const float zz = fmaf(w0, f[nt][0], fmaf(w1, f[nt][1], fmaf(w2, f[nt][2], b)));
-        if (TRAIN && valid[nt]) Z[(size_t)nr * bcap + pid[nt]] = zz;
         B[kk][nt][j] = (__bf16)silu(zz);
       }
     }
@@ -278,10 +251,10 @@ __device__ __forceinline__ void mlp_tile_forward(const __bf16* __restrict__ sW,
 #pragma unroll 1
   for (int layer = 0; layer < 2; ++layer) {
     hidden_mfma(sW + layer * kLdsLayer, sBh + layer * kH, B, acc, g, c);
-    forward_activate<TRAIN, false>(acc, B, Z, bcap, pid, valid, layer, g);
+    forward_activate<false>(acc, B);
   }
   hidden_mfma(sW + 2 * kLdsLayer, sBh + 2 * kH, B, acc, g, c);
-  forward_activate<TRAIN, true>(acc, B, Z, bcap, pid, valid, 2, g);
+  forward_activate<true>(acc, B);
   // output layer (float32): partial sums over this lane's neurons, then
   // reduce over the four lane groups that hold the same point column
 #pragma unroll
@@ -440,26 +413,20 @@ __device__ __forceinline__ void conservative_field(const MLPCfg& cf, float x, fl
   pot = cf.os[0] * y0 + cf.ob[0] + bv[0];
 }
 
-// Forward pass over 32-point tiles per wave.  TRAIN also stores the
-// features and pre-activations, the loss and dL/dy.
-template <bool TRAIN>
-__global__ __launch_bounds__(block_threads<TRAIN>()) void mlp_fwd_kernel(MLPKArgs a) {
-  constexpr int kBlock = block_threads<TRAIN>(), kBlockPts = block_points<TRAIN>();
+// Forward pass over 32-point tiles per wave.
+__global__ __launch_bounds__(kBlockInf) void mlp_fwd_kernel(MLPKArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   __bf16* sW = reinterpret_cast<__bf16*>(smem);
   float* sS = reinterpret_cast<float*>(smem + kLdsWBytes);
-  __shared__ double s_loss[kBlock / 64];
-
   load_small(a.params, sS);
   load_weights(a.Wp, sW);
   __syncthreads();
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int g = lane >> 4, c = lane & 15;
-  double loss = 0.0;
-  const int64_t ntiles = (a.n + kBlockPts - 1) / kBlockPts;
+  const int64_t ntiles = (a.n + kInfPts - 1) / kInfPts;
   for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int64_t base = tile * kBlockPts + wave * kWaveTile;
+    const int64_t base = tile * kInfPts + wave * kWaveTile;
     int64_t pid[kNT];
     bool valid[kNT];
     float f[kNT][3];
@@ -469,49 +436,19 @@ __global__ __launch_bounds__(block_threads<TRAIN>()) void mlp_fwd_kernel(MLPKArg
       valid[nt] = pid[nt] < a.n;
       const int64_t q = valid[nt] ? pid[nt] : 0;
       mlp_features(a.cfg, a.x[q], a.y[q], a.z[q], f[nt]);
-      if (TRAIN && valid[nt] && g == 0)
-        for (int d = 0; d < 3; ++d) a.feat[d * a.bcap + pid[nt]] = f[nt][d];
     }
     float yk[kNT][4];
-    mlp_tile_forward<TRAIN>(sW, sS, f, yk, g, c, a.Z, a.bcap, pid, valid);
-    if (!TRAIN) {
+    mlp_tile_forward(sW, sS, f, yk, g, c);
 #pragma unroll
-      for (int nt = 0; nt < kNT; ++nt)
-        if (valid[nt] && g == 0) {
-          const float px = a.x[pid[nt]], py = a.y[pid[nt]];
-          float bv[4];
-          mlp_base_eval(a.cfg.base, sqrtf(px * px + py * py), a.z[pid[nt]], bv);
+    for (int nt = 0; nt < kNT; ++nt)
+      if (valid[nt] && g == 0) {
+        const float px = a.x[pid[nt]], py = a.y[pid[nt]];
+        float bv[4];
+        mlp_base_eval(a.cfg.base, sqrtf(px * px + py * py), a.z[pid[nt]], bv);
 #pragma unroll
-          for (int k = 0; k < 4; ++k)
-            a.out[(size_t)k * a.n + pid[nt]] = a.cfg.os[k] * yk[nt][k] + a.cfg.ob[k] + bv[k];
-        }
-      continue;
-    }
-    // ---- loss and backward ------------------------------------------------
-    float gy[kNT][4];
-#pragma unroll
-    for (int nt = 0; nt < kNT; ++nt) {
-      const float w = valid[nt] ? (a.weight ? a.weight[pid[nt]] : 1.f) : 0.f;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const float t = valid[nt] ? a.target[(size_t)k * a.n + pid[nt]] : 0.f;
-        const float d = valid[nt] ? yk[nt][k] - t : 0.f;
-        gy[nt][k] = 2.f * w * a.cfg.lw[k] * d * a.inv_n;
-        if (g == 0) loss += (double)(w * a.cfg.lw[k] * d * d);
-        if (valid[nt] && g == 0) a.gY[(size_t)k * a.bcap + pid[nt]] = gy[nt][k];
+        for (int k = 0; k < 4; ++k)
+          a.out[(size_t)k * a.n + pid[nt]] = a.cfg.os[k] * yk[nt][k] + a.cfg.ob[k] + bv[k];
       }
-    }
-  }
-  if (TRAIN) {
-    // fixed-order block sum of the loss
-    for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off);
-    if (lane == 0) s_loss[wave] = loss;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      double s = 0.0;
-      for (int w = 0; w < kBlock / 64; ++w) s += s_loss[w];
-      a.loss_part[blockIdx.x] = s;
-    }
   }
 }
 
@@ -550,188 +487,444 @@ __global__ __launch_bounds__(kBlockGrad) void mlp_fwd_grad_kernel(MLPKArgs a) {
   }
 }
 
-// Backward chain: gZ4 = (W4^T dL/dy) silu'(Z4), then gZ_l = (W_l^T gZ_{l+1})
-// silu'(Z_l) for l = 3, 2, 1, with the transposed K-permuted weights in LDS.
-__global__ __launch_bounds__(kBlockTrain) void mlp_bwd_kernel(MLPKArgs a) {
-  constexpr int kBlockPts = block_points<true>();
-  extern __shared__ __align__(16) unsigned char smem[];
-  __bf16* sW = reinterpret_cast<__bf16*>(smem);
-  float* sS = reinterpret_cast<float*>(smem + kLdsWBytes);
-  const float* sW4 = sS + kH * kNIn + 4 * kH;
-  load_small(a.params, sS);
-  load_weights(a.Wt, sW);
-  __syncthreads();
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int g = lane >> 4, c = lane & 15;
-  const int64_t ntiles = (a.n + kBlockPts - 1) / kBlockPts;
-  for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int64_t base = tile * kBlockPts + wave * kWaveTile;
-    int64_t pid[kNT];
-    bool valid[kNT];
-    float gy[kNT][4];
+// ---------------------------------------------------------------------------
+// Training: one kernel takes tiles of 128 points through the forward pass, the
+// loss, the backward chain and the weight gradients; a second one reduces the
+// blocks' partial sums.
+//
+// Eight waves of 16 points.  The pre-activations of the four layers stay in
+// registers (float32, 128 per lane: nothing but partial sums goes to memory;
+// as global arrays they were 134 MB written and read twice per 65 536 points).
+// The six weight operands W1, W2, W3, W3^T, W2^T, W1^T pass through two LDS
+// buffers, the next copied (global to LDS directly) while one is multiplied:
+// 16-byte chunk q of row r lies at q ^ (r mod 16), so the 16 rows a read
+// touches are on different banks without padding.
+// dW_l = gZ_{l+1} H_l^T sums over points, whose values lie across lanes: gZ
+// and H go to LDS as bf16 [point][neuron] and come back transposed
+// (ds_read_tr16: of a 16-lane group's 16 chunks of four neurons, lane l gets
+// neuron l of four points).  Wave w makes output rows 16 w .. 16 w + 15.  The
+// k order of the products is point 4 g + j, then 16 + 4 g + j, for lane group
+// g, in both operands.  The sums run in float32 over a tile and in float64
+// over tiles.  b0..b3, W0 and W4 gradients: float32 sums over the wave's 16
+// points by pairs (reduce_rows), float64 beyond.
+// Measured for 65 536 points: 910 us as separate forward, backward, weight
+// gradient and reduction kernels (72 + 200 + 337 + 63 + 197 + 41), 90 us for
+// this one and 16 for the reduction (100 MB of partial sums); about half of a
+// tile's 37 us is vector-ALU issue (SiLUs and the sums over lanes), the rest
+// waits of two waves per SIMD at 256 registers.
+constexpr int kTrainThreads = 512;
+constexpr int kTrainPts = 128;
+constexpr int kStageRow = kH + 16;   // bf16 per stage row: 8-row stride of 64 banks
+constexpr int kStageElems = kTrainPts * kStageRow;
+constexpr int kNSmall = kH * kNIn + 4 * kH + kNOut * kH + kNOut;   // gradients outside W1..W3
+constexpr int kSmallRow = kNSmall + 1;                             // and the loss
+constexpr size_t kTrainLds = (2 * (size_t)kH * kH + 2 * (size_t)kStageElems) * sizeof(__bf16) +
+                             kSmallFloats * sizeof(float);
+
+struct MLPTrainArgs {
+  const float* x;
+  const float* y;
+  const float* z;
+  const float* target;   // [4][n] normalised targets
+  const float* weight;   // [n] per-point loss weight or NULL
+  int64_t n;
+  int tiles;             // 128-point tiles per block
+  float inv_n;
+  const float* params;
+  const __bf16* Wp;
+  const __bf16* Wt;
+  float* dwpart;         // [tile][3][128][128]
+  float* small_wave;     // [tile][8 waves][11][128]
+  double* small_part;    // [block][kSmallRow]: dW0[d][nr], db0..db3, dW4, db4, loss
+  MLPCfg cfg;
+};
+
+typedef const void __attribute__((address_space(1)))* GlobalPtr;
+typedef void __attribute__((address_space(3)))* LdsPtr;
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef s16x4 __attribute__((address_space(3)))* LdsS4;
+
+// Starts the copy of one 128 x 128 weight operand into an LDS buffer (every
+// thread calls it; waited for by train_sync).
+__device__ __forceinline__ void train_load(const __bf16* __restrict__ W, __bf16* buf, int wave,
+                                           int lane) {
 #pragma unroll
-    for (int nt = 0; nt < kNT; ++nt) {
-      pid[nt] = base + 16 * nt + c;
-      valid[nt] = pid[nt] < a.n;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) gy[nt][k] = valid[nt] ? a.gY[(size_t)k * a.bcap + pid[nt]] : 0.f;
-    }
-    bf16x8 Bg[4][kNT];
-#pragma unroll
-    for (int mt = 0; mt < 8; ++mt)
-#pragma unroll
-      for (int nt = 0; nt < kNT; ++nt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int nr = 16 * mt + 4 * g + i;
-          float gh = 0.f;
-#pragma unroll
-          for (int k = 0; k < 4; ++k) gh = fmaf(sW4[k * kH + nr], gy[nt][k], gh);
-          float gz = 0.f;
-          if (valid[nt]) {
-            const float z4 = a.Z[((size_t)3 * kH + nr) * a.bcap + pid[nt]];
-            gz = gh * dsilu(z4);
-            a.gZ[((size_t)3 * kH + nr) * a.bcap + pid[nt]] = gz;
-          }
-          Bg[mt >> 1][nt][(mt & 1) * 4 + i] = (__bf16)gz;
-        }
-    floatx4 acc[8][kNT];
-#pragma unroll 1
-    for (int layer = 2; layer >= 0; --layer) {
-      hidden_mfma(sW + layer * kLdsLayer, nullptr, Bg, acc, g, c);
-#pragma unroll
-      for (int mt = 0; mt < 8; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < kNT; ++nt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int nr = 16 * mt + 4 * g + i;
-            float gz = 0.f;
-            if (valid[nt]) {
-              const float zl = a.Z[((size_t)layer * kH + nr) * a.bcap + pid[nt]];
-              gz = acc[mt][nt][i] * dsilu(zl);
-              a.gZ[((size_t)layer * kH + nr) * a.bcap + pid[nt]] = gz;
-            }
-            Bg[mt >> 1][nt][(mt & 1) * 4 + i] = (__bf16)gz;
-          }
-    }
+  for (int k = 0; k < 4; ++k) {
+    const int row = 16 * wave + 4 * k + (lane >> 4), q = (lane & 15) ^ (row & 15);
+    __builtin_amdgcn_global_load_lds((GlobalPtr)(W + row * kH + 8 * q),
+                                     (LdsPtr)(buf + (16 * wave + 4 * k) * kH), 16, 0, 0);
   }
 }
 
-// dW_l[o][i] = sum_p gZ_{l+1}[o][p] * silu(Z_l)[i][p] for hidden layers l = 1..3,
-// one block per (chunk of kChunk points, layer); 4 waves x (2 M-tiles x 8 N-tiles).
-constexpr int kChunk = 256;
-__global__ __launch_bounds__(256) void mlp_dw_kernel(const float* __restrict__ Z,
-                                                      const float* __restrict__ gZ, int64_t n,
-                                                      int64_t bcap, float* __restrict__ part) {
-  const int chunk = blockIdx.x, layer = blockIdx.y;   // layer 0..2 -> W1..W3
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int g = lane >> 4, c = lane & 15;
-  const float* G = gZ + (size_t)(layer + 1) * kH * bcap;   // gZ_{l+1}
-  const float* H = Z + (size_t)layer * kH * bcap;          // Z_l (silu applied on load)
-  floatx4 acc[2][8];
+// The block's copies and stage writes have arrived, and every wave is done
+// with the buffers they replace.
+__device__ __forceinline__ void train_sync() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  __syncthreads();
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// Four consecutive floats of the small parameters (16-byte aligned: every
+// array there starts at a multiple of four).
+__device__ __forceinline__ float4 small4(const float* p) {
+  return *reinterpret_cast<const float4*>(__builtin_assume_aligned(p, 16));
+}
+
+// acc = bias + W x B for one 16-point tile, W in a swizzled LDS buffer (BIAS
+// false: no bias).
+template <bool BIAS>
+__device__ __forceinline__ void train_mfma(const __bf16* __restrict__ sW, const float* bias,
+                                           const bf16x8 (&B)[4], floatx4 (&acc)[8], int g, int c) {
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 8; ++b) acc[a][b] = floatx4{0.f, 0.f, 0.f, 0.f};
-  const int64_t p0 = (int64_t)chunk * kChunk;
-  for (int ks = 0; ks < kChunk / 32; ++ks) {
-    __builtin_amdgcn_sched_barrier(0);
-    const int64_t pk = p0 + 32 * ks + 8 * g;
-    bf16x8 A[2], Bv[8];
-#pragma unroll
-    for (int a = 0; a < 2; ++a) {
-      const float* src = G + (size_t)(16 * (2 * wave + a) + c) * bcap + pk;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) A[a][j] = (__bf16)((pk + j < n) ? src[j] : 0.f);
+  for (int mt = 0; mt < 8; ++mt) {
+    if constexpr (BIAS) {
+      const float4 b = small4(bias + 16 * mt + 4 * g);
+      acc[mt] = floatx4{b.x, b.y, b.z, b.w};
+    } else {
+      acc[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
     }
-#pragma unroll
-    for (int b = 0; b < 8; ++b) {
-      const float* src = H + (size_t)(16 * b + c) * bcap + pk;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) Bv[b][j] = (__bf16)((pk + j < n) ? silu(src[j]) : 0.f);
-    }
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int b = 0; b < 8; ++b) acc[a][b] = mfma16(A[a], Bv[b], acc[a][b]);
   }
-  float* out = part + ((size_t)layer * gridDim.x + chunk) * kH * kH;
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int kk = 0; kk < 4; ++kk) {
+    // two K-steps' operand reads in flight at a time (register budget)
+    if (kk == 2) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int b = 0; b < 8; ++b)
+    for (int mt = 0; mt < 8; ++mt) {
+      const bf16x8 a = *reinterpret_cast<const bf16x8*>(sW + (16 * mt + c) * kH + (((4 * kk + g) ^ c) << 3));
+      acc[mt] = mfma16(a, B[kk], acc[mt]);
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// The lane's 32 values (neuron 16 mt + 4 g + i at v[4 mt + i]) as bf16 into
+// row p of a stage.
+__device__ __forceinline__ void train_stage(__bf16* st, int p, int g, const float (&v)[32]) {
+  typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+  for (int mt = 0; mt < 8; ++mt) {
+    bf16x4 b;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) b[i] = (__bf16)v[4 * mt + i];
+    *reinterpret_cast<bf16x4*>(st + p * kStageRow + 16 * mt + 4 * g) = b;
+  }
+}
+
+// K-step ks (points 32 ks ..) of the neurons n0 .. n0 + 15 as an MFMA operand.
+__device__ __forceinline__ bf16x8 train_operand(const __bf16* st, int ks, int n0, int g, int c) {
+  const __bf16* p = st + (32 * ks + 4 * g + (c >> 2)) * kStageRow + n0 + 4 * (c & 3);
+  union {
+    s16x4 h[2];
+    bf16x8 v;
+  } u;
+  u.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsS4)p);
+  u.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsS4)(p + 16 * kStageRow));
+  return u.v;
+}
+
+// The staged points' product G H^T, rows 16 wave .. of part ([128][128]).
+__device__ __forceinline__ void train_dw(const __bf16* sG, const __bf16* sH, float* __restrict__ part,
+                                         int wave, int g, int c) {
+  floatx4 acc[8];
+  float* o = part + (16 * wave + 4 * g) * kH + c;
+#pragma unroll
+  for (int b = 0; b < 8; ++b) acc[b] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int ks = 0; ks < kTrainPts / 32; ++ks) {
+    const bf16x8 a = train_operand(sG, ks, 16 * wave, g, c);
+#pragma unroll
+    for (int b = 0; b < 8; ++b) acc[b] = mfma16(a, train_operand(sH, ks, 16 * b, g, c), acc[b]);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int b = 0; b < 8; ++b)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i * kH + 16 * b] = acc[b][i];
+}
+
+// Keeps the compiler from holding what it computed from z (the sigmoids, one
+// register a value) until they are needed again: recomputed they cost two
+// transcendentals, held they spill.
+__device__ __forceinline__ void forget(floatx4 (&z)[8]) {
+#pragma unroll
+  for (int k = 0; k < 8; ++k) asm volatile("" : "+v"(z[k]));
+}
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_get(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+
+// Sums of the 32 values over the 16 lanes of a row (one point each): each
+// exchange halves the values a lane keeps; lane c ends with the sums of
+// values 2 c and 2 c + 1.
+__device__ __forceinline__ void reduce_rows(float (&v)[32], int c, float (&s)[2]) {
+  const bool b3 = c & 8, b2 = c & 4, b1 = c & 2, b0 = c & 1;
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    const float keep = b3 ? v[k + 16] : v[k], send = b3 ? v[k] : v[k + 16];
+    v[k] = keep + dpp_get<0x140>(send);   // row_mirror: lane 15 - c
+  }
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const float keep = b2 ? v[k + 8] : v[k], send = b2 ? v[k] : v[k + 8];
+    v[k] = keep + dpp_get<0x141>(send);   // row_half_mirror
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const float keep = b1 ? v[k + 4] : v[k], send = b1 ? v[k] : v[k + 4];
+    v[k] = keep + dpp_get<0x4E>(send);    // lanes 2 apart
+  }
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const float keep = b0 ? v[k + 2] : v[k], send = b0 ? v[k] : v[k + 2];
+    s[k] = keep + dpp_get<0xB1>(send);    // neighbours
+  }
+}
+
+// z = Z[l] and Z[l] = z for a uniform l that is not known at compile time.
+__device__ __forceinline__ void layer_get(const floatx4 (&Z)[4][8], int l, floatx4 (&z)[8]) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    if (l == k) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) z[j] = Z[k][j];
+    }
+}
+__device__ __forceinline__ void layer_put(floatx4 (&Z)[4][8], int l, const floatx4 (&z)[8]) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    if (l == k) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) Z[k][j] = z[j];
+    }
+}
+__device__ __forceinline__ float pick4(const float (&v)[4], int k) {
+  return k == 0 ? v[0] : k == 1 ? v[1] : k == 2 ? v[2] : v[3];
+}
+
+// Sums over the wave's 16 points of m v, to the wave's row of small sums:
+// lane c of group g has neurons 16 (c / 2) + 4 g + 2 (c & 1) + {0, 1}.
+__device__ __forceinline__ void small_sums(const float (&v)[32], float m, float* __restrict__ row,
+                                           int g, int c) {
+  float u[32], s[2];
+#pragma unroll
+  for (int j = 0; j < 32; ++j) u[j] = m * v[j];
+  reduce_rows(u, c, s);
+  *reinterpret_cast<float2*>(row + 16 * (c >> 1) + 4 * g + 2 * (c & 1)) = make_float2(s[0], s[1]);
+}
+
+__global__ __launch_bounds__(kTrainThreads) void mlp_train_kernel(MLPTrainArgs a) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  __bf16* buf = reinterpret_cast<__bf16*>(smem);   // two operands of kH * kH
+  __bf16* sG = buf + 2 * kH * kH;
+  __bf16* sH = sG + kStageElems;
+  float* sS = reinterpret_cast<float*>(sH + kStageElems);
+  __shared__ double s_loss[8][5];
+  const float* sW0 = sS;
+  const float* sB0 = sS + kH * kNIn;
+  const float* sBh = sB0 + kH;
+  const float* sW4 = sS + kH * kNIn + 4 * kH;
+  const float* sB4 = sW4 + kNOut * kH;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int g = lane >> 4, c = lane & 15;
+  train_load(a.Wp, buf, wave, lane);
+  load_small(a.params, sS);
+  if (lane < 5) s_loss[wave][lane] = 0.0;          // the wave's loss and db4
+  int tiles = 0;
+#pragma unroll 1
+  for (int t = 0; t < a.tiles; ++t) {
+    const int64_t tile = (int64_t)blockIdx.x * a.tiles + t;
+    const int64_t p0 = tile * kTrainPts;
+    if (p0 >= a.n) break;
+    ++tiles;
+    float* part = a.dwpart + (size_t)tile * 3 * kH * kH;
+    float* rows = a.small_wave + ((size_t)tile * 8 + wave) * 11 * kH;   // dW0 (3), db0..3, dW4 (4)
+    const int row = 16 * wave + c;   // the lane's point in the tile
+    const int64_t p = p0 + row;
+    const bool valid = p < a.n;
+    const int64_t q = valid ? p : 0;
+    float f[4], tg[4];
+    {
+      float f3[3];
+      mlp_features(a.cfg, a.x[q], a.y[q], a.z[q], f3);
+      f[0] = f3[0]; f[1] = f3[1]; f[2] = f3[2];
+      f[3] = 1.f;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) tg[k] = a.target[(size_t)k * a.n + q];
+    const float wt = valid ? (a.weight ? a.weight[q] : 1.f) : 0.f;
+    floatx4 Z[4][8], z[8];
+    bf16x8 B[4];
+    float v[32];
+    train_sync();   // W1 (and the small parameters)
+#pragma unroll
+    for (int mt = 0; mt < 8; ++mt) {
+      const int nr = 16 * mt + 4 * g;
+      const float4 w0 = small4(sW0 + 3 * nr), w1 = small4(sW0 + 3 * nr + 4), w2 = small4(sW0 + 3 * nr + 8);
+      const float4 b = small4(sB0 + nr);
+      const float w[12] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w, w2.x, w2.y, w2.z, w2.w};
+      const float bb[4] = {b.x, b.y, b.z, b.w};
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        out[(size_t)(16 * (2 * wave + a) + 4 * g + i) * kH + 16 * b + c] = acc[a][b][i];
-}
-
-// grads[W_l] = sum over chunks (fixed order) of the partials.
-__global__ void mlp_dw_reduce_kernel(const float* __restrict__ part, int nchunk,
-                                     float* __restrict__ grads) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  const int layer = blockIdx.y;
-  if (e >= kH * kH) return;
-  const float* p = part + (size_t)layer * nchunk * kH * kH + e;
-  double s = 0.0;
-  for (int k = 0; k < nchunk; ++k) s += p[(size_t)k * kH * kH];
-  grads[kHidOff[layer] + e] = (float)s;
-}
-
-// Gradients of W0, b0..b3, W4, b4: one block per parameter, fixed-order sums.
-__global__ __launch_bounds__(256) void mlp_small_grads_kernel(const float* __restrict__ feat,
-                                                              const float* __restrict__ Z,
-                                                              const float* __restrict__ gZ,
-                                                              const float* __restrict__ gY,
-                                                              int64_t n, int64_t bcap,
-                                                              float* __restrict__ grads) {
-  __shared__ double sh[256];
-  int q = blockIdx.x;  // 0..(384 + 512 + 512 + 4)
-  const float* u = nullptr;
-  const float* v = nullptr;
-  bool silu_v = false;
-  int dst;
-  if (q < kH * kNIn) {                      // dW0[nr][d]
-    const int nr = q / 3, d = q % 3;
-    u = gZ + (size_t)nr * bcap;
-    v = feat + (size_t)d * bcap;
-    dst = kOffW0 + q;
-  } else if ((q -= kH * kNIn) < 4 * kH) {   // db0..db3
-    const int l = q / kH, nr = q % kH;
-    u = gZ + ((size_t)l * kH + nr) * bcap;
-    dst = (l == 0 ? kOffB0 : l == 1 ? kOffB1 : l == 2 ? kOffB2 : kOffB3) + nr;
-  } else if ((q -= 4 * kH) < kNOut * kH) {  // dW4[k][nr]
-    const int k = q / kH, nr = q % kH;
-    u = gY + (size_t)k * bcap;
-    v = Z + ((size_t)3 * kH + nr) * bcap;
-    silu_v = true;
-    dst = kOffW4 + q;
-  } else {                                  // db4[k]
-    q -= kNOut * kH;
-    u = gY + (size_t)q * bcap;
-    dst = kOffB4 + q;
+        Z[0][mt][i] = fmaf(w[3 * i], f[0], fmaf(w[3 * i + 1], f[1], fmaf(w[3 * i + 2], f[2], bb[i])));
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) z[j] = Z[0][j];
+    // layers as loops: unrolled, the kernel's 60 KB of code were read from
+    // the L2 once per tile, which took longer than running them
+#pragma unroll 1
+    for (int l = 0; l < 3; ++l) {
+#pragma unroll
+      for (int j = 0; j < 32; ++j) B[j >> 3][j & 7] = (__bf16)silu(z[j >> 2][j & 3]);
+      if (l > 0) train_sync();   // W_{l+1}; then the next operand into the other buffer
+      train_load(l < 2 ? a.Wp + (l + 1) * kH * kH : a.Wt + 2 * kH * kH, buf + ((l + 1) & 1) * kH * kH,
+                 wave, lane);
+      train_mfma<true>(buf + (l & 1) * kH * kH, sBh + l * kH, B, z, g, c);
+      layer_put(Z, l + 1, z);
+    }
+    // output layer and loss (all four lane groups hold the same point)
+    float gy[4];
+#pragma unroll
+    for (int k = 0; k < 32; ++k) v[k] = silu(z[k >> 2][k & 3]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      float s = 0.f;
+#pragma unroll
+      for (int mt = 0; mt < 8; ++mt) {
+        const float4 w = small4(sW4 + k * kH + 16 * mt + 4 * g);
+        s = fmaf(w.x, v[4 * mt], s);
+        s = fmaf(w.y, v[4 * mt + 1], s);
+        s = fmaf(w.z, v[4 * mt + 2], s);
+        s = fmaf(w.w, v[4 * mt + 3], s);
+      }
+      s += __shfl_xor(s, 16);
+      s += __shfl_xor(s, 32);
+      const float d = valid ? s + sB4[k] - tg[k] : 0.f;
+      gy[k] = 2.f * wt * a.cfg.lw[k] * d * a.inv_n;
+      // the same in the four lane groups: over the 16 points in float64
+      double ls = (double)(wt * a.cfg.lw[k] * d * d), bs = (double)gy[k];
+#pragma unroll
+      for (int off = 8; off > 0; off >>= 1) {
+        ls += __shfl_xor(ls, off);
+        bs += __shfl_xor(bs, off);
+      }
+      if (lane == 0) {
+        s_loss[wave][0] += ls;
+        s_loss[wave][1 + k] += bs;
+      }
+    }
+#pragma unroll 1
+    for (int k = 0; k < 4; ++k) small_sums(v, pick4(gy, k), rows + (7 + k) * kH, g, c);
+    // gZ_4, and down the chain gZ_l = (W_l^T gZ_{l+1}) silu'(Z_l)
+    asm volatile("" ::: "memory");   // W4 is read again, not kept
+    forget(z);
+#pragma unroll
+    for (int mt = 0; mt < 8; ++mt) {
+      float gh[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float4 w = small4(sW4 + k * kH + 16 * mt + 4 * g);
+        gh[0] = fmaf(w.x, gy[k], gh[0]);
+        gh[1] = fmaf(w.y, gy[k], gh[1]);
+        gh[2] = fmaf(w.z, gy[k], gh[2]);
+        gh[3] = fmaf(w.w, gy[k], gh[3]);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[4 * mt + i] = gh[i] * dsilu(z[mt][i]);
+    }
+#pragma unroll 1
+    for (int l = 2; l >= 0; --l) {
+      // v = gZ_{l+2}: operand of the chain, of dW_{l+1}, and its bias sums
+#pragma unroll
+      for (int j = 0; j < 32; ++j) B[j >> 3][j & 7] = (__bf16)v[j];
+      train_stage(sG, row, g, v);
+      small_sums(v, 1.f, rows + (4 + l) * kH, g, c);
+      layer_get(Z, l, z);
+#pragma unroll
+      for (int j = 0; j < 32; ++j) v[j] = silu(z[j >> 2][j & 3]);
+      train_stage(sH, row, g, v);
+      forget(z);
+      train_sync();   // the stages and W_{l+1}^T
+      // next operand: W^T of the layer below, or W1 of the next tile
+      train_load(l > 0 ? a.Wt + (l - 1) * kH * kH : a.Wp, buf + (l & 1) * kH * kH, wave, lane);
+      train_dw(sG, sH, part + l * kH * kH, wave, g, c);
+      floatx4 acc[8];
+      train_mfma<false>(buf + ((l + 1) & 1) * kH * kH, nullptr, B, acc, g, c);
+#pragma unroll
+      for (int j = 0; j < 32; ++j) v[j] = acc[j >> 2][j & 3] * dsilu(z[j >> 2][j & 3]);
+      __syncthreads();   // every wave has read the stages
+    }
+#pragma unroll 1
+    for (int d = 0; d < 4; ++d) small_sums(v, pick4(f, d), rows + d * kH, g, c);
   }
-  double s = 0.0;
-  for (int64_t p = threadIdx.x; p < n; p += 256) {
-    double t = u[p];
-    if (v) t *= silu_v ? (double)silu(v[p]) : (double)v[p];
-    s += t;
-  }
-  sh[threadIdx.x] = s;
+  // the small sums over the block's tiles and waves, the waves' loss and db4
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  __threadfence_block();
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
+  const float* rows = a.small_wave + (size_t)blockIdx.x * a.tiles * 8 * 11 * kH;
+  double* out = a.small_part + (size_t)blockIdx.x * kSmallRow;
+  for (int e = threadIdx.x; e < 11 * kH; e += kTrainThreads) {
+    double s = 0.0;
+#pragma unroll 8
+    for (int w = 0; w < 8 * tiles; ++w) s += (double)rows[(size_t)w * 11 * kH + e];
+    out[e] = s;
+  }
+  if (threadIdx.x < 5) {
+    double s = 0.0;
+    for (int w = 0; w < 8; ++w) s += s_loss[w][threadIdx.x];
+    out[threadIdx.x == 0 ? kNSmall : 11 * kH + threadIdx.x - 1] = s;
+  }
+}
+
+// Gradients from the blocks' partial sums, each in a fixed order in float64.
+// The first kDwBlocks blocks: 64 elements of dW1..dW3 each, four threads per
+// element over a quarter of the tiles; the others: 16 small sums each, 16
+// threads per sum over every 16th block.
+constexpr int kDwBlocks = 3 * kH * kH / 64;
+constexpr int kSmallBlocks = (kSmallRow + 15) / 16;
+__global__ __launch_bounds__(256) void mlp_reduce_kernel(const float* __restrict__ dwpart,
+                                                         const double* __restrict__ small_part,
+                                                         int ntile, int nblk,
+                                                         float* __restrict__ grads,
+                                                         double* __restrict__ loss_out) {
+  __shared__ double sh[256];
+  const int t = threadIdx.x;
+  if (blockIdx.x < kDwBlocks) {
+    const int e = blockIdx.x * 64 + (t & 63);
+    const int per = (ntile + 3) / 4, b0 = (t >> 6) * per, b1 = min(b0 + per, ntile);
+    double s = 0.0;
+#pragma unroll 8
+    for (int b = b0; b < b1; ++b) s += (double)dwpart[(size_t)b * 3 * kH * kH + e];
+    sh[t] = s;
+    __syncthreads();
+    if (t < 64)
+      grads[kHidOff[e / (kH * kH)] + e % (kH * kH)] = (float)(((sh[t] + sh[64 + t]) + sh[128 + t]) + sh[192 + t]);
+    return;
+  }
+  const int e = (blockIdx.x - kDwBlocks) * 16 + (t & 15), j = t >> 4;
+  double s = 0.0;
+  if (e < kSmallRow) {
+#pragma unroll 4
+    for (int b = j; b < nblk; b += 16) s += small_part[(size_t)b * kSmallRow + e];
+  }
+  sh[t] = s;
+  __syncthreads();
+  for (int w = 8; w > 0; w >>= 1) {
+    if (j < w) sh[t] += sh[t + 16 * w];
     __syncthreads();
   }
-  if (threadIdx.x == 0) grads[dst] = (float)sh[0];
-}
-
-__global__ void loss_reduce_kernel(const double* __restrict__ part, int nb, double* __restrict__ out) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    double s = 0.0;
-    for (int b = 0; b < nb; ++b) s += part[b];
-    out[0] = s;
-  }
+  if (j != 0 || e >= kSmallRow) return;
+  const double v = sh[t];
+  if (e < 3 * kH) grads[kOffW0 + (e % kH) * kNIn + e / kH] = (float)v;
+  else if (e < 7 * kH) {
+    const int l = e / kH - 3;
+    grads[(l == 0 ? kOffB0 : l == 1 ? kOffB1 : l == 2 ? kOffB2 : kOffB3) + e % kH] = (float)v;
+  } else if (e < 11 * kH) grads[kOffW4 + e - 7 * kH] = (float)v;
+  else if (e < kNSmall) grads[kOffB4 + e - 11 * kH] = (float)v;
+  else if (loss_out) loss_out[0] = v;
 }
 
 // bf16 operand copies of W1..W3: Wp[l][o][k] = W[o][pi(k)], Wt[l][i][k] = W[pi(k)][i].
@@ -880,14 +1073,10 @@ __global__ __launch_bounds__(GRAD ? kBlockGrad : kBlockInf) void mlp_leapfrog_ke
       }
       // surrogate forward for the wave's points (column c, tiles nt)
       float f[NT][3];
-      int64_t pid[NT];
-      bool valid[NT];
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
         const float qx = __shfl(px, 16 * nt + c), qy = __shfl(py, 16 * nt + c), qz = __shfl(pz, 16 * nt + c);
         mlp_features(a.cfg, qx, qy, qz, f[nt]);
-        pid[nt] = 0;
-        valid[nt] = false;
       }
       float yk[NT][4];
       if constexpr (GRAD) {
@@ -901,7 +1090,7 @@ __global__ __launch_bounds__(GRAD ? kBlockGrad : kBlockInf) void mlp_leapfrog_ke
           yk[nt][3] = dy[nt][2];
         }
       } else {
-        mlp_tile_forward<false>(sW, sS, f, yk, g, c, nullptr, 0, pid, valid);
+        mlp_tile_forward(sW, sS, f, yk, g, c);
       }
       if (live) {
         float yv[4];
@@ -1040,25 +1229,26 @@ int mlp_ready(Context* c) {
   return 0;
 }
 
-int mlp_batch_buffers(Context* c, int64_t n, hipStream_t s) {
+// 128-point tiles of a batch, and how many each block takes: as many as
+// leave one block for each of the 256 CUs (a block fills a CU's LDS).
+int64_t train_tiles(int64_t n) { return (n + kTrainPts - 1) / kTrainPts; }
+int tiles_per_block(int64_t tiles) { return (int)((tiles + 255) / 256); }
+
+int mlp_batch_buffers(Context* c, int64_t tiles, hipStream_t s) {
   MLPState& M = c->mlp;
-  if (n <= M.bcap) return 0;
+  if (tiles <= M.bcap) return 0;
   BFE_HIP(c, hipStreamSynchronize(s));
-  for (float** p : {&M.feat, &M.Z, &M.gZ, &M.gY, &M.dwpart}) {
-    if (*p) (void)hipFree(*p);
-    *p = nullptr;
-  }
-  if (M.loss_part) (void)hipFree(M.loss_part);
-  M.loss_part = nullptr;
-  const int64_t cap = ((n + kChunk - 1) / kChunk) * kChunk;
-  const int64_t nchunk = cap / kChunk;
-  BFE_HIP(c, hipMalloc(&M.feat, sizeof(float) * 3 * cap));
-  BFE_HIP(c, hipMalloc(&M.Z, sizeof(float) * 4 * kH * cap));
-  BFE_HIP(c, hipMalloc(&M.gZ, sizeof(float) * 4 * kH * cap));
-  BFE_HIP(c, hipMalloc(&M.gY, sizeof(float) * 4 * cap));
-  BFE_HIP(c, hipMalloc(&M.dwpart, sizeof(float) * 3 * nchunk * kH * kH));
-  BFE_HIP(c, hipMalloc(&M.loss_part, sizeof(double) * ((cap + block_points<true>() - 1) / block_points<true>())));
-  M.bcap = cap;
+  if (M.dwpart) (void)hipFree(M.dwpart);
+  if (M.small_wave) (void)hipFree(M.small_wave);
+  if (M.small_part) (void)hipFree(M.small_part);
+  M.dwpart = nullptr;
+  M.small_wave = nullptr;
+  M.small_part = nullptr;
+  M.bcap = 0;
+  BFE_HIP(c, hipMalloc(&M.dwpart, sizeof(float) * 3 * kH * kH * (size_t)tiles));
+  BFE_HIP(c, hipMalloc(&M.small_wave, sizeof(float) * 8 * 11 * kH * (size_t)tiles));
+  BFE_HIP(c, hipMalloc(&M.small_part, sizeof(double) * kSmallRow * 256));
+  M.bcap = tiles;
   return 0;
 }
 
@@ -1066,35 +1256,35 @@ MLPKArgs base_args(Context* c) {
   MLPKArgs a{};
   a.params = c->mlp.params;
   a.Wp = c->mlp.Wp;
-  a.Wt = c->mlp.Wt;
   a.cfg = make_cfg(c->mlp);
   return a;
 }
 
-// Forward + backward + gradient assembly for n points (n <= bcap).
+// Gradient of the loss over n points.
 int mlp_gradient(Context* c, const float* x, const float* y, const float* z, const float* target,
                  const float* weight, int64_t n, float* grads, double* loss_out, hipStream_t s) {
-  int rc = mlp_batch_buffers(c, n, s);
+  const int64_t tiles = train_tiles(n);
+  if (tiles > (int64_t)0x7fffffff) return set_error(c, BFE_ELIMIT, "mlp_gradient: n too large");
+  int rc = mlp_batch_buffers(c, tiles, s);
   if (rc) return rc;
   MLPState& M = c->mlp;
-  MLPKArgs a = base_args(c);
+  MLPTrainArgs a{};
   a.x = x; a.y = y; a.z = z; a.n = n;
   a.target = target;
   a.weight = weight;
-  a.feat = M.feat; a.Z = M.Z; a.gZ = M.gZ; a.gY = M.gY; a.bcap = M.bcap;
-  a.loss_part = M.loss_part;
+  a.tiles = tiles_per_block(tiles);
+  const int nblk = (int)((tiles + a.tiles - 1) / a.tiles);   // at most 256
   a.inv_n = 1.f / (float)n;
-  const int nb = (int)((n + block_points<true>() - 1) / block_points<true>());
-  hipLaunchKernelGGL(mlp_fwd_kernel<true>, dim3(nb), dim3(kBlockTrain), kLdsBytes, s, a);
-  hipLaunchKernelGGL(mlp_bwd_kernel, dim3(nb), dim3(kBlockTrain), kLdsBytes, s, a);
-  BFE_HIP(c, hipGetLastError());
-  const int nchunk = (int)((n + kChunk - 1) / kChunk);
-  hipLaunchKernelGGL(mlp_dw_kernel, dim3(nchunk, 3), dim3(256), 0, s, M.Z, M.gZ, n, M.bcap, M.dwpart);
-  hipLaunchKernelGGL(mlp_dw_reduce_kernel, dim3((kH * kH + 255) / 256, 3), dim3(256), 0, s, M.dwpart,
-                     nchunk, grads);
-  hipLaunchKernelGGL(mlp_small_grads_kernel, dim3(kH * kNIn + 4 * kH + kNOut * kH + kNOut), dim3(256),
-                     0, s, M.feat, M.Z, M.gZ, M.gY, n, M.bcap, grads);
-  if (loss_out) hipLaunchKernelGGL(loss_reduce_kernel, dim3(1), dim3(64), 0, s, M.loss_part, nb, loss_out);
+  a.params = M.params;
+  a.Wp = M.Wp;
+  a.Wt = M.Wt;
+  a.dwpart = M.dwpart;
+  a.small_wave = M.small_wave;
+  a.small_part = M.small_part;
+  a.cfg = make_cfg(M);
+  hipLaunchKernelGGL(mlp_train_kernel, dim3((unsigned)nblk), dim3(kTrainThreads), kTrainLds, s, a);
+  hipLaunchKernelGGL(mlp_reduce_kernel, dim3(kDwBlocks + kSmallBlocks), dim3(256), 0, s, M.dwpart,
+                     M.small_part, (int)tiles, nblk, grads, loss_out);
   BFE_HIP(c, hipGetLastError());
   return 0;
 }
@@ -1111,13 +1301,13 @@ int mlp_sync(Context* c, hipStream_t s) {
 namespace bfe {
 void mlp_free(Context* c) {
   MLPState& M = c->mlp;
-  for (float** p : {&M.params, &M.grads, &M.m, &M.v, &M.feat, &M.Z, &M.gZ, &M.gY, &M.dwpart}) {
+  for (float** p : {&M.params, &M.grads, &M.m, &M.v, &M.dwpart, &M.small_wave}) {
     if (*p) (void)hipFree(*p);
     *p = nullptr;
   }
   if (M.Wp) (void)hipFree(M.Wp);
   if (M.Wt) (void)hipFree(M.Wt);
-  if (M.loss_part) (void)hipFree(M.loss_part);
+  if (M.small_part) (void)hipFree(M.small_part);
   M = MLPState();
 }
 }  // namespace bfe
@@ -1138,12 +1328,10 @@ extern "C" int bfe_mlp_set_params(bfe_ctx* h, const float* params, int64_t count
     BFE_HIP(c, hipMalloc(&M.v, sizeof(float) * kNParams));
     BFE_HIP(c, hipMalloc(&M.Wp, sizeof(__bf16) * 3 * kH * kH));
     BFE_HIP(c, hipMalloc(&M.Wt, sizeof(__bf16) * 3 * kH * kH));
-    BFE_HIP(c, hipFuncSetAttribute((const void*)mlp_fwd_kernel<true>,
+    BFE_HIP(c, hipFuncSetAttribute((const void*)mlp_fwd_kernel,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes));
-    BFE_HIP(c, hipFuncSetAttribute((const void*)mlp_fwd_kernel<false>,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes));
-    BFE_HIP(c, hipFuncSetAttribute((const void*)mlp_bwd_kernel,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes));
+    BFE_HIP(c, hipFuncSetAttribute((const void*)mlp_train_kernel,
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTrainLds));
     BFE_HIP(c, hipFuncSetAttribute((const void*)mlp_leapfrog_kernel<false>,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes));
     BFE_HIP(c, hipFuncSetAttribute((const void*)mlp_leapfrog_kernel<true>,
@@ -1227,9 +1415,9 @@ extern "C" int bfe_mlp_forward(bfe_ctx* h, const float* x, const float* y, const
     BFE_HIP(c, hipGetLastError());
     return 0;
   }
-  const int64_t ntiles = (n + block_points<false>() - 1) / block_points<false>();
+  const int64_t ntiles = (n + kInfPts - 1) / kInfPts;
   const int nb = (int)(ntiles < 1024 ? ntiles : 1024);
-  hipLaunchKernelGGL(mlp_fwd_kernel<false>, dim3(nb), dim3(kBlockInf), kLdsBytes, s, a);
+  hipLaunchKernelGGL(mlp_fwd_kernel, dim3(nb), dim3(kBlockInf), kLdsBytes, s, a);
   BFE_HIP(c, hipGetLastError());
   return 0;
 }
@@ -1287,7 +1475,7 @@ extern "C" int bfe_mlp_leapfrog(bfe_ctx* h, float* x, float* y, float* z, float*
   if (n == 0) return 0;
   BFE_HIP(c, hipSetDevice(c->device));
   hipStream_t s = (hipStream_t)stream;
-  const int64_t ntiles = (n + block_points<false>() - 1) / block_points<false>();
+  const int64_t ntiles = (n + kInfPts - 1) / kInfPts;
   const int nb = (int)(ntiles < 2048 ? ntiles : 2048);
   const int chunk = energy_every > 0 ? energy_every : (int)(nsteps < 100 ? (nsteps > 0 ? nsteps : 1) : 100);
   const int nchecks = energy_every > 0 ? (int)(nsteps / energy_every) + 1 : 1;
