@@ -19,6 +19,13 @@
 namespace bfe {
 
 constexpr int kTile = 256;   // EOF: particles per tile (one per lane for geometry)
+// The input-order EOF kernel's tile while that gives at most a segment budget of
+// blocks: a block walks its tile one particle after the other, each a dependent
+// table read, so few particles are bound by one tile's walk.  With eight
+// particles' reads in flight as well, whole calls on MI355X, tiles of 256 before
+// and of 64 now: 500 56 -> 18.7 us, 10 000 71 -> 23.4, 30 000 87 -> 31,
+// 65 000 88 -> 36.
+constexpr int kSmallTile = 64;
 constexpr int kSLTile = 64;  // SL: particles per tile
 constexpr int kFlush = 16;   // float32 partial sums are moved to float64 every kFlush particles
 
@@ -47,14 +54,14 @@ __device__ __forceinline__ void segment_range(const Segments& S, int64_t sg, int
   }
 }
 
-template <int OPT>
+template <int OPT, int TILE>
 __global__ __launch_bounds__(256) void eof_accumulate_kernel(
     const float* __restrict__ px, const float* __restrict__ py, const float* __restrict__ pz,
     const float* __restrict__ pm, Segments S, EOFGeom g, const float* __restrict__ T, int K,
     double* __restrict__ partials) {
-  __shared__ int s_base[kTile];
-  __shared__ float s_c[4][kTile];
-  __shared__ float s_w[2 * kMaxM + 1][kTile + 1];  // +1: spread rows over banks
+  __shared__ int s_base[TILE];
+  __shared__ float s_c[4][TILE];
+  __shared__ float s_w[2 * kMaxM + 1][TILE + 1];  // +1: spread rows over banks
 
   const int tid = threadIdx.x;
   const int ny1 = g.numy + 1;
@@ -73,9 +80,11 @@ __global__ __launch_bounds__(256) void eof_accumulate_kernel(
   segment_range(S, sg, s0, s1);
 #pragma unroll
   for (int o = 0; o < OPT; ++o) accd[o] = 0.0;
-  for (int64_t t0 = s0; t0 < s1; t0 += kTile) {
+  for (int64_t t0 = s0; t0 < s1; t0 += TILE) {
     const int64_t p = t0 + tid;
-    if (p < s1) {
+    if (TILE < 256 && tid >= TILE) {
+      // no particle of its own: it only owns coefficients
+    } else if (p < s1) {
       const double x = px[p], y = py[p], z = pz[p], mass = pm[p];
       const double R = sqrt(x * x + y * y + 1.e-10);
       double c1, s1;
@@ -104,7 +113,8 @@ __global__ __launch_bounds__(256) void eof_accumulate_kernel(
     }
     __syncthreads();
     const int64_t left = s1 - t0;
-    const int np = left < kTile ? (int)left : kTile;
+    const int np = left < TILE ? (int)left : TILE;
+#pragma unroll 8
     for (int q = 0; q < np; ++q) {
       const size_t b = (size_t)s_base[q];
       const float* T00 = T + b * K;
@@ -310,6 +320,7 @@ __global__ __launch_bounds__(256) void sl_accumulate_kernel(
     }
     __syncthreads();
     // radial functions phi_ln(r_p) for the tile, coalesced over ln
+#pragma unroll 8
     for (int idx = tid; idx < kSLTile * LN; idx += 256) {
       const int q = idx / LN, ln = idx - q * LN;
       const size_t i = (size_t)s_i[q];
@@ -318,6 +329,7 @@ __global__ __launch_bounds__(256) void sl_accumulate_kernel(
     __syncthreads();
     const int64_t left = s1 - t0;
     const int np = left < kSLTile ? (int)left : kSLTile;
+#pragma unroll 8
     for (int q = 0; q < np; ++q) {
 #pragma unroll
       for (int o = 0; o < OPT; ++o) acc[o] = fmaf(s_Y[yrow[o] + q], s_phi[q * LN + prow[o]], acc[o]);
@@ -1574,6 +1586,29 @@ static DepShape dep_shape(int rows, int N, const DepShape* cands, int ncand, int
 static const DepShape kEofShapes[kEofDepShapes] = {{1, 4}, {1, 8}, {1, 16}, {2, 2}, {2, 4}, {2, 8}, {2, 16}, {4, 8}};
 static const DepShape kSlShapes[kSlDepShapes] = {{1, 8}, {1, 16}, {1, 24}, {2, 8}, {2, 16}, {2, 24}, {4, 16}};
 
+// Segment plan of the input-order EOF accumulate: tiles of kSmallTile while
+// they fit the segment budget, one each, then tiles of kTile.  Either way the
+// float32 sums are those of the same 16 consecutive particles.
+static AccPlan plan_input_order(int64_t cap, int64_t n) {
+  return plan_single(cap, n, (n + kSmallTile - 1) / kSmallTile <= cap ? kSmallTile : kTile);
+}
+
+static void eof_input_order_launch(const AccPlan& P, const float* x, const float* y, const float* z,
+                                   const float* m, const EOFGeom& g, const float* pot32, int K,
+                                   double* partials, hipStream_t s) {
+  const int opt = (K + 255) / 256;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(P.grid), dim3(256), 0, s, x, y, z, m, P.S, g, pot32, K, partials);
+  };
+  if (!P.S.segb && P.S.seglen <= kSmallTile) {
+    if (opt == 1) go(eof_accumulate_kernel<1, kSmallTile>);
+    else if (opt == 2) go(eof_accumulate_kernel<2, kSmallTile>);
+    else go(eof_accumulate_kernel<4, kSmallTile>);
+  } else if (opt == 1) go(eof_accumulate_kernel<1, kTile>);
+  else if (opt == 2) go(eof_accumulate_kernel<2, kTile>);
+  else go(eof_accumulate_kernel<4, kTile>);
+}
+
 int eof_dep_prepare(Context* c) {
   const DepShape dsh = dep_shape(2 * c->mmax + 1, c->norder, kEofShapes, kEofDepShapes,
                                  c->eof_dep_shape);
@@ -1706,8 +1741,15 @@ static int eof_accumulate_run(Context* c, const float* x, const float* y, const 
                               double* cos_out, double* sin_out, hipStream_t s,
                               bool beside = false) {
   const int K = c->eof_K;
+  // cell-ordered form: (2 mmax + 1) rows x chunks of radial orders per lane,
+  // LDS for the per-wave weights and the float64 wave reduction
+  const size_t dlds = std::max((size_t)4 * ((2 * c->mmax + 1) * kDepStride + kDepExtra) * sizeof(float),
+                               (size_t)4 * K * sizeof(double));
+  const DepShape dsh = dep_shape(2 * c->mmax + 1, c->norder, kEofShapes, kEofDepShapes, c->eof_dep_shape);
+  const bool ordered = n >= c->order_min && n > 0 && dsh.ppt > 0 && dlds <= 64 * 1024;
   AccPlan P = off ? plan_batch(c->eof_acc_blocks, c->eof_seg_tiles, off, nsnap, kTile)
-                  : plan_single(c->eof_acc_blocks, n, kTile);
+                  : ordered ? plan_single(c->eof_acc_blocks, n, kTile)
+                            : plan_input_order(c->eof_acc_blocks, n);
   const size_t pbytes = (size_t)P.S.nseg * K * sizeof(double);
   const size_t need = pbytes;
   const int64_t* rowb = nullptr;
@@ -1721,14 +1763,8 @@ static int eof_accumulate_run(Context* c, const float* x, const float* y, const 
   if (rc) return rc;
   double* partials = (double*)c->scratch;
   EOFGeom g = eof_geom(c);
-  const int opt = (K + 255) / 256;
   const float4* sorted = nullptr;
-  // cell-ordered form: (2 mmax + 1) rows x chunks of radial orders per lane,
-  // LDS for the per-wave weights and the float64 wave reduction
-  const size_t dlds = std::max((size_t)4 * ((2 * c->mmax + 1) * kDepStride + kDepExtra) * sizeof(float),
-                               (size_t)4 * K * sizeof(double));
-  const DepShape dsh = dep_shape(2 * c->mmax + 1, c->norder, kEofShapes, kEofDepShapes, c->eof_dep_shape);
-  if (n >= c->order_min && n > 0 && dsh.ppt > 0 && dlds <= 64 * 1024) {
+  if (ordered) {
     if ((rc = eof_dep_prepare(c))) return rc;
     rc = order_particles(c, 0, x, y, z, m, n, off_dev, nsnap, s, &sorted, off);
     if (rc) return rc;
@@ -1751,12 +1787,8 @@ static int eof_accumulate_run(Context* c, const float* x, const float* y, const 
   } else if (n == 0) {
     hipLaunchKernelGGL(fill_f64_kernel, dim3((unsigned)((P.S.nseg * K + 255) / 256)), dim3(256), 0, s,
                        partials, P.S.nseg * (int64_t)K);
-  } else if (opt == 1) {
-    hipLaunchKernelGGL(eof_accumulate_kernel<1>, dim3(P.grid), dim3(256), 0, s, x, y, z, m, P.S, g, c->eof_pot32, K, partials);
-  } else if (opt == 2) {
-    hipLaunchKernelGGL(eof_accumulate_kernel<2>, dim3(P.grid), dim3(256), 0, s, x, y, z, m, P.S, g, c->eof_pot32, K, partials);
   } else {
-    hipLaunchKernelGGL(eof_accumulate_kernel<4>, dim3(P.grid), dim3(256), 0, s, x, y, z, m, P.S, g, c->eof_pot32, K, partials);
+    eof_input_order_launch(P, x, y, z, m, g, c->eof_pot32, K, partials, s);
   }
   timer_end(c, "eof_accumulate", s);
   BFE_HIP(c, hipGetLastError());
@@ -1777,8 +1809,24 @@ static int sl_accumulate_run(Context* c, const float* x, const float* y, const f
   if (K > 1024) return set_error(c, BFE_ELIMIT, "sl_accumulate: (lmax+1)^2 nmax = %d > 1024", K);
   const size_t lds = ((size_t)R * (kSLTile + 1) + (size_t)kSLTile * LN + 3 * kSLTile) * 4;
   if (lds > 64 * 1024) return set_error(c, BFE_ELIMIT, "sl_accumulate: LDS %zu B > 64 KiB", lds);
+  const DepShape dsh = dep_shape(R, c->nmax, kSlShapes, kSlDepShapes, c->sl_dep_shape);
+  const size_t dlds = std::max((size_t)4 * sl_dep_rows(R) * kDepStride * sizeof(float),
+                               (size_t)4 * K * sizeof(double));
+  const bool bf16_mode = (flags & BFE_ACC_BF16) != 0;
+  const bool mfma_ok = c->lmax <= 7 && (c->lmax + 1) * ((c->nmax + 15) / 16) <= 4 * kMSlots;
+  const bool mfma = n > 0 && mfma_ok && (bf16_mode || c->sl_acc_path == 1);
+  const bool ordered = !mfma && n >= c->order_min && n > 0 && dsh.ppt > 0 && dlds <= 64 * 1024;
   AccPlan P = off ? plan_batch(c->sl_acc_blocks, c->sl_seg_tiles, off, nsnap, kSLTile)
                   : plan_single(beside ? c->sl_acc_blocks_beside : c->sl_acc_blocks, n, kSLTile);
+  // cell-ordered segments of up to four tiles leave a wave at most one tile,
+  // summed by itself: four tiles per segment then give the same float32 sums
+  // with no idle waves (100 000 particles: 1 563 blocks with three of four
+  // waves idle, 33 us, or 391)
+  if (!off && ordered && P.S.seglen < 4 * kSLTile) {
+    P.S.seglen = 4 * kSLTile;
+    P.S.nseg = (n + P.S.seglen - 1) / P.S.seglen;
+    P.grid = (int)P.S.nseg;
+  }
   const size_t pbytes = (size_t)P.S.nseg * K * sizeof(double);
   const int64_t* rowb = nullptr;
   const int64_t* off_dev = nullptr;
@@ -1789,16 +1837,13 @@ static int sl_accumulate_run(Context* c, const float* x, const float* y, const f
   const int no_odd = (flags & BFE_NO_ODD) ? 1 : 0;
   const int opt = (K + 255) / 256;
   // matrix-product form on the MFMA units (lmax <= 7, at most 16 output tiles)
-  const int mtiles = (c->lmax + 1) * ((c->nmax + 15) / 16);
-  const bool bf16_mode = (flags & BFE_ACC_BF16) != 0;
-  const bool mfma_ok = c->lmax <= 7 && mtiles <= 4 * kMSlots;
   if (bf16_mode && !mfma_ok)
     return set_error(c, BFE_ELIMIT, "sl_accumulate: BFE_ACC_BF16 needs lmax <= 7 and (lmax+1) ceil(nmax/16) <= 16");
   // measured at lmax 6, nmax 20, 1M particles on MI355X: MFMA 0.59 ms, the
   // cell-ordered vector-ALU path 0.19 ms + 0.09 ms sort, so "auto" takes the
   // vector-ALU paths (building the bf16 operand pieces costs more than the
   // products save at these sizes)
-  if (n > 0 && mfma_ok && (bf16_mode || c->sl_acc_path == 1)) {
+  if (mfma) {
     const int np = bf16_mode ? 2 : 3;
     const size_t mlds = (size_t)np * R * kMS * 2 + 3 * kMT * 4;
     timer_begin(c, "sl_accumulate", s);
@@ -1815,11 +1860,8 @@ static int sl_accumulate_run(Context* c, const float* x, const float* y, const f
   }
   // cell-ordered form: (lmax+1)^2 rows x chunks of radial orders per lane,
   // LDS for the per-wave Y rows and the float64 wave reduction
-  const DepShape dsh = dep_shape(R, c->nmax, kSlShapes, kSlDepShapes, c->sl_dep_shape);
-  const size_t dlds = std::max((size_t)4 * sl_dep_rows(R) * kDepStride * sizeof(float),
-                               (size_t)4 * K * sizeof(double));
   const float4* sorted = nullptr;
-  if (n >= c->order_min && n > 0 && dsh.ppt > 0 && dlds <= 64 * 1024) {
+  if (ordered) {
     rc = order_particles(c, 1, x, y, z, m, n, off_dev, nsnap, s, &sorted, off);
     if (rc) return rc;
   }
@@ -1897,22 +1939,17 @@ static int eof_accumulate_noalloc_run(Context* c, const float* x, const float* y
   // at most kScratchDoubles / K segments of K partial sums each
   const int64_t cap = std::min<int64_t>(std::max<int64_t>(c->eof_acc_blocks, 1),
                                         noalloc::kScratchDoubles / K);
-  AccPlan P = plan_single(cap, n, kTile);
+  AccPlan P = plan_input_order(cap, n);
   if (P.S.nseg * (int64_t)K > noalloc::kScratchDoubles)
     return set_error(c, BFE_ELIMIT, "eof_accumulate_noalloc: %lld partial sums > %lld",
                      (long long)(P.S.nseg * (int64_t)K), (long long)noalloc::kScratchDoubles);
   double* partials = c->noalloc_scratch;
   const EOFGeom g = eof_geom(c);
-  const int opt = (K + 255) / 256;
   if (n == 0) {
     hipLaunchKernelGGL(fill_f64_kernel, dim3((unsigned)((P.S.nseg * K + 255) / 256)), dim3(256), 0, s,
                        partials, P.S.nseg * (int64_t)K);
-  } else if (opt == 1) {
-    hipLaunchKernelGGL(eof_accumulate_kernel<1>, dim3(P.grid), dim3(256), 0, s, x, y, z, m, P.S, g, c->eof_pot32, K, partials);
-  } else if (opt == 2) {
-    hipLaunchKernelGGL(eof_accumulate_kernel<2>, dim3(P.grid), dim3(256), 0, s, x, y, z, m, P.S, g, c->eof_pot32, K, partials);
   } else {
-    hipLaunchKernelGGL(eof_accumulate_kernel<4>, dim3(P.grid), dim3(256), 0, s, x, y, z, m, P.S, g, c->eof_pot32, K, partials);
+    eof_input_order_launch(P, x, y, z, m, g, c->eof_pot32, K, partials, s);
   }
   BFE_HIP(c, hipGetLastError());
   const int nc = (c->mmax + 1) * c->norder;
