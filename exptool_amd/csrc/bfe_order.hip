@@ -37,8 +37,17 @@
 namespace bfe {
 
 constexpr int kSortThreads = 256;
-constexpr int kSortIPT = 8;                              // items per thread (2 and 4 measured slower)
+constexpr int kSortIPT = 8;                              // items per thread at 2M points (2 and 4 measured slower)
 constexpr int kSortTile = kSortThreads * kSortIPT;       // items per tile (block)
+// Items per thread of small sorts: a sort of few tiles waits for one tile's
+// serial work, not for memory, so tiles of 512 items while they are at most two
+// per CU.  Whole accumulates (disc / halo) with 1, 2, 4 and 8 items per thread:
+//   66 000: 71.0 71.3 75.3 83.2 / 53.6 53.2 56.3 64.8 us
+//  130 000: 73.8 72.6 75.6 83.3 / 59.7 57.0 59.0 74.4 us
+//  262 144: 82.5 77.9 78.4 85.4 / 77.5 73.1 72.9 82.2 us
+//  500 000: 108  97.6 96.7 100  / 94.2 82.8 80.8 83.8 us
+constexpr int kSortSmallIPT = 2;
+constexpr int64_t kSortSmallMax = 262144;
 constexpr int kRadix = 256;                              // 8-bit digits
 
 // Snapshot of point i for concatenated snapshots: the last s with off[s] <= i.
@@ -217,34 +226,37 @@ __device__ __forceinline__ uint32_t block_scan_incl(uint32_t v, uint32_t* wsum) 
 struct TileRange {
   int64_t t0, end;
 };
+template <int IPT>
 __device__ __forceinline__ TileRange sort_tile(const int64_t* __restrict__ tb, int64_t n) {
   if (tb) return TileRange{tb[2 * blockIdx.x], tb[2 * blockIdx.x + 1]};
-  const int64_t t0 = (int64_t)blockIdx.x * kSortTile;
-  return TileRange{t0, t0 + kSortTile < n ? t0 + kSortTile : n};
+  const int64_t t0 = (int64_t)blockIdx.x * (kSortThreads * IPT);
+  return TileRange{t0, t0 + kSortThreads * IPT < n ? t0 + kSortThreads * IPT : n};
 }
+template <int IPT>
 __device__ __forceinline__ int64_t sort_item(const TileRange& r, int i) {
   const int t = threadIdx.x;
-  return r.t0 + (int64_t)((t >> 6) * kSortIPT + i) * 64 + (t & 63);
+  return r.t0 + (int64_t)((t >> 6) * IPT + i) * 64 + (t & 63);
 }
 
 // Digit histogram of each tile: counts[d * nb + tile].  First pass (kin ==
 // NULL): keys computed from the source and written to kfirst.
+template <int IPT>
 __global__ __launch_bounds__(kSortThreads) void sort_count_kernel(
     KeySrc S, const uint32_t* __restrict__ kin, uint32_t* __restrict__ kfirst, int64_t n,
     const int64_t* __restrict__ tb, const int* __restrict__ tseg, int shift,
     uint32_t* __restrict__ counts, int nb) {
   __shared__ uint32_t hist[4][kRadix];
   const int t = threadIdx.x, w = t >> 6, l = t & 63;
-  const TileRange tr = sort_tile(tb, n);
+  const TileRange tr = sort_tile<IPT>(tb, n);
   // segmented sort: digits of the key less its segment's first key, so
   // that the passes cover the cell bits only
   const int tsnap = tseg ? tseg[blockIdx.x] : -1;
   const uint32_t kb = tseg ? (uint32_t)tsnap * S.ncell : 0u;
   for (int j = t; j < 4 * kRadix; j += kSortThreads) (&hist[0][0])[j] = 0u;
-  uint32_t key[kSortIPT];
+  uint32_t key[IPT];
 #pragma unroll
-  for (int i = 0; i < kSortIPT; ++i) {
-    const int64_t idx = sort_item(tr, i);
+  for (int i = 0; i < IPT; ++i) {
+    const int64_t idx = sort_item<IPT>(tr, i);
     key[i] = 0u;
     if (idx < tr.end) {
       if (kin) {
@@ -259,8 +271,8 @@ __global__ __launch_bounds__(kSortThreads) void sort_count_kernel(
   // counts only, so LDS atomics (lanes on one digit serialise in the LDS,
   // no worse than the eight ballots of a rank)
 #pragma unroll
-  for (int i = 0; i < kSortIPT; ++i) {
-    const bool live = sort_item(tr, i) < tr.end;
+  for (int i = 0; i < IPT; ++i) {
+    const bool live = sort_item<IPT>(tr, i) < tr.end;
     const uint32_t d = ((key[i] - kb) >> shift) & (kRadix - 1);
     if (live) atomicAdd(&hist[w][d], 1u);
   }
@@ -391,6 +403,7 @@ __global__ __launch_bounds__(kSortThreads) void sort_rowscan_seg_kernel(
 // Segmented sort (tb != NULL): tile b belongs to segment tseg[b], whose digit
 // totals are totals[tseg[b] * kRadix + d] and whose items start at
 // segoff[tseg[b]].
+template <int IPT>
 __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(
     KeySrc S, const uint32_t* __restrict__ kin, const float4* __restrict__ vin, int64_t n,
     const int64_t* __restrict__ tb, const int* __restrict__ tseg,
@@ -401,18 +414,18 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(
   __shared__ uint32_t dstart[kRadix];    // tile-local start of each digit
   __shared__ uint32_t gpos[kRadix];      // output position of the tile's first item of each digit
   __shared__ uint32_t wsum[4];
-  __shared__ uint32_t skey[kSortTile];
-  __shared__ float4 sval[kSortTile];
+  __shared__ uint32_t skey[kSortThreads * IPT];
+  __shared__ float4 sval[kSortThreads * IPT];
   const int t = threadIdx.x, w = t >> 6, l = t & 63;
-  const TileRange tr = sort_tile(tb, n);
+  const TileRange tr = sort_tile<IPT>(tb, n);
   const int sg = tseg ? tseg[blockIdx.x] : 0;
   const uint32_t kb = tseg ? (uint32_t)sg * S.ncell : 0u;
   for (int j = t; j < 4 * kRadix; j += kSortThreads) (&hist[0][0])[j] = 0u;
-  uint32_t key[kSortIPT];
-  float4 val[kSortIPT];
+  uint32_t key[IPT];
+  float4 val[IPT];
 #pragma unroll
-  for (int i = 0; i < kSortIPT; ++i) {
-    const int64_t idx = sort_item(tr, i);
+  for (int i = 0; i < IPT; ++i) {
+    const int64_t idx = sort_item<IPT>(tr, i);
     key[i] = 0u;
     val[i] = make_float4(0.f, 0.f, 0.f, 0.f);
     if (idx < tr.end) {
@@ -423,10 +436,10 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(
   __syncthreads();
   // rank within the wave: items of earlier slots, then lower lanes of this slot
   const uint64_t lt = (1ull << l) - 1ull;
-  uint32_t rank[kSortIPT];
+  uint32_t rank[IPT];
 #pragma unroll
-  for (int i = 0; i < kSortIPT; ++i) {
-    const bool live = sort_item(tr, i) < tr.end;
+  for (int i = 0; i < IPT; ++i) {
+    const bool live = sort_item<IPT>(tr, i) < tr.end;
     const uint32_t d = ((key[i] - kb) >> shift) & (kRadix - 1);
     const uint64_t mk = match_digit(d, live);
     uint32_t before = 0u;
@@ -450,8 +463,8 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(
   gpos[t] = gb + pre;
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < kSortIPT; ++i) {
-    if (sort_item(tr, i) < tr.end) {
+  for (int i = 0; i < IPT; ++i) {
+    if (sort_item<IPT>(tr, i) < tr.end) {
       const uint32_t d = ((key[i] - kb) >> shift) & (kRadix - 1);
       const uint32_t lp = dstart[d] + hist[w][d] + rank[i];
       skey[lp] = key[i];
@@ -480,7 +493,11 @@ struct OrderLayout {
   size_t k0, ka, kb, va, vb, perm, energy, counts, totals, tb, ts, total;
 };
 
-static int sort_tiles(int64_t n) { return (int)((n + kSortTile - 1) / kSortTile); }
+static int sort_ipt(int64_t n) { return n <= kSortSmallMax ? kSortSmallIPT : kSortIPT; }
+static int sort_tiles(int64_t n) {
+  const int64_t tile = (int64_t)kSortThreads * sort_ipt(n);
+  return (int)((n + tile - 1) / tile);
+}
 
 static OrderLayout order_layout(int64_t n, int nb, int nseg) {
   OrderLayout L;
@@ -584,8 +601,13 @@ static int sort_source(Context* c, const KeySrc& S, int64_t n, uint64_t nkeys, b
     const uint32_t* kin = p == 0 ? (const uint32_t*)k0 : kbuf[(p - 1) & 1];
     const float4* vin = p == 0 ? nullptr : vbuf[(p - 1) & 1];
     uint32_t* kout = (!last || want_keys) ? kbuf[p & 1] : nullptr;
-    hipLaunchKernelGGL(sort_count_kernel, dim3((unsigned)nb), dim3(kSortThreads), 0, s, S,
-                       p == 0 ? nullptr : kin, k0, n, tb, ts, shift, counts, nb);
+    const bool small = !segmented && sort_ipt(n) == kSortSmallIPT;
+    auto count = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)nb), dim3(kSortThreads), 0, s, S,
+                         p == 0 ? nullptr : kin, k0, n, tb, ts, shift, counts, nb);
+    };
+    if (small) count(sort_count_kernel<kSortSmallIPT>);
+    else count(sort_count_kernel<kSortIPT>);
     BFE_HIP(c, hipGetLastError());
     if (segmented)
       hipLaunchKernelGGL(sort_rowscan_seg_kernel, dim3(kRadix), dim3(kSortThreads), 0, s, counts,
@@ -594,9 +616,13 @@ static int sort_source(Context* c, const KeySrc& S, int64_t n, uint64_t nkeys, b
       hipLaunchKernelGGL(sort_rowscan_kernel, dim3(kRadix), dim3(kSortThreads), 0, s, counts, nb,
                          totals);
     BFE_HIP(c, hipGetLastError());
-    hipLaunchKernelGGL(sort_scatter_kernel, dim3((unsigned)nb), dim3(kSortThreads), 0, s, S, kin,
-                       vin, n, tb, ts, segmented ? S.off : nullptr, shift, counts, totals, nb,
-                       kout, vbuf[p & 1], (last && want_perm) ? perm : nullptr);
+    auto scatter = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)nb), dim3(kSortThreads), 0, s, S, kin, vin, n, tb, ts,
+                         segmented ? S.off : nullptr, shift, counts, totals, nb, kout, vbuf[p & 1],
+                         (last && want_perm) ? perm : nullptr);
+    };
+    if (small) scatter(sort_scatter_kernel<kSortSmallIPT>);
+    else scatter(sort_scatter_kernel<kSortIPT>);
     BFE_HIP(c, hipGetLastError());
   }
   out->values = vbuf[(passes - 1) & 1];
