@@ -1494,7 +1494,8 @@ __global__ __launch_bounds__(256) void eof_mfma_table_kernel(const float* __rest
 struct AccPlan {
   Segments S;
   int grid;
-  std::vector<int64_t> segb, rowb;  // batch only (host copies)
+  int64_t len;                // batch: particles per segment
+  std::vector<int64_t> rowb;  // batch: first segment of each snapshot
 };
 
 static AccPlan plan_single(int64_t cap, int64_t n, int tile) {
@@ -1503,6 +1504,7 @@ static AccPlan plan_single(int64_t cap, int64_t n, int tile) {
   int64_t nseg = ntiles < cap ? ntiles : cap;
   if (nseg < 1) nseg = 1;
   const int64_t per = (ntiles + nseg - 1) / nseg;
+  P.len = 0;
   P.S.segb = nullptr;
   P.S.seglen = (per > 0 ? per : 1) * tile;
   P.S.n = n;
@@ -1520,44 +1522,35 @@ static AccPlan plan_batch(int64_t cap, int64_t seg_tiles, const int64_t* off, in
     seg_tiles = (total_tiles + cap - 1) / cap;
     if (seg_tiles < 1) seg_tiles = 1;
   }
+  P.len = seg_tiles * tile;
   P.rowb.push_back(0);
-  P.segb.push_back(off[0]);
-  for (int q = 0; q < nsnap; ++q) {
-    const int64_t b = off[q], e = off[q + 1];
-    for (int64_t p = b; p < e; p += seg_tiles * tile) {
-      const int64_t pe = p + seg_tiles * tile < e ? p + seg_tiles * tile : e;
-      P.segb.push_back(pe);
-    }
-    if (e == b) P.segb.push_back(e);   // empty snapshot: one empty segment
-    P.rowb.push_back((int64_t)P.segb.size() - 1);
-  }
-  P.S.segb = nullptr;  // device copy set by upload_plan
+  for (int q = 0; q < nsnap; ++q)   // an empty snapshot has one empty segment
+    P.rowb.push_back(P.rowb[q] + std::max<int64_t>((off[q + 1] - off[q] + P.len - 1) / P.len, 1));
+  P.S.segb = nullptr;  // device copy set by place_plan
   P.S.seglen = 0;
   P.S.n = off[nsnap];
-  P.S.nseg = (int64_t)P.segb.size() - 1;
+  P.S.nseg = P.rowb.back();
   P.grid = (int)(P.S.nseg < cap ? P.S.nseg : cap);
   return P;
 }
 
-// Copies the batch plan and the snapshot offsets to device memory behind the
-// partials in scratch (waiting first for earlier work that may still read it).
-static int upload_plan(Context* c, AccPlan& P, size_t pbytes, const int64_t* off, int nsnap,
-                       hipStream_t s, const int64_t** rowb_dev, const int64_t** off_dev) {
+// Writes the batch plan and the snapshot offsets to device memory behind the
+// partials in scratch, on the stream.
+static int place_plan(Context* c, AccPlan& P, size_t pbytes, const int64_t* off, int nsnap,
+                      hipStream_t s, const int64_t** rowb_dev, const int64_t** off_dev) {
   const size_t segb_off = (pbytes + 255) & ~(size_t)255;
-  const size_t rowb_off = segb_off + ((P.segb.size() * 8 + 255) & ~(size_t)255);
+  const size_t rowb_off = segb_off + ((((size_t)P.S.nseg + 1) * 8 + 255) & ~(size_t)255);
   const size_t offs_off = rowb_off + ((P.rowb.size() * 8 + 255) & ~(size_t)255);
   int rc = ensure_scratch(c, offs_off + ((size_t)nsnap + 1) * 8 + 256);
   if (rc) return rc;
-  BFE_HIP(c, hipStreamSynchronize(s));
-  int64_t* segb = (int64_t*)((char*)c->scratch + segb_off);
-  int64_t* rowb = (int64_t*)((char*)c->scratch + rowb_off);
-  int64_t* offs = (int64_t*)((char*)c->scratch + offs_off);
-  BFE_HIP(c, hipMemcpy(segb, P.segb.data(), P.segb.size() * 8, hipMemcpyHostToDevice));
-  BFE_HIP(c, hipMemcpy(rowb, P.rowb.data(), P.rowb.size() * 8, hipMemcpyHostToDevice));
-  BFE_HIP(c, hipMemcpy(offs, off, ((size_t)nsnap + 1) * 8, hipMemcpyHostToDevice));
-  P.S.segb = segb;
-  *rowb_dev = rowb;
-  *off_dev = offs;
+  BatchPieces d;
+  d.bounds = (int64_t*)((char*)c->scratch + segb_off);
+  d.first = (int64_t*)((char*)c->scratch + rowb_off);
+  d.off = (int64_t*)((char*)c->scratch + offs_off);
+  if ((rc = batch_pieces(c, off, nsnap, P.rowb, P.len, d, s))) return rc;
+  P.S.segb = d.bounds;
+  *rowb_dev = d.first;
+  *off_dev = d.off;
   return 0;
 }
 
@@ -1697,7 +1690,7 @@ static int eof_accumulate_mfma_run(Context* c, const float* x, const float* y, c
                   : plan_single(c->eof_acc_blocks, n, kTile);
   const int64_t* rowb = nullptr;
   const int64_t* off_dev = nullptr;
-  if (off && (rc = upload_plan(c, P, 0, off, nsnap, s, &rowb, &off_dev))) return rc;
+  if (off && (rc = place_plan(c, P, 0, off, nsnap, s, &rowb, &off_dev))) return rc;
   if ((rc = ensure_mfma_work(c, total))) return rc;
   float* cs = (float*)c->mfma_work;
   __bf16* Ahi = (__bf16*)((char*)c->mfma_work + a_off);
@@ -1756,7 +1749,7 @@ static int eof_accumulate_run(Context* c, const float* x, const float* y, const 
   const int64_t* off_dev = nullptr;
   int rc;
   if (off) {
-    rc = upload_plan(c, P, need, off, nsnap, s, &rowb, &off_dev);   // partials | plan
+    rc = place_plan(c, P, need, off, nsnap, s, &rowb, &off_dev);   // partials | plan
   } else {
     rc = ensure_scratch(c, need);
   }
@@ -1830,7 +1823,7 @@ static int sl_accumulate_run(Context* c, const float* x, const float* y, const f
   const size_t pbytes = (size_t)P.S.nseg * K * sizeof(double);
   const int64_t* rowb = nullptr;
   const int64_t* off_dev = nullptr;
-  int rc = off ? upload_plan(c, P, pbytes, off, nsnap, s, &rowb, &off_dev) : ensure_scratch(c, pbytes);
+  int rc = off ? place_plan(c, P, pbytes, off, nsnap, s, &rowb, &off_dev) : ensure_scratch(c, pbytes);
   if (rc) return rc;
   double* partials = (double*)c->scratch;
   SLGeom g = sl_geom(c);

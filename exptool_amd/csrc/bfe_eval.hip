@@ -953,10 +953,10 @@ extern "C" int bfe_field_eval_batch(bfe_ctx* h, const float* x, const float* y, 
     BFE_HIP(c, hipMalloc(&c->batch_off, ((size_t)nsnap + 1) * sizeof(int64_t)));
     c->batch_off_cap = (size_t)nsnap + 1;
   }
-  // the offsets buffer may still be read by an earlier call on this stream
-  BFE_HIP(c, hipStreamSynchronize(s));
-  BFE_HIP(c, hipMemcpy(c->batch_off, offsets, ((size_t)nsnap + 1) * sizeof(int64_t),
-                       hipMemcpyHostToDevice));
+  BatchPieces d;
+  d.off = c->batch_off;
+  int rc = batch_pieces(c, offsets, nsnap, {}, 0, d, s);
+  if (rc) return rc;
   const size_t slf = sl_fold_floats(c), eoff = eof_fold_floats(c);
   FieldTables T;
   T.slg = sl_geom(c);
@@ -970,7 +970,7 @@ extern "C" int bfe_field_eval_batch(bfe_ctx* h, const float* x, const float* y, 
   T.srot = sin(rotpos);
   const uint32_t* sorted = nullptr;
   const float4* pts = nullptr;
-  int rc = order_points(c, T, x, y, z, n, s, nullptr, c->batch_off, nsnap, &sorted, &pts, offsets);
+  rc = order_points(c, T, x, y, z, n, s, nullptr, c->batch_off, nsnap, &sorted, &pts, offsets);
   if (rc) return rc;
   // results go through a float4 per point, split coalesced (as field_eval_run)
   rc = ensure_scratch(c, (size_t)n * sizeof(float4));

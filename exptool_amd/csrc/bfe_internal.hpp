@@ -242,6 +242,21 @@ inline EOFGeom eof_geom(const Context* c) {
                  c->xmin, c->dx, c->ymin, c->dy, 1.0 / c->hscale, 1.0 / c->dx, 1.0 / c->dy};
 }
 
+// Device tables of a batch's snapshots, each optional: off[nsnap + 1] and
+// first[nsnap + 1]; of the pieces bounds[pieces + 1] (ends, for pieces that
+// follow one another), pair[2 pieces] (start, end) and snap[pieces].
+struct BatchPieces {
+  int64_t* off = nullptr;
+  int64_t* first = nullptr;
+  int64_t* bounds = nullptr;
+  int64_t* pair = nullptr;
+  int* snap = nullptr;
+};
+// Writes them on stream s from the host's offsets and first pieces (empty:
+// offsets only) for pieces of len items.  Refuses a capturing stream.
+int batch_pieces(Context* c, const int64_t* off, int nsnap, const std::vector<int64_t>& first,
+                 int64_t len, const BatchPieces& d, hipStream_t s);
+
 struct FieldTables;
 // Permutation perm[j] = i listing the points in order of their SL radial
 // cell and cos(theta) bin, so that the lanes of a block share SL nodes and a

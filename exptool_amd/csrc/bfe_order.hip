@@ -38,7 +38,6 @@ namespace bfe {
 
 constexpr int kSortThreads = 256;
 constexpr int kSortIPT = 8;                              // items per thread at 2M points (2 and 4 measured slower)
-constexpr int kSortTile = kSortThreads * kSortIPT;       // items per tile (block)
 // Items per thread of small sorts: a sort of few tiles waits for one tile's
 // serial work, not for memory, so tiles of 512 items while they are at most two
 // per CU.  Whole accumulates (disc / halo) with 1, 2, 4 and 8 items per thread:
@@ -49,6 +48,70 @@ constexpr int kSortTile = kSortThreads * kSortIPT;       // items per tile (bloc
 constexpr int kSortSmallIPT = 2;
 constexpr int64_t kSortSmallMax = 262144;
 constexpr int kRadix = 256;                              // 8-bit digits
+
+// Pieces of a batch's snapshots (accumulate segments, sort tiles): snapshot q
+// is cut into pieces of `len` items, the first of them piece first[q].  One
+// block of threads a chunk of snapshots, the offsets as kernel arguments, so
+// that a batch call neither waits for the stream nor copies from the host
+// (five copies and a wait a call, 160 us of an idle device, before; 5 us now).
+constexpr int kPieceSnaps = 128;
+struct PieceChunk {
+  int q0, nq;                     // snapshots [q0, q0 + nq)
+  int64_t off[kPieceSnaps + 1], first[kPieceSnaps + 1];
+};
+__global__ __launch_bounds__(256) void batch_pieces_kernel(PieceChunk c, int64_t len, BatchPieces d) {
+  __shared__ int64_t off[kPieceSnaps + 1], first[kPieceSnaps + 1];
+  const int t = threadIdx.x;
+  if (t <= c.nq) {
+    off[t] = c.off[t];
+    first[t] = c.first[t];
+  }
+  __syncthreads();
+  if (blockIdx.x == 0 && t <= c.nq) {
+    if (d.off) d.off[c.q0 + t] = off[t];
+    if (d.first) d.first[c.q0 + t] = first[t];
+    if (d.bounds && c.q0 + t == 0) d.bounds[0] = off[0];
+  }
+  const int64_t p = first[0] + (int64_t)blockIdx.x * 256 + t;
+  if (p >= first[c.nq]) return;
+  int lo = 0, hi = c.nq - 1;      // the snapshot of piece p: the last with first[q] <= p
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (first[mid] <= p) lo = mid; else hi = mid - 1;
+  }
+  const int64_t a = off[lo] + (p - first[lo]) * len;
+  const int64_t e = a + len < off[lo + 1] ? a + len : off[lo + 1];
+  if (d.bounds) d.bounds[p + 1] = e;
+  if (d.pair) {
+    d.pair[2 * p] = a;
+    d.pair[2 * p + 1] = e;
+  }
+  if (d.snap) d.snap[p] = c.q0 + lo;
+}
+
+int batch_pieces(Context* c, const int64_t* off, int nsnap, const std::vector<int64_t>& first,
+                 int64_t len, const BatchPieces& d, hipStream_t s) {
+  // the tables live in growing workspaces, so a captured call would hold them
+  // past a later growth
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  BFE_HIP(c, hipStreamIsCapturing(s, &cap));
+  if (cap != hipStreamCaptureStatusNone)
+    return check_hip(c, hipErrorStreamCaptureUnsupported, "batch call on a capturing stream");
+  for (int q0 = 0; q0 < nsnap; q0 += kPieceSnaps) {
+    PieceChunk k;
+    k.q0 = q0;
+    k.nq = std::min(kPieceSnaps, nsnap - q0);
+    for (int j = 0; j <= kPieceSnaps; ++j) {
+      k.off[j] = off[q0 + std::min(j, k.nq)];
+      k.first[j] = first.empty() ? 0 : first[q0 + std::min(j, k.nq)];
+    }
+    const int64_t np = k.first[k.nq] - k.first[0];
+    hipLaunchKernelGGL(batch_pieces_kernel, dim3((unsigned)std::max<int64_t>((np + 255) / 256, 1)),
+                       dim3(256), 0, s, k, len, d);
+    BFE_HIP(c, hipGetLastError());
+  }
+  return 0;
+}
 
 // Snapshot of point i for concatenated snapshots: the last s with off[s] <= i.
 __device__ __forceinline__ int snapshot_of(const int64_t* __restrict__ off, int nsnap, int64_t i) {
@@ -220,8 +283,8 @@ __device__ __forceinline__ uint32_t block_scan_incl(uint32_t v, uint32_t* wsum) 
   return v + add;
 }
 
-// Items [t0, end) of tile b: b kSortTile and on, or the bounds tb[2b], tb[2b + 1]
-// (at most kSortTile items) of a segmented sort.  Slot i of thread (w, l)
+// Items [t0, end) of tile b: b kSortThreads IPT and on, or the bounds tb[2b], tb[2b + 1]
+// (at most kSortThreads IPT items) of a segmented sort.  Slot i of thread (w, l)
 // holds item t0 + (w kSortIPT + i) 64 + l.
 struct TileRange {
   int64_t t0, end;
@@ -555,38 +618,33 @@ static int sort_source(Context* c, const KeySrc& S, int64_t n, uint64_t nkeys, b
   if (n > (int64_t)0x7fffffff) return set_error(c, BFE_ELIMIT, "order: n = %lld > 2^31 - 1", (long long)n);
   if (nkeys > 0xffffffffull) return set_error(c, BFE_ELIMIT, "order: too many table cells");
   const bool segmented = off_host && S.off && S.nsnap > 1;
-  std::vector<int64_t> tbv;
-  std::vector<int> tsv;
+  const int ipt = sort_ipt(n);
+  std::vector<int64_t> first;     // segmented: the first tile of each snapshot
   if (segmented) {
+    const int64_t tile = (int64_t)kSortThreads * ipt;
+    first.assign(1, 0);
     for (int q = 0; q < S.nsnap; ++q)
-      for (int64_t a = off_host[q]; a < off_host[q + 1]; a += kSortTile) {
-        tbv.push_back(a);
-        tbv.push_back(std::min(a + (int64_t)kSortTile, off_host[q + 1]));
-        tsv.push_back(q);
-      }
-    if ((int64_t)tsv.size() > (int64_t)0x7fffffff)
-      return set_error(c, BFE_ELIMIT, "order: too many tiles");
+      first.push_back(first[q] + (off_host[q + 1] - off_host[q] + tile - 1) / tile);
+    if (first.back() > (int64_t)0x7fffffff) return set_error(c, BFE_ELIMIT, "order: too many tiles");
   }
   const uint64_t span = segmented ? (uint64_t)S.ncell : nkeys;
   int bits = 1;
   while (bits < 32 && (1ull << bits) < span) ++bits;
   const int passes = (bits + 7) / 8;
-  const int nb = segmented ? (int)tsv.size() : sort_tiles(n);
+  const int nb = segmented ? (int)first.back() : sort_tiles(n);
   const OrderLayout L = order_layout(n, nb, segmented ? S.nsnap : 1);
   int rc = ensure_order(c, L.total);
   if (rc) return rc;
   const int64_t* tb = nullptr;
   const int* ts = nullptr;
   if (segmented && nb > 0) {
-    // the tile table is read by this call's kernels only; earlier work on s
-    // may still read the buffer
-    BFE_HIP(c, hipStreamSynchronize(s));
-    int64_t* tbd = (int64_t*)((char*)c->order + L.tb);
-    int* tsd = (int*)((char*)c->order + L.ts);
-    BFE_HIP(c, hipMemcpy(tbd, tbv.data(), tbv.size() * sizeof(int64_t), hipMemcpyHostToDevice));
-    BFE_HIP(c, hipMemcpy(tsd, tsv.data(), tsv.size() * sizeof(int), hipMemcpyHostToDevice));
-    tb = tbd;
-    ts = tsd;
+    BatchPieces d;
+    d.pair = (int64_t*)((char*)c->order + L.tb);
+    d.snap = (int*)((char*)c->order + L.ts);
+    rc = batch_pieces(c, off_host, S.nsnap, first, (int64_t)kSortThreads * ipt, d, s);
+    if (rc) return rc;
+    tb = d.pair;
+    ts = d.snap;
   }
   char* base = (char*)c->order;
   uint32_t* k0 = (uint32_t*)(base + L.k0);
@@ -601,7 +659,7 @@ static int sort_source(Context* c, const KeySrc& S, int64_t n, uint64_t nkeys, b
     const uint32_t* kin = p == 0 ? (const uint32_t*)k0 : kbuf[(p - 1) & 1];
     const float4* vin = p == 0 ? nullptr : vbuf[(p - 1) & 1];
     uint32_t* kout = (!last || want_keys) ? kbuf[p & 1] : nullptr;
-    const bool small = !segmented && sort_ipt(n) == kSortSmallIPT;
+    const bool small = ipt == kSortSmallIPT;
     auto count = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3((unsigned)nb), dim3(kSortThreads), 0, s, S,
                          p == 0 ? nullptr : kin, k0, n, tb, ts, shift, counts, nb);

@@ -277,8 +277,8 @@ int bfe_field_set_batch(bfe_ctx* ctx, const double* eof_cos, const double* eof_s
 /* Fields.return_forces_cart (potential.py:445-497) of the batch fields: the
  * points of snapshot s, [offsets[s], offsets[s+1]) (HOST offsets, nsnap as
  * given to bfe_field_set_batch), are evaluated in field s.  Outputs as
- * bfe_field_eval_cart (sums; no components).  Blocks the host until earlier
- * work on `stream` is done (the offsets are copied to the device). */
+ * bfe_field_eval_cart (sums; no components).  The offsets are read before the
+ * call returns; batch calls are refused on a capturing stream. */
 int bfe_field_eval_batch(bfe_ctx* ctx, const float* x, const float* y, const float* z,
                          const int64_t* offsets, int nsnap, double rotpos, float* fx, float* fy,
                          float* fz, float* pot, void* stream);

@@ -50,3 +50,41 @@ def test_sort_edges(big, particles, n):  # noqa: F811
     s.set_tuning("order_min", 65536)
     for a, b in zip(*out):
         assert (a is None and b is None) or torch.equal(a, b)
+
+
+@pytest.mark.parametrize("omin", [1 << 40, 1], ids=["input", "cells"])
+@pytest.mark.parametrize("nsnap", [2, 127, 128, 129, 257])
+def test_batch_pieces_edges(nsnap, omin):
+    """Batches around the 128 snapshots of a table chunk, with empty snapshots
+    and snapshots at the edges of a segment and a tile: every snapshot as its
+    own call (another segment plan regroups the float32 sums), every point's
+    bits as in its own field."""
+    import torch
+    from exptool_amd.bfe import BFESystem
+    from exptool_amd.utils import workloads as W
+    st, et = W.disc_halo_tables(seed=2, n_eof_sample=4000, lmax_s=10, nmax_s=8,
+                                eof=dict(mmax=3, norder=6, numx=24, numy=16),
+                                sl=dict(lmax=3, nmax=6, numr=200))
+    s = BFESystem(sl=st, eof=et)
+    rng = np.random.default_rng(nsnap)
+    counts = rng.choice([0, 1, 63, 64, 65, 255, 256, 257, 511, 512, 513, 1500], nsnap)
+    counts[:2] = (0, 513)
+    d, h = W.disc_halo_particles(int(counts.sum()), int(counts.sum()), seed=8)
+    d, h = ([torch.tensor(np.asarray(a, np.float32), device="cuda") for a in p] for p in (d, h))
+    s.set_tuning("order_min", omin)
+    c, sn = s.eof_accumulate_batch(*d, counts)
+    hl = s.sl_accumulate_batch(*h, counts)
+    s.set_field_batch(c, sn, hl)
+    f = s.field_forces_batch(*h[:3], counts, rotpos=0.3)
+    o = np.concatenate([[0], np.cumsum(counts)])
+    for q in sorted({0, 1, 2 % nsnap, nsnap // 2, nsnap - 2, nsnap - 1}):
+        a, b = int(o[q]), int(o[q + 1])
+        cq, sq = (v.cpu().numpy() for v in s.eof_accumulate(*(v[a:b] for v in d)))
+        hq = s.sl_accumulate(*(v[a:b] for v in h)).cpu().numpy()
+        assert block_rel_eof(c[q].cpu().numpy(), cq) <= TOL
+        assert block_rel_eof(sn[q].cpu().numpy()[1:], sq[1:]) <= TOL
+        assert block_rel_sl(hl[q].cpu().numpy(), hq, 3) <= TOL
+        if b > a:
+            s.set_field(c[q], sn[q], hl[q])
+            for u, v in zip(f, s.field_forces(*(v[a:b] for v in h[:3]), rotpos=0.3)):
+                assert torch.equal(u[a:b], v)
