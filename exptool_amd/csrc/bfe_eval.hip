@@ -9,100 +9,142 @@
 namespace bfe {
 
 struct SLFoldArgs {
-  double lmul[kMaxL + 1];  // per-l multiplier (halofac, 0 for skipped l)
+  double mul[kMaxLM];  // per-pair multiplier: N_lm times halofac (0 for skipped l)
   int lmax, nmax_use;
 };
 
-// Four lanes per (radial node i, (l, m) pair p in m-major order), lane q
-// summing n = q, q + 4, ...: E and Dn at i and i+1 and G at c-1, c, c+1
-// (c = max(i, 1)) are summed over n in float64 from the float64 scaled
-// tables S = [ef/sqrt(ev), ef sqrt(ev), ef p0/sqrt(ev)] ([l][i][n] each),
-// the four partial sums are combined across the lanes, D1/D2 formed, and the
-// blocks rounded once to float32 (layout in bfe_field.hpp; the last node,
-// never a cell start, is zero).  grid.y runs over coefficient sets: set q
-// reads coef + q * coef_stride and writes out + q * out_stride.
+// Four lanes per (kFoldRows radial nodes from i0, (l, m) pair p in m-major
+// order), lane q summing radial orders q, q + 4, ...: the sums of a table row are
+// shared by the nodes that read it (a node takes rows i and i + 1 of E and D and
+// three rows of G), so kFoldRows nodes cost 3 kFoldRows + 4 rows instead of
+// 7 kFoldRows.  The four partial sums are combined across the lanes, D1/D2 formed,
+// and the blocks rounded once to float32 (layout in bfe_field.hpp; the last node,
+// never a cell start, is zero).  What bounds it is the latency and number of the
+// row gathers: lmax 6, nmax 20, numr 2000, one set / 12 sets, with one node a
+// group of lanes and seven rows each 12.3 / 75 us, one, two and four nodes with
+// shared rows 15.6 / 91, 10.5 / 55 and 10.3 / 47; smaller tables (lmax 4, numr
+// 1000) 6.4, then 8.0, 6.2 and 7.8.
+struct SLFoldIn {
+  const double* S;       // fold inputs
+  const double* coef;
+  int nmax, numr, nset;
+  float* out;
+  int64_t coef_stride, out_stride;
+};
 constexpr int kFoldLanes = 4;
-__global__ __launch_bounds__(256) void sl_fold_kernel(const double* __restrict__ S,
-                                                      const double* __restrict__ coef, int nmax,
-                                                      int numr, SLFoldArgs a,
-                                                      float* __restrict__ out, int64_t coef_stride,
-                                                      int64_t out_stride) {
-  coef += (size_t)blockIdx.y * coef_stride;
-  out += (size_t)blockIdx.y * out_stride;
-  const int np = sl_npairs(a.lmax);
-  const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+constexpr int kFoldRows = 2;
+__device__ __forceinline__ void sl_fold_block(const SLFoldIn& f, const SLFoldArgs& a, unsigned block,
+                                              int set) {
+  constexpr int R = kFoldRows;
+  const int np = sl_npairs(a.lmax), nmax = f.nmax, numr = f.numr;
+  const unsigned gid = block * blockDim.x + threadIdx.x;
   const int q = (int)(gid & (kFoldLanes - 1));
-  const int64_t idx = gid / kFoldLanes;
+  const unsigned idx = gid / kFoldLanes;
+  const int g = (int)(idx / (unsigned)np);
+  const int i0 = g * R;
   // groups of four lanes are whole within a wave, so a group leaves together
-  if (idx >= (int64_t)numr * np) return;
-  const int i = (int)(idx / np);
-  const int p = (int)(idx - (int64_t)i * np);
-  float* o = out + ((size_t)i * np + p) * 8;
-  float* od = out + (size_t)numr * np * 8 + ((size_t)i * np + p) * 4;
-  if (i == numr - 1) {
-    if (q == 0)
-      for (int k = 0; k < 8; ++k) o[k] = 0.f;
-    if (q == 1)
-      for (int k = 0; k < 4; ++k) od[k] = 0.f;
-    return;
-  }
-  int m = 0, rem = p;
-  while (rem > a.lmax - m) { rem -= a.lmax - m + 1; ++m; }
-  const int l = m + rem;
-  // N_lm (spheresl.py:858-861) folded into the table
-  double ratio = 1.0;
-  for (int k = 1; k <= m; ++k) ratio /= (double)(l - k + 1) * (double)(l + k);
-  double N = sqrt((0.5 * l + 0.25) / kPi * ratio);
-  if (m > 0) N *= 1.4142135623730951;
-  const double mul = a.lmul[l] * N;
-  const double* cc = coef + (size_t)(l * l + (m > 0 ? 2 * m - 1 : 0)) * nmax;
-  const double* cs = coef + (size_t)(l * l + 2 * m) * nmax;
+  if (i0 >= numr) return;
+  // lanes in l-major order, so that neighbours read the same rows
+  int l = 0, m = (int)(idx - (unsigned)g * (unsigned)np);
+  while (m > l) m -= ++l;
+  const int p = m * (a.lmax + 1) - m * (m - 1) / 2 + l - m;
+  const double mul = a.mul[p];
   const bool two = m > 0;
-  const int ctr = i == 0 ? 1 : i;
+  const double* c = f.coef + (size_t)set * f.coef_stride;
+  const double* cc = c + (size_t)(l * l + (two ? 2 * m - 1 : 0)) * nmax;
+  const double* cs = c + (size_t)(l * l + 2 * m) * nmax;
   const size_t plane = (size_t)(a.lmax + 1) * numr * nmax;
-  const double* E = S + ((size_t)l * numr + i) * nmax;   // rows i, i+1
-  const double* D = E + plane;
-  const double* G = S + 2 * plane + ((size_t)l * numr + ctr) * nmax;  // rows c-1, c, c+1
-  // v[cs]: E_i, E_i+1, Dn_i, Dn_i+1, G_c-1, G_c, G_c+1
-  double v[2][7] = {{0, 0, 0, 0, 0, 0, 0}, {0, 0, 0, 0, 0, 0, 0}};
-#pragma unroll 2
+  const double* E = f.S + (size_t)l * numr * nmax;
+  // rows of E and D: i0 .. i0 + R; of G: i0 - 1 .. i0 + R (the first node is
+  // centred on row 1, so there row -1 stands for row 2); rows past the table
+  // repeat its last
+  int re[R + 1], rg[R + 2];
+#pragma unroll
+  for (int k = 0; k <= R; ++k) re[k] = (i0 + k < numr ? i0 + k : numr - 1) * nmax;
+#pragma unroll
+  for (int k = 0; k < R + 2; ++k) {
+    const int r = i0 + k - 1;
+    rg[k] = (r < 0 ? 2 : r < numr ? r : numr - 1) * nmax;
+  }
+  double e[R + 1][2], d[R + 1][2], w[R + 2][2];
+#pragma unroll
+  for (int k = 0; k <= R; ++k) e[k][0] = e[k][1] = d[k][0] = d[k][1] = 0.0;
+#pragma unroll
+  for (int k = 0; k < R + 2; ++k) w[k][0] = w[k][1] = 0.0;
   for (int n = q; n < a.nmax_use; n += kFoldLanes) {
     const double c0 = cc[n] * mul;
     const double c1 = two ? cs[n] * mul : 0.0;
-    const double t[7] = {E[n], E[n + nmax], D[n], D[n + nmax], G[n - nmax], G[n], G[n + nmax]};
+    const double *En = E + n, *Dn = En + plane, *Gn = Dn + plane;
 #pragma unroll
-    for (int k = 0; k < 7; ++k) {
-      v[0][k] += c0 * t[k];
-      v[1][k] += c1 * t[k];
+    for (int k = 0; k <= R; ++k) {
+      const double te = En[re[k]], td = Dn[re[k]];
+      e[k][0] += c0 * te;
+      e[k][1] += c1 * te;
+      d[k][0] += c0 * td;
+      d[k][1] += c1 * td;
+    }
+#pragma unroll
+    for (int k = 0; k < R + 2; ++k) {
+      const double tg = Gn[rg[k]];
+      w[k][0] += c0 * tg;
+      w[k][1] += c1 * tg;
     }
   }
   // fixed-order combination: (q0 + q1) + (q2 + q3) on every lane of the group
+  auto sum = [](double v) {
+    v += __shfl_xor(v, 1, kFoldLanes);
+    return v + __shfl_xor(v, 2, kFoldLanes);
+  };
 #pragma unroll
-  for (int k = 0; k < 7; ++k) {
+  for (int h = 0; h < 2; ++h) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      v[h][k] += __shfl_xor(v[h][k], 1, kFoldLanes);
-      v[h][k] += __shfl_xor(v[h][k], 2, kFoldLanes);
+    for (int k = 0; k <= R; ++k) {
+      e[k][h] = sum(e[k][h]);
+      d[k][h] = sum(d[k][h]);
+    }
+#pragma unroll
+    for (int k = 0; k < R + 2; ++k) w[k][h] = sum(w[k][h]);
+  }
+  float4* o = reinterpret_cast<float4*>(f.out + (size_t)set * f.out_stride);
+  float4* od = o + (size_t)numr * np * 2;
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    const int i = i0 + k;
+    if (i >= numr) break;
+    const size_t at = (size_t)i * np + p;
+    const bool last = i == numr - 1;
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (q == 0) {
+      // node i and the step to node i+1, so that the evaluation interpolates
+      // with one FMA: E_i + x2 (E_i+1 - E_i)
+      if (!last)
+        v = make_float4((float)e[k][0], (float)e[k][1], (float)(e[k + 1][0] - e[k][0]),
+                        (float)(e[k + 1][1] - e[k][1]));
+      o[2 * at] = v;
+    } else if (q == 1) {
+      // rows c - 1, c, c + 1 about c = max(i, 1)
+      const bool first = k == 0 && i0 == 0;
+      double b[2], z[2], t[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        b[h] = first ? w[1][h] : w[k][h];
+        z[h] = first ? w[2][h] : w[k + 1][h];
+        t[h] = first ? w[0][h] : w[k + 2][h];
+      }
+      if (!last)
+        v = make_float4((float)(0.5 * (t[0] - b[0])), (float)(0.5 * (t[1] - b[1])),
+                        (float)(b[0] - 2.0 * z[0] + t[0]), (float)(b[1] - 2.0 * z[1] + t[1]));
+      o[2 * at + 1] = v;
+    } else if (q == 2) {
+      if (!last)
+        v = make_float4((float)d[k][0], (float)d[k][1], (float)d[k + 1][0], (float)d[k + 1][1]);
+      od[at] = v;
     }
   }
-  if (q == 0) {
-    // node i and the step to node i+1, so that the evaluation interpolates
-    // with one FMA: E_i + x2 (E_i+1 - E_i)
-    o[0] = (float)v[0][0];
-    o[1] = (float)v[1][0];
-    o[2] = (float)(v[0][1] - v[0][0]);
-    o[3] = (float)(v[1][1] - v[1][0]);
-  } else if (q == 1) {
-    o[4] = (float)(0.5 * (v[0][6] - v[0][4]));
-    o[5] = (float)(0.5 * (v[1][6] - v[1][4]));
-    o[6] = (float)(v[0][4] - 2.0 * v[0][5] + v[0][6]);
-    o[7] = (float)(v[1][4] - 2.0 * v[1][5] + v[1][6]);
-  } else if (q == 2) {
-    od[0] = (float)v[0][2];
-    od[1] = (float)v[1][2];
-    od[2] = (float)v[0][3];
-    od[3] = (float)v[1][3];
-  }
+}
+
+__global__ __launch_bounds__(256) void sl_fold_kernel(SLFoldIn f, SLFoldArgs a) {
+  sl_fold_block(f, a, blockIdx.x, blockIdx.y);
 }
 
 struct EOFFoldArgs {
@@ -120,6 +162,7 @@ __device__ __forceinline__ void eof_fold_edge(const double* __restrict__ E, int6
                                               int norder, const EOFFoldArgs& a,
                                               float* __restrict__ out_set) {
   double s[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 6
   for (int n = 0; n < a.nuse; ++n) {
     const double c = cf[n];
 #pragma unroll
@@ -131,67 +174,129 @@ __device__ __forceinline__ void eof_fold_edge(const double* __restrict__ E, int6
   *o = make_double4(s[0] * mul, s[1] * mul, s[2] * mul, s[3] * mul);
 }
 
-// One thread per (row group q, node): q = m for cos m = 0..mmax, mmax + m
-// for sin m = 1..mmax; nodes fastest so the function-major float32 tables
-// are read coalesced (sums in float64), and q uniform per block so the coefficients are
-// scalar loads.  Writes its half [pot, rf, zf, dens] of the 8-float block
-// [potC, rfC, zfC, dC, potS, rfS, zfS, dS]; cos m = 0 also zeroes the sin
-// half.  grid.x = ceil(nedge / 256) blocks for the float64 edge blocks
-// (eof_fold_edge) of the m = 0 cos rows, first so that they do not trail,
-// then (2 mmax + 1) * chunks blocks of these; grid.y = coefficient sets.
-__global__ __launch_bounds__(256) void eof_fold_kernel(
+// A block of eight waves folds kFoldNodes nodes: lane = node, so the
+// function-major float32 tables are read coalesced (sums in float64), and a wave
+// takes one row group q at a time (q = m for cos m = 0..mmax, mmax + m for sin
+// m = 1..mmax), so the coefficients are scalar loads.  Each row group is one half
+// [pot, rf, zf, dens] of the 8-float block [potC, rfC, zfC, dC, potS, rfS, zfS, dS]
+// of its m (the sin half of m = 0 is zero); four m at a time, the halves are put
+// together in LDS and leave as 128 bytes of a node, where 16-byte stores cost an
+// L2 request each.  grid.x = ceil(nedge / 512) blocks a set for the float64 edge
+// blocks (eof_fold_edge) of the m = 0 cos rows, first so that they do not trail,
+// then the node blocks, each XCD (block index modulo eight) a contiguous range of
+// them; grid.y = groups of SETS coefficient sets, which share the reads of the
+// tables.  What bounds it is memory: 93 MB of tables at mmax 6, norder 18, 257 x
+// 129 nodes (one set 21.5 -> 19 us), and 7.4 MB of results a set (12 sets: one set
+// a thread 230 us; four sets 92, their stores made whole 72; six sets 69).
+constexpr int kFoldNodes = 64;
+constexpr int kFoldThreads = 512;
+constexpr int kFoldM = 4;            // m per group: one row group a wave
+constexpr int kEofFoldSets = 6;
+struct EOFFoldIn {
+  const float* T[4];
+  const double *ccos, *csin;
+  int mmax, norder, nset, per_xcd;
+  int64_t nodes, nedge;
+  const double* E;
+  float* out;
+  int64_t coef_stride, out_stride;
+};
+template <int SETS, bool DENS>
+__device__ __forceinline__ void eof_fold_block(
     const float* __restrict__ T0, const float* __restrict__ T1, const float* __restrict__ T2,
     const float* __restrict__ T3, const double* __restrict__ ccos, const double* __restrict__ csin,
-    int mmax, int norder, int64_t nodes, int chunks, EOFFoldArgs a, float* __restrict__ out,
-    int64_t coef_stride, int64_t out_stride, const double* __restrict__ E, int64_t nedge) {
-  const unsigned eblocks = (unsigned)((nedge + 255) / 256);
-  if (blockIdx.x < eblocks) {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e < nedge)
-      eof_fold_edge(E, nedge, e, ccos + (size_t)blockIdx.y * coef_stride, mmax, norder, a,
-                    out + (size_t)blockIdx.y * out_stride);
+    const double* __restrict__ E, float* __restrict__ out, const EOFFoldIn& f, const EOFFoldArgs& a,
+    unsigned block, int set0) {
+  __shared__ float4 s_fold[SETS][kFoldNodes][2 * kFoldM];
+  const int mmax = f.mmax, norder = f.norder, nset = f.nset, per_xcd = f.per_xcd;
+  const int64_t nodes = f.nodes, nedge = f.nedge, coef_stride = f.coef_stride, out_stride = f.out_stride;
+  const unsigned eblocks = (unsigned)((nedge + kFoldThreads - 1) / kFoldThreads) * SETS;
+  if (block < eblocks) {
+    const int k = set0 + (int)(block % SETS);
+    const int64_t e = (int64_t)(block / SETS) * kFoldThreads + threadIdx.x;
+    if (k < nset && e < nedge)
+      eof_fold_edge(E, nedge, e, ccos + (size_t)k * coef_stride, mmax, norder, a,
+                    out + (size_t)k * out_stride);
     return;
   }
-  const unsigned b = blockIdx.x - eblocks;
-  const int q = (int)(b / chunks);
-  const int64_t node = (int64_t)(b - (unsigned)q * chunks) * 256 + threadIdx.x;
-  if (node >= nodes) return;
-  const bool sn = q > mmax;
-  const int m = sn ? q - mmax : q;
-  const double* cf = (sn ? csin : ccos) + (size_t)blockIdx.y * coef_stride + (size_t)m * norder;
-  const double mul = a.mmul[m];
-  const size_t row = (size_t)q * norder * nodes + node;
-  const float* t0 = T0 + row;
-  const float* t1 = T1 + row;
-  const float* t2 = T2 + row;
-  const float* t3 = T3 + row;
-  double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-  if (a.dens) {
+  const unsigned b = block - eblocks;
+  const int64_t node0 = ((int64_t)(b & 7) * per_xcd + (b >> 3)) * kFoldNodes;
+  if (node0 >= nodes) return;
+  const int lane = threadIdx.x & 63;
+  const int64_t node = node0 + lane < nodes ? node0 + lane : nodes - 1;
+  const unsigned nn = nodes - node0 < kFoldNodes ? (unsigned)(nodes - node0) : kFoldNodes;
+  for (int m0 = 0; m0 <= mmax; m0 += kFoldM) {
+    const int wave = uni(threadIdx.x >> 6), m = m0 + (wave & (kFoldM - 1));
+    const bool sn = wave >= kFoldM;
+    if (m <= mmax && !(sn && m == 0)) {
+      const int q = sn ? mmax + m : m;
+      const double* cf[SETS];
+#pragma unroll
+      for (int k = 0; k < SETS; ++k)   // a group past the last set repeats it and writes nothing
+        cf[k] = (sn ? csin : ccos) + (size_t)(set0 + k < nset ? set0 + k : nset - 1) * coef_stride +
+                (size_t)m * norder;
+      const double mul = a.mmul[m];
+      const size_t row = (size_t)q * norder * nodes + node;
+      const float* t0 = T0 + row;
+      const float* t1 = T1 + row;
+      const float* t2 = T2 + row;
+      const float* t3 = T3 + row;
+      double v[SETS][DENS ? 4 : 3];
+#pragma unroll
+      for (int k = 0; k < SETS; ++k)
+#pragma unroll
+        for (int f = 0; f < (DENS ? 4 : 3); ++f) v[k][f] = 0.0;
 #pragma unroll 6
-    for (int n = 0; n < a.nuse; ++n) {
-      const double c = cf[n];
-      const size_t o = (size_t)n * nodes;
-      s0 += c * t0[o];
-      s1 += c * t1[o];
-      s2 += c * t2[o];
-      s3 += c * t3[o];
+      for (int n = 0; n < a.nuse; ++n) {
+        const size_t o = (size_t)n * nodes;
+        const float t[4] = {t0[o], t1[o], t2[o], DENS ? t3[o] : 0.f};
+#pragma unroll
+        for (int k = 0; k < SETS; ++k) {
+          const double c = cf[k][n];
+#pragma unroll
+          for (int f = 0; f < (DENS ? 4 : 3); ++f) v[k][f] += c * t[f];
+        }
+      }
+      // slot j of a node at j ^ (node & 7): eight lanes' stores on eight bank groups
+      const int j = 2 * (m - m0) + (sn ? 1 : 0), sw = lane & 7;
+#pragma unroll
+      for (int k = 0; k < SETS; ++k) {
+        s_fold[k][lane][j ^ sw] =
+            make_float4((float)(v[k][0] * mul), (float)(v[k][1] * mul), (float)(v[k][2] * mul),
+                        DENS ? (float)(v[k][DENS ? 3 : 0] * mul) : 0.f);
+        if (m == 0) s_fold[k][lane][1 ^ sw] = make_float4(0.f, 0.f, 0.f, 0.f);
+      }
     }
-  } else {
-#pragma unroll 6
-    for (int n = 0; n < a.nuse; ++n) {
-      const double c = cf[n];
-      const size_t o = (size_t)n * nodes;
-      s0 += c * t0[o];
-      s1 += c * t1[o];
-      s2 += c * t2[o];
+    __syncthreads();
+    const unsigned len = 2u * (unsigned)(mmax + 1 - m0 < kFoldM ? mmax + 1 - m0 : kFoldM);
+#pragma unroll
+    for (int k = 0; k < SETS; ++k) {
+      if (set0 + k >= nset) break;
+      float4* o = reinterpret_cast<float4*>(out + (size_t)(set0 + k) * out_stride) +
+                  (size_t)node0 * (2 * (mmax + 1)) + 2 * m0;
+      for (unsigned f = threadIdx.x; f < nn * len; f += kFoldThreads) {
+        const unsigned d = f / len, j = f - d * len;
+        o[d * (2u * (unsigned)(mmax + 1)) + j] = s_fold[k][d][j ^ (d & 7)];
+      }
     }
+    __syncthreads();
   }
-  float* o = out + (size_t)blockIdx.y * out_stride + ((size_t)node * (mmax + 1) + m) * 8 + (sn ? 4 : 0);
-  o[0] = (float)(s0 * mul);
-  o[1] = (float)(s1 * mul);
-  o[2] = (float)(s2 * mul);
-  o[3] = (float)(s3 * mul);
-  if (q == 0) o[4] = o[5] = o[6] = o[7] = 0.f;
+}
+
+template <int SETS, bool DENS>
+__global__ __launch_bounds__(kFoldThreads) void eof_fold_kernel(EOFFoldIn f, EOFFoldArgs a) {
+  eof_fold_block<SETS, DENS>(f.T[0], f.T[1], f.T[2], f.T[3], f.ccos, f.csin, f.E, f.out, f, a, blockIdx.x, blockIdx.y * SETS);
+}
+
+// Both folds of one frozen field in one launch: the SL fold waits on its own
+// gathers and runs in the shadow of the EOF fold's table reads (23 us; as two
+// launches on two streams 21 and 12 us and 15 us of events between them).
+__global__ __launch_bounds__(kFoldThreads) void field_fold_kernel(SLFoldIn sf, SLFoldArgs sa,
+                                                                     unsigned slblocks, EOFFoldIn ef,
+                                                                     EOFFoldArgs ea) {
+  if (blockIdx.x < slblocks) sl_fold_block(sf, sa, blockIdx.x, 0);
+  else eof_fold_block<1, false>(ef.T[0], ef.T[1], ef.T[2], ef.T[3], ef.ccos, ef.csin, ef.E, ef.out, ef, ea,
+                                blockIdx.x - slblocks, 0);
 }
 
 static int ensure_folded(Context* c, float** d, size_t* have, size_t floats, hipStream_t s) {
@@ -215,23 +320,42 @@ static size_t eof_fold_floats(const Context* c) {
          (size_t)eof_edge_count(c->numx, c->numy) * 8;
 }
 
-// Folds nset coefficient sets (stride (lmax+1)^2 nmax) into out (stride sl_fold_floats).
-static int sl_fold_into(Context* c, const double* coef, int nset, double halofac, int lmax_use,
-                        int nmax_use, int L1, int L2, bool no_odd, float* out, hipStream_t s) {
-  const int np = sl_npairs(c->lmax);
-  SLFoldArgs a;
+// The arguments of the SL fold of nset coefficient sets (stride (lmax+1)^2 nmax)
+// into out (stride sl_fold_floats); returns its lanes.
+static int64_t sl_fold_args(Context* c, const double* coef, int nset, double halofac, int lmax_use,
+                            int nmax_use, int L1, int L2, bool no_odd, float* out, SLFoldIn* f,
+                            SLFoldArgs* args) {
+  SLFoldArgs& a = *args;
+  double lmul[kMaxL + 1];
   for (int l = 0; l <= kMaxL; ++l) {
     bool keep = l <= lmax_use;
     if (l >= 1 && (l > L2 || l < L1)) keep = false;
     if (l >= 1 && no_odd && (l & 1)) keep = false;
-    a.lmul[l] = keep ? halofac : 0.0;
+    lmul[l] = keep ? halofac : 0.0;
   }
   a.lmax = c->lmax;
   a.nmax_use = nmax_use;
-  const int64_t total = (int64_t)c->numr * np * kFoldLanes;
-  hipLaunchKernelGGL(sl_fold_kernel, dim3((unsigned)((total + 255) / 256), nset), dim3(256), 0, s,
-                     c->sl_fold64, coef, c->nmax, c->numr, a, out,
-                     (int64_t)(c->lmax + 1) * (c->lmax + 1) * c->nmax, (int64_t)sl_fold_floats(c));
+  // N_lm (spheresl.py:858-861) folded into the table
+  for (int m = 0, p = 0; m <= c->lmax; ++m)
+    for (int l = m; l <= c->lmax; ++l, ++p) {
+      double ratio = 1.0;
+      for (int k = 1; k <= m; ++k) ratio /= (double)(l - k + 1) * (double)(l + k);
+      double N = sqrt((0.5 * l + 0.25) / kPi * ratio);
+      if (m > 0) N *= 1.4142135623730951;
+      a.mul[p] = lmul[l] * N;
+    }
+  *f = SLFoldIn{c->sl_fold64, coef, c->nmax, c->numr, nset, out,
+                (int64_t)(c->lmax + 1) * (c->lmax + 1) * c->nmax, (int64_t)sl_fold_floats(c)};
+  return (int64_t)((c->numr + kFoldRows - 1) / kFoldRows) * sl_npairs(c->lmax) * kFoldLanes;
+}
+
+static int sl_fold_into(Context* c, const double* coef, int nset, double halofac, int lmax_use,
+                        int nmax_use, int L1, int L2, bool no_odd, float* out, hipStream_t s) {
+  SLFoldIn f;
+  SLFoldArgs a;
+  const int64_t lanes = sl_fold_args(c, coef, nset, halofac, lmax_use, nmax_use, L1, L2, no_odd, out, &f, &a);
+  hipLaunchKernelGGL(sl_fold_kernel, dim3((unsigned)((lanes + 255) / 256), (unsigned)nset), dim3(256), 0, s,
+                     f, a);
   BFE_HIP(c, hipGetLastError());
   return 0;
 }
@@ -247,11 +371,12 @@ static int sl_fold(Context* c, int slot, const double* coef, double halofac, int
   return 0;
 }
 
-static int eof_fold_into(Context* c, const double* ccos, const double* csin, int nset,
-                         int mmax_use, int nuse, int m1, int m2, bool no_odd, bool compat_mask,
-                         bool dens, float* out, hipStream_t s) {
+// The arguments of the EOF fold, likewise; returns the blocks of `sets` sets.
+static unsigned eof_fold_args(Context* c, const double* ccos, const double* csin, int nset, int sets,
+                              int mmax_use, int nuse, int m1, int m2, bool no_odd, bool compat_mask,
+                              bool dens, float* out, EOFFoldIn* f, EOFFoldArgs* args) {
   const int64_t nodes = (int64_t)(c->numx + 1) * (c->numy + 1);
-  EOFFoldArgs a;
+  EOFFoldArgs& a = *args;
   for (int m = 0; m <= kMaxM; ++m) {
     double mul = 1.0;
     if (m > mmax_use || m > m2 || m < m1) mul = 0.0;
@@ -265,14 +390,29 @@ static int eof_fold_into(Context* c, const double* ccos, const double* csin, int
   a.dens = dens ? 1 : 0;
   a.numx = c->numx;
   a.numy = c->numy;
-  const int chunks = (int)((nodes + 255) / 256);
   const int64_t nedge = eof_edge_count(c->numx, c->numy);
-  const unsigned grid = (unsigned)((2 * c->mmax + 1) * chunks + (nedge + 255) / 256);
-  hipLaunchKernelGGL(eof_fold_kernel, dim3(grid, nset), dim3(256), 0, s, c->eof_fold32[0],
-                     c->eof_fold32[1], c->eof_fold32[2],
-                     dens ? c->eof_fold32[3] : c->eof_fold32[0], ccos, csin, c->mmax, c->norder,
-                     nodes, chunks, a, out, (int64_t)(c->mmax + 1) * c->norder,
-                     (int64_t)eof_fold_floats(c), c->eof_edge64, nedge);
+  const int64_t chunks = (nodes + kFoldNodes - 1) / kFoldNodes;
+  const int per_xcd = (int)((chunks + 7) / 8);
+  *f = EOFFoldIn{{c->eof_fold32[0], c->eof_fold32[1], c->eof_fold32[2],
+                  dens ? c->eof_fold32[3] : c->eof_fold32[0]},
+                 ccos, csin, c->mmax, c->norder, nset, per_xcd, nodes, nedge, c->eof_edge64, out,
+                 (int64_t)(c->mmax + 1) * c->norder, (int64_t)eof_fold_floats(c)};
+  return 8u * (unsigned)per_xcd + (unsigned)((nedge + kFoldThreads - 1) / kFoldThreads) * sets;
+}
+
+static int eof_fold_into(Context* c, const double* ccos, const double* csin, int nset, int mmax_use,
+                         int nuse, int m1, int m2, bool no_odd, bool compat_mask, bool dens, float* out,
+                         hipStream_t s) {
+  EOFFoldIn f;
+  EOFFoldArgs a;
+  auto go = [&](auto kernel, int sets) {
+    const unsigned grid = eof_fold_args(c, ccos, csin, nset, sets, mmax_use, nuse, m1, m2, no_odd,
+                                        compat_mask, dens, out, &f, &a);
+    hipLaunchKernelGGL(kernel, dim3(grid, (unsigned)((nset + sets - 1) / sets)), dim3(kFoldThreads), 0, s, f, a);
+  };
+  if (nset > 1 && !dens) go(eof_fold_kernel<kEofFoldSets, false>, kEofFoldSets);
+  else if (dens) go(eof_fold_kernel<1, true>, 1);
+  else go(eof_fold_kernel<1, false>, 1);
   BFE_HIP(c, hipGetLastError());
   return 0;
 }
@@ -702,15 +842,21 @@ static int field_set_run(Context* c, const double* eof_cos, const double* eof_si
   const int ll = halo_l < 0 ? c->lmax : std::min(halo_l, c->lmax);
   const int hn = halo_n < 0 ? c->nmax : std::min(halo_n, c->nmax);
   const bool no_odd = (flags & BFE_NO_ODD) != 0;
-  // the SL fold (a few thousand waves) runs beside the HBM-bound EOF fold
-  hipStream_t s2 = nullptr;
-  int rc = fork_begin(c, s, &s2);
+  int rc = ensure_folded(c, &c->slf[1].d, &c->slf[1].floats, sl_fold_floats(c), s);
+  if (!rc) rc = ensure_folded(c, &c->eoff[1].d, &c->eoff[1].floats, eof_fold_floats(c), s);
   if (rc) return rc;
-  const int rs = sl_fold(c, 1, sl_coef, halofac, ll, hn, -(1 << 30), 1 << 30, no_odd, s2);
-  const int re = rs ? 0 : eof_fold(c, 1, eof_cos, eof_sin, mm, nn, 0, 1 << 30, no_odd,
-                                   (flags & BFE_COMPAT_EOF_MASK) != 0, false, s);
-  rc = fork_end(c, s);
-  if (rs || re || rc) return rs ? rs : (re ? re : rc);
+  SLFoldIn sf;
+  SLFoldArgs sa;
+  EOFFoldIn ef;
+  EOFFoldArgs ea;
+  const int64_t lanes = sl_fold_args(c, sl_coef, 1, halofac, ll, hn, -(1 << 30), 1 << 30, no_odd,
+                                     c->slf[1].d, &sf, &sa);
+  const unsigned eb = eof_fold_args(c, eof_cos, eof_sin, 1, 1, mm, nn, 0, 1 << 30, no_odd,
+                                    (flags & BFE_COMPAT_EOF_MASK) != 0, false, c->eoff[1].d, &ef, &ea);
+  const unsigned sb = (unsigned)((lanes + kFoldThreads - 1) / kFoldThreads);
+  hipLaunchKernelGGL(field_fold_kernel, dim3(sb + eb), dim3(kFoldThreads), 0, s, sf, sa, sb, ef, ea);
+  BFE_HIP(c, hipGetLastError());
+  c->slf[1].valid = c->eoff[1].valid = true;
   c->field_halofac = halofac;
   c->field_flags = (int)(flags & (BFE_COMPAT_SL_COS_L | BFE_COMPAT_SL_EDGE));
   return 0;

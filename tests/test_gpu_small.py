@@ -4,7 +4,7 @@ of one to five tiles, and sorts of 512- and 2048-item tiles."""
 import numpy as np
 import pytest
 
-from tests.test_gpu_parity import big, block_rel_eof, block_rel_sl, disc_halo, f32  # noqa: F401
+from tests.test_gpu_parity import big, block_rel_eof, block_rel_sl, disc_halo, f32, relmax  # noqa: F401
 from oracle import bfe_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -88,3 +88,40 @@ def test_batch_pieces_edges(nsnap, omin):
             s.set_field(c[q], sn[q], hl[q])
             for u, v in zip(f, s.field_forces(*(v[a:b] for v in h[:3]), rotpos=0.3)):
                 assert torch.equal(u[a:b], v)
+
+
+@pytest.mark.parametrize("nset", [1, 2, 5, 6, 7, 13])
+@pytest.mark.parametrize("lmax,mmax,numr,numx,numy", [(0, 0, 4, 8, 6), (3, 3, 5, 9, 6), (6, 4, 201, 20, 15),
+                                                      (9, 8, 64, 31, 17)])
+def test_folds_of_a_batch_equal_single_folds(nset, lmax, mmax, numr, numx, numy):
+    """Batch folds (several sets a block) and the two folds of one field in one
+    launch, at sizes that leave remainders of the node and row groups: every
+    point's bits as with the separate single folds of the point evaluators'
+    kernels (per-set fields), and the field of the oracle."""
+    import torch
+    from exptool_amd.bfe import BFESystem
+    from exptool_amd.utils import workloads as W
+    st, et = W.disc_halo_tables(seed=2, n_eof_sample=3000, lmax_s=10, nmax_s=8,
+                                eof=dict(mmax=mmax, norder=5, numx=numx, numy=numy),
+                                sl=dict(lmax=lmax, nmax=7, numr=numr))
+    s = BFESystem(sl=st, eof=et)
+    d, h = W.disc_halo_particles(64 * nset, 64 * nset, seed=3)
+    d, h = ([torch.tensor(np.asarray(a, np.float32), device="cuda") for a in p] for p in (d, h))
+    counts = [64] * nset
+    c, sn = s.eof_accumulate_batch(*d, counts)
+    hl = s.sl_accumulate_batch(*h, counts)
+    s.set_field_batch(c, sn, hl)
+    f = s.field_forces_batch(*d[:3], counts)
+    for q in range(nset):
+        s.set_field(c[q], sn[q], hl[q])
+        for u, v in zip(f, s.field_forces(*(v[64 * q:64 * q + 64] for v in d[:3]))):
+            assert torch.equal(u[64 * q:64 * q + 64], v)
+    slo = O.SLTable(st["lmax"], st["nmax"], st["numr"], st["cmap"], st["rmin"], st["rmax"], st["scale"],
+                    st["ev"], st["ef"], st["xi"], st["p0"], st["d0"])
+    eo = O.EOFTable(et["mmax"], et["norder"], et["numx"], et["numy"], et["cmap"], et["rmin"], et["rmax"],
+                    et["ascale"], et["hscale"], et["potC"], et["rforceC"], et["zforceC"], et["potS"],
+                    et["rforceS"], et["zforceS"], et["densC"], et["densS"])
+    F = O.FieldSpec(eo, c[-1].cpu().numpy(), sn[-1].cpu().numpy(), slo, hl[-1].cpu().numpy())
+    x, y, z = (v[-64:].cpu().numpy().astype(np.float64) for v in d[:3])
+    for u, r in zip(f, O.total_force(F, x, y, z)):
+        assert relmax(u[-64:].cpu().numpy(), r) <= 1e-5    # the field's bound, per output
