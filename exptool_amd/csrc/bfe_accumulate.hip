@@ -54,14 +54,23 @@ __device__ __forceinline__ void segment_range(const Segments& S, int64_t sg, int
   }
 }
 
+// LDS of the input-order EOF kernel for a tile
+template <int TILE>
+struct EofTileLds {
+  int base[TILE];
+  float c[4][TILE];
+  float w[2 * kMaxM + 1][TILE + 1];  // +1: spread rows over banks
+};
+
+// Segments `block`, block + nblocks, ... of S.
 template <int OPT, int TILE>
-__global__ __launch_bounds__(256) void eof_accumulate_kernel(
-    const float* __restrict__ px, const float* __restrict__ py, const float* __restrict__ pz,
-    const float* __restrict__ pm, Segments S, EOFGeom g, const float* __restrict__ T, int K,
-    double* __restrict__ partials) {
-  __shared__ int s_base[TILE];
-  __shared__ float s_c[4][TILE];
-  __shared__ float s_w[2 * kMaxM + 1][TILE + 1];  // +1: spread rows over banks
+__device__ __forceinline__ void eof_accumulate_block(
+    EofTileLds<TILE>& L, const float* __restrict__ px, const float* __restrict__ py,
+    const float* __restrict__ pz, const float* __restrict__ pm, const Segments& S, const EOFGeom& g,
+    const float* __restrict__ T, int K, double* __restrict__ partials, int block, int nblocks) {
+  int(&s_base)[TILE] = L.base;
+  float(&s_c)[4][TILE] = L.c;
+  float(&s_w)[2 * kMaxM + 1][TILE + 1] = L.w;
 
   const int tid = threadIdx.x;
   const int ny1 = g.numy + 1;
@@ -75,7 +84,7 @@ __global__ __launch_bounds__(256) void eof_accumulate_kernel(
     const int k = tid + o * 256;
     rowg[o] = (k < K) ? k / g.norder : 0;
   }
-  for (int64_t sg = blockIdx.x; sg < S.nseg; sg += gridDim.x) {
+  for (int64_t sg = block; sg < S.nseg; sg += nblocks) {
   int64_t s0, s1;
   segment_range(S, sg, s0, s1);
 #pragma unroll
@@ -156,6 +165,15 @@ __global__ __launch_bounds__(256) void eof_accumulate_kernel(
   }
 }
 
+template <int OPT, int TILE>
+__global__ __launch_bounds__(256) void eof_accumulate_kernel(
+    const float* __restrict__ px, const float* __restrict__ py, const float* __restrict__ pz,
+    const float* __restrict__ pm, Segments S, EOFGeom g, const float* __restrict__ T, int K,
+    double* __restrict__ partials) {
+  __shared__ EofTileLds<TILE> L;
+  eof_accumulate_block<OPT, TILE>(L, px, py, pz, pm, S, g, T, K, partials, blockIdx.x, gridDim.x);
+}
+
 // Fixed-order float64 reduction of the per-segment partials, column k
 // (a column's rows are K doubles apart): row lane j Kahan-sums rows j,
 // j + kRedLanes, ... of its column, then a fixed tree adds the lanes.  The
@@ -167,20 +185,19 @@ __global__ __launch_bounds__(256) void eof_accumulate_kernel(
 constexpr int kRedCols = 8;    // a row read is 64 contiguous bytes
 constexpr int kRedLanes = 32;
 template <bool SPLIT>
-__global__ __launch_bounds__(256) void reduce_partials_kernel(const double* __restrict__ partials,
-                                                              int nb, int K,
-                                                              double* __restrict__ out,
-                                                              const int64_t* __restrict__ rowb,
-                                                              double* __restrict__ sin_out,
-                                                              int nc, int norder) {
-  __shared__ double sh[kRedLanes][kRedCols];
+__device__ __forceinline__ void reduce_partials_block(double (&sh)[kRedLanes][kRedCols],
+                                                      const double* __restrict__ partials, int nb, int K,
+                                                      double* __restrict__ out,
+                                                      const int64_t* __restrict__ rowb,
+                                                      double* __restrict__ sin_out, int nc, int norder,
+                                                      unsigned block, unsigned set) {
   const int c = threadIdx.x % kRedCols;
   const int j = threadIdx.x / kRedCols;
-  const int k = blockIdx.x * kRedCols + c;
+  const int k = block * kRedCols + c;
   int64_t r0 = 0, r1 = nb;
   if (rowb) {
-    r0 = rowb[blockIdx.y];
-    r1 = rowb[blockIdx.y + 1];
+    r0 = rowb[set];
+    r1 = rowb[set + 1];
   }
   double s = 0.0, comp = 0.0;
   if (k < K) {
@@ -201,9 +218,9 @@ __global__ __launch_bounds__(256) void reduce_partials_kernel(const double* __re
   if (j == 0 && k < K) {
     const double v = sh[0][c];
     if (!SPLIT) {
-      out[(size_t)blockIdx.y * K + k] = v;
+      out[(size_t)set * K + k] = v;
     } else {
-      const size_t q = (size_t)blockIdx.y * nc;
+      const size_t q = (size_t)set * nc;
       if (k < nc) {
         out[q + k] = v;
         if (k < norder) sin_out[q + k] = 0.0;
@@ -212,6 +229,31 @@ __global__ __launch_bounds__(256) void reduce_partials_kernel(const double* __re
       }
     }
   }
+}
+
+template <bool SPLIT>
+__global__ __launch_bounds__(256) void reduce_partials_kernel(const double* __restrict__ partials,
+                                                              int nb, int K,
+                                                              double* __restrict__ out,
+                                                              const int64_t* __restrict__ rowb,
+                                                              double* __restrict__ sin_out,
+                                                              int nc, int norder) {
+  __shared__ double sh[kRedLanes][kRedCols];
+  reduce_partials_block<SPLIT>(sh, partials, nb, K, out, rowb, sin_out, nc, norder, blockIdx.x, blockIdx.y);
+}
+
+// The reductions of an EOF and an SL accumulate in one launch.
+__global__ __launch_bounds__(256) void reduce_both_kernel(const double* __restrict__ pe, int nbe, int Ke,
+                                                          double* __restrict__ cos_out,
+                                                          double* __restrict__ sin_out, int nc, int norder,
+                                                          const double* __restrict__ ps, int nbs, int Ks,
+                                                          double* __restrict__ coef_out) {
+  __shared__ double sh[kRedLanes][kRedCols];
+  const unsigned eb = (Ke + kRedCols - 1) / kRedCols;
+  if (blockIdx.x < eb)
+    reduce_partials_block<true>(sh, pe, nbe, Ke, cos_out, nullptr, sin_out, nc, norder, blockIdx.x, 0);
+  else
+    reduce_partials_block<false>(sh, ps, nbs, Ks, coef_out, nullptr, nullptr, 0, 0, blockIdx.x - eb, 0);
 }
 
 __global__ void fill_f64_kernel(double* __restrict__ a, int64_t n) {
@@ -223,11 +265,11 @@ __global__ void fill_f64_kernel(double* __restrict__ a, int64_t n) {
 // SL accumulate
 // ---------------------------------------------------------------------------
 template <int OPT>
-__global__ __launch_bounds__(256) void sl_accumulate_kernel(
-    const float* __restrict__ px, const float* __restrict__ py, const float* __restrict__ pz,
-    const float* __restrict__ pm, Segments S, SLGeom g, const float* __restrict__ E,
-    const double* __restrict__ lmc, int no_odd, double* __restrict__ partials) {
-  extern __shared__ float smem[];
+__device__ __forceinline__ void sl_accumulate_block(
+    float* smem, const float* __restrict__ px, const float* __restrict__ py,
+    const float* __restrict__ pz, const float* __restrict__ pm, const Segments& S, const SLGeom& g,
+    const float* __restrict__ E, const double* __restrict__ lmc, int no_odd,
+    double* __restrict__ partials, int block, int nblocks) {
   const int R = (g.lmax + 1) * (g.lmax + 1);
   const int LN = (g.lmax + 1) * g.nmax;
   const int K = R * g.nmax;
@@ -255,7 +297,7 @@ __global__ __launch_bounds__(256) void sl_accumulate_kernel(
     yrow[o] = row * YS;
     prow[o] = l * g.nmax + nn;
   }
-  for (int64_t sg = blockIdx.x; sg < S.nseg; sg += gridDim.x) {
+  for (int64_t sg = block; sg < S.nseg; sg += nblocks) {
   int64_t s0, s1;
   segment_range(S, sg, s0, s1);
 #pragma unroll
@@ -354,6 +396,39 @@ __global__ __launch_bounds__(256) void sl_accumulate_kernel(
     if (k < K) partials[(size_t)sg * K + k] = accd[o];
   }
   }
+}
+
+template <int OPT>
+__global__ __launch_bounds__(256) void sl_accumulate_kernel(
+    const float* __restrict__ px, const float* __restrict__ py, const float* __restrict__ pz,
+    const float* __restrict__ pm, Segments S, SLGeom g, const float* __restrict__ E,
+    const double* __restrict__ lmc, int no_odd, double* __restrict__ partials) {
+  extern __shared__ float smem[];
+  sl_accumulate_block<OPT>(smem, px, py, pz, pm, S, g, E, lmc, no_odd, partials, blockIdx.x, gridDim.x);
+}
+
+// The input-order accumulates of a disc and a halo in one launch, the disc's
+// segments first.  Each is bound by the latency of its own tile, so they fit
+// beside each other; on two streams the events that part and join them cost
+// more than they give (30 000-point dump: 44 us of launches and events, of
+// 87 us a call).
+struct AccIn {
+  const float *x, *y, *z, *m;
+  Segments S;
+  double* partials;
+};
+template <int OPTE, int OPTS>
+__global__ __launch_bounds__(256) void accumulate_both_kernel(AccIn d, EOFGeom eg, const float* __restrict__ T,
+                                                              int Ke, int eblocks, AccIn h, SLGeom sg,
+                                                              const float* __restrict__ E,
+                                                              const double* __restrict__ lmc, int no_odd) {
+  extern __shared__ float smem[];
+  if ((int)blockIdx.x < eblocks)
+    eof_accumulate_block<OPTE, kSmallTile>(*reinterpret_cast<EofTileLds<kSmallTile>*>(smem), d.x, d.y, d.z,
+                                           d.m, d.S, eg, T, Ke, d.partials, blockIdx.x, eblocks);
+  else
+    sl_accumulate_block<OPTS>(smem, h.x, h.y, h.z, h.m, h.S, sg, E, lmc, no_odd, h.partials,
+                              (int)blockIdx.x - eblocks, (int)gridDim.x - eblocks);
 }
 
 // ---------------------------------------------------------------------------
@@ -1896,6 +1971,55 @@ static int sl_accumulate_run(Context* c, const float* x, const float* y, const f
   return 0;
 }
 
+// Disc and halo coefficients of few particles on one stream: one launch of
+// both input-order accumulates and one of both reductions.  Sets *done = false
+// and does nothing where either would not take that path (from order_min
+// particles on cell order pays; MFMA mode; empty inputs; kernel timing on,
+// which times each by itself).
+int accumulate_both_small(Context* c, const float* dx, const float* dy, const float* dz,
+                          const float* dm, int64_t nd, const float* hx, const float* hy,
+                          const float* hz, const float* hm, int64_t nh, uint32_t flags,
+                          double* cos_out, double* sin_out, double* coef_out, hipStream_t s, bool* done) {
+  *done = false;
+  const int Ke = c->eof_K, R = (c->lmax + 1) * (c->lmax + 1), LN = (c->lmax + 1) * c->nmax, Ks = R * c->nmax;
+  const size_t lds = ((size_t)R * (kSLTile + 1) + (size_t)kSLTile * LN + 3 * kSLTile) * 4;
+  if (nd < 1 || nh < 1 || nd >= c->order_min || nh >= c->order_min || (flags & BFE_ACC_BF16) ||
+      c->sl_acc_path == 1 || c->kernel_timing || Ke > 1024 || Ks > 1024 || lds > 64 * 1024)
+    return 0;
+  const AccPlan Pd = plan_input_order(c->eof_acc_blocks, nd);
+  if (Pd.S.seglen > kSmallTile) return 0;
+  const AccPlan Ph = plan_single(c->sl_acc_blocks_beside, nh, kSLTile);
+  const size_t ebytes = ((size_t)Pd.S.nseg * Ke * sizeof(double) + 255) & ~(size_t)255;
+  const int rc = ensure_scratch(c, ebytes + (size_t)Ph.S.nseg * Ks * sizeof(double));
+  if (rc) return rc;
+  const AccIn d{dx, dy, dz, dm, Pd.S, (double*)c->scratch};
+  const AccIn h{hx, hy, hz, hm, Ph.S, (double*)((char*)c->scratch + ebytes)};
+  const int no_odd = (flags & BFE_NO_ODD) ? 1 : 0;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(Pd.grid + Ph.grid), dim3(256),
+                       std::max(lds, sizeof(EofTileLds<kSmallTile>)), s, d, eof_geom(c), c->eof_pot32, Ke,
+                       Pd.grid, h, sl_geom(c), c->sl_e32, c->sl_lmc, no_odd);
+  };
+  const int oe = (Ke + 255) / 256, os = (Ks + 255) / 256;
+  auto go_s = [&](auto e) {
+    constexpr int OE = decltype(e)::value;
+    if (os == 1) go(accumulate_both_kernel<OE, 1>);
+    else if (os == 2) go(accumulate_both_kernel<OE, 2>);
+    else go(accumulate_both_kernel<OE, 4>);
+  };
+  if (oe == 1) go_s(std::integral_constant<int, 1>{});
+  else if (oe == 2) go_s(std::integral_constant<int, 2>{});
+  else go_s(std::integral_constant<int, 4>{});
+  BFE_HIP(c, hipGetLastError());
+  hipLaunchKernelGGL(reduce_both_kernel,
+                     dim3((Ke + kRedCols - 1) / kRedCols + (Ks + kRedCols - 1) / kRedCols), dim3(256), 0, s,
+                     d.partials, (int)Pd.S.nseg, Ke, cos_out, sin_out, (c->mmax + 1) * c->norder, c->norder,
+                     h.partials, (int)Ph.S.nseg, Ks, coef_out);
+  BFE_HIP(c, hipGetLastError());
+  *done = true;
+  return 0;
+}
+
 // ---------------------------------------------------------------------------
 // Allocation-free EOF accumulate (bfe_eof_accumulate_noalloc)
 // ---------------------------------------------------------------------------
@@ -2067,6 +2191,10 @@ extern "C" int bfe_accumulate_disc_halo(bfe_ctx* h, const float* dx, const float
   if (rc) return rc;
   BFE_HIP(c, hipSetDevice(c->device));
   hipStream_t s = (hipStream_t)stream, s2 = nullptr;
+  bool done = false;
+  rc = accumulate_both_small(c, dx, dy, dz, dm, nd, hx, hy, hz, hm, nh, sl_flags, cos_out, sin_out,
+                             coef_out, s, &done);
+  if (rc || done) return rc;
   rc = fork_begin(c, s, &s2);
   if (rc) return rc;
   swap_work(c);

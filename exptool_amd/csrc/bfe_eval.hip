@@ -975,7 +975,8 @@ extern "C" int bfe_field_eval_cart(bfe_ctx* h, const float* x, const float* y, c
 //                  only positions and table geometry; the disc branch is
 //                  the shorter one, so the sort fills its idle tail);
 //   internal       halo SL accumulate (second buffer set), then the SL fold;
-// then, after the join, the evaluation.  Results equal
+// then, after the join, the evaluation.  Few particles take one stream with
+// both accumulates, reductions and folds each in one launch.  Results equal
 // bfe_accumulate_disc_halo + bfe_field_set + bfe_field_eval_cart over the
 // concatenated points.
 extern "C" int bfe_forces_disc_halo(bfe_ctx* h, const float* dx, const float* dy,
@@ -998,22 +999,10 @@ extern "C" int bfe_forces_disc_halo(bfe_ctx* h, const float* dx, const float* dy
   BFE_HIP(c, hipSetDevice(c->device));
   hipStream_t s = (hipStream_t)stream, s1 = nullptr;
   const int64_t n = nd + nh;
-  const int mm = disk_m < 0 ? c->mmax : std::min(disk_m, c->mmax);
-  const int nn = disk_n < 0 ? c->norder : std::min(disk_n, c->norder);
-  const int ll = halo_l < 0 ? c->lmax : std::min(halo_l, c->lmax);
-  const int hn = halo_n < 0 ? c->nmax : std::min(halo_n, c->nmax);
-  const bool no_odd = (field_flags & BFE_NO_ODD) != 0;
-  int rc = fork_begin(c, s, &s1);
+  bool done = false;
+  int rc = accumulate_both_small(c, dx, dy, dz, dm, nd, hx, hy, hz, hm, nh, acc_flags, cos_out, sin_out,
+                                 coef_out, s, &done);
   if (rc) return rc;
-  // halo: accumulate and fold on the first internal stream
-  swap_work(c);
-  int r1 = sl_accumulate_one(c, hx, hy, hz, hm, nh, acc_flags, coef_out, s1);
-  swap_work(c);
-  if (!r1) r1 = sl_fold(c, 1, coef_out, halofac, ll, hn, -(1 << 30), 1 << 30, no_odd, s1);
-  // disc: accumulate and fold on the caller's stream
-  int r0 = eof_accumulate_one(c, dx, dy, dz, dm, nd, cos_out, sin_out, s);
-  if (!r0) r0 = eof_fold(c, 1, cos_out, sin_out, mm, nn, 0, 1 << 30, no_odd,
-                         (field_flags & BFE_COMPAT_EOF_MASK) != 0, false, s);
   // the two inputs are evaluated as one set: by split blocks, or ordered
   const float4* pts = nullptr;
   FieldTables G;
@@ -1022,11 +1011,32 @@ extern "C" int bfe_forces_disc_halo(bfe_ctx* h, const float* dx, const float* dy
   G.lmax = c->lmax;
   G.flags = field_flags & (BFE_COMPAT_SL_COS_L | BFE_COMPAT_SL_EDGE);
   const bool split = n / 2 < c->order_min && n <= c->split_eval_max && split_ok(G);
-  if (!r0 && n > 0 && !split) {
-    r0 = order_points2(c, G, dx, dy, dz, nd, hx, hy, hz, nh, s, &pts);
+  if (done) {
+    rc = field_set_run(c, cos_out, sin_out, coef_out, halofac, disk_m, disk_n, halo_l, halo_n,
+                       field_flags, s);
+    if (!rc && !split) rc = order_points2(c, G, dx, dy, dz, nd, hx, hy, hz, nh, s, &pts);
+    if (rc) return rc;
+  } else {
+    const int mm = disk_m < 0 ? c->mmax : std::min(disk_m, c->mmax);
+    const int nn = disk_n < 0 ? c->norder : std::min(disk_n, c->norder);
+    const int ll = halo_l < 0 ? c->lmax : std::min(halo_l, c->lmax);
+    const int hn = halo_n < 0 ? c->nmax : std::min(halo_n, c->nmax);
+    const bool no_odd = (field_flags & BFE_NO_ODD) != 0;
+    rc = fork_begin(c, s, &s1);
+    if (rc) return rc;
+    // halo: accumulate and fold on the first internal stream
+    swap_work(c);
+    int r1 = sl_accumulate_one(c, hx, hy, hz, hm, nh, acc_flags, coef_out, s1);
+    swap_work(c);
+    if (!r1) r1 = sl_fold(c, 1, coef_out, halofac, ll, hn, -(1 << 30), 1 << 30, no_odd, s1);
+    // disc: accumulate and fold on the caller's stream
+    int r0 = eof_accumulate_one(c, dx, dy, dz, dm, nd, cos_out, sin_out, s);
+    if (!r0) r0 = eof_fold(c, 1, cos_out, sin_out, mm, nn, 0, 1 << 30, no_odd,
+                           (field_flags & BFE_COMPAT_EOF_MASK) != 0, false, s);
+    if (!r0 && n > 0 && !split) r0 = order_points2(c, G, dx, dy, dz, nd, hx, hy, hz, nh, s, &pts);
+    rc = fork_end(c, s);
+    if (r0 || r1 || rc) return r0 ? r0 : (r1 ? r1 : rc);
   }
-  rc = fork_end(c, s);
-  if (r0 || r1 || rc) return r0 ? r0 : (r1 ? r1 : rc);
   c->field_halofac = halofac;
   c->field_flags = (int)(field_flags & (BFE_COMPAT_SL_COS_L | BFE_COMPAT_SL_EDGE));
   FieldTables T;

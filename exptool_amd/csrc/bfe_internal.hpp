@@ -297,6 +297,10 @@ int eof_accumulate_one(Context* c, const float* x, const float* y, const float* 
                        const float* m, int64_t n, double* cos_out, double* sin_out, hipStream_t s);
 int sl_accumulate_one(Context* c, const float* x, const float* y, const float* z, const float* m,
                       int64_t n, uint32_t flags, double* coef_out, hipStream_t s);
+int accumulate_both_small(Context* c, const float* dx, const float* dy, const float* dz,
+                          const float* dm, int64_t nd, const float* hx, const float* hy,
+                          const float* hz, const float* hm, int64_t nh, uint32_t flags,
+                          double* cos_out, double* sin_out, double* coef_out, hipStream_t s, bool* done);
 // float64 per-point scratch in the ordering buffer (n entries), valid after
 // order_points for the same n.
 double* order_energy_buffer(Context* c, int64_t n);

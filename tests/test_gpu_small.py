@@ -125,3 +125,38 @@ def test_folds_of_a_batch_equal_single_folds(nset, lmax, mmax, numr, numx, numy)
     x, y, z = (v[-64:].cpu().numpy().astype(np.float64) for v in d[:3])
     for u, r in zip(f, O.total_force(F, x, y, z)):
         assert relmax(u[-64:].cpu().numpy(), r) <= 1e-5    # the field's bound, per output
+
+
+@pytest.mark.parametrize("lmax,nmax,mmax,norder", [(2, 5, 2, 5), (6, 9, 6, 21), (6, 20, 8, 33)])
+@pytest.mark.parametrize("nd,nh", [(1, 1), (64, 65), (1300, 3), (0, 70), (70, 0), (5000, 4097)])
+def test_small_dump_in_one_stream(nd, nh, lmax, nmax, mmax, norder):
+    """forces_disc_halo of few particles (both accumulates, reductions and folds
+    in one launch each): the coefficients of the oracle, and the bits of the
+    separate freeze and evaluation with them."""
+    import torch
+    from exptool_amd.bfe import BFESystem
+    from exptool_amd.utils import workloads as W
+    st, et = W.disc_halo_tables(seed=2, n_eof_sample=3000, lmax_s=10, nmax_s=max(8, norder),
+                                eof=dict(mmax=mmax, norder=norder, numx=20, numy=12),
+                                sl=dict(lmax=lmax, nmax=nmax, numr=150))
+    s = BFESystem(sl=st, eof=et)
+    d, h = (f32(*p) for p in W.disc_halo_particles(max(nd, 1), max(nh, 1), seed=5))
+    d, h = [a[:nd] for a in d], [a[:nh] for a in h]
+    slo = O.SLTable(st["lmax"], st["nmax"], st["numr"], st["cmap"], st["rmin"], st["rmax"], st["scale"],
+                    st["ev"], st["ef"], st["xi"], st["p0"], st["d0"])
+    eo = O.EOFTable(et["mmax"], et["norder"], et["numx"], et["numy"], et["cmap"], et["rmin"], et["rmax"],
+                    et["ascale"], et["hscale"], et["potC"], et["rforceC"], et["zforceC"], et["potS"],
+                    et["rforceS"], et["zforceS"], et["densC"], et["densS"])
+    out = s.forces_disc_halo(d, h, rotpos=0.2)
+    c, sn, g = out["cos"], out["sin"], out["coef"]
+    if nd:
+        rc, rs = O.eof_accumulate(eo, *d)
+        assert block_rel_eof(c.cpu().numpy(), rc) <= TOL
+        assert block_rel_eof(sn.cpu().numpy()[1:], rs[1:]) <= TOL
+    assert not nd or torch.all(sn[0] == 0)
+    if nh:
+        assert block_rel_sl(g.cpu().numpy(), O.sl_accumulate(slo, *h), lmax) <= TOL
+    s.set_field(c, sn, g)
+    ref = s.field_forces(*(np.concatenate([a, b]) for a, b in zip(d[:3], h[:3])), rotpos=0.2)
+    for k, v in zip(("fx", "fy", "fz", "pot"), ref):
+        assert torch.equal(out[k], v), k
