@@ -392,6 +392,9 @@ extern "C" int bfe_set_tuning(bfe_ctx* h, const char* name, int64_t value) {
   } else if (!strcmp(name, "order_min")) {
     if (value < 0) return set_error(c, BFE_EINVAL, "order_min < 0");
     c->order_min = value;
+  } else if (!strcmp(name, "point_blocks")) {
+    if (value < 0 || value > 65535) return set_error(c, BFE_EINVAL, "point_blocks outside [0, 65535]");
+    c->point_blocks = value;
   } else if (!strcmp(name, "split_max") || !strcmp(name, "split_eval_max")) {
     if (value < 0) return set_error(c, BFE_EINVAL, "%s < 0", name);
     (name[5] == '_' && name[6] == 'm' ? c->split_max : c->split_eval_max) = value;
@@ -427,6 +430,7 @@ extern "C" int bfe_get_tuning(const bfe_ctx* h, const char* name, int64_t* value
   else if (!strcmp(name, "sl_seg_tiles")) *value = c->sl_seg_tiles;
   else if (!strcmp(name, "order_min")) *value = c->order_min;
   else if (!strcmp(name, "split_max")) *value = c->split_max;
+  else if (!strcmp(name, "point_blocks")) *value = c->point_blocks;
   else if (!strcmp(name, "split_eval_max")) *value = c->split_eval_max;
   else if (!strcmp(name, "kernel_timing")) *value = c->kernel_timing ? 1 : 0;
   else if (!strcmp(name, "sl_acc_path")) *value = c->sl_acc_path;

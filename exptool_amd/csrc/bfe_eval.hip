@@ -33,24 +33,19 @@ struct SLFoldIn {
 };
 constexpr int kFoldLanes = 4;
 constexpr int kFoldRows = 2;
-__device__ __forceinline__ void sl_fold_block(const SLFoldIn& f, const SLFoldArgs& a, unsigned block,
-                                              int set) {
-  constexpr int R = kFoldRows;
+// Nodes i0 .. i0 + R - 1 of the pair at place j of the l-major order, into the
+// node blocks at o (2 np float4 a node) and the density blocks at od.
+template <int R>
+__device__ __forceinline__ void sl_fold_nodes(const SLFoldIn& f, const SLFoldArgs& a, int i0, int j,
+                                              int q, const double* __restrict__ c, float4* o,
+                                              float4* od) {
   const int np = sl_npairs(a.lmax), nmax = f.nmax, numr = f.numr;
-  const unsigned gid = block * blockDim.x + threadIdx.x;
-  const int q = (int)(gid & (kFoldLanes - 1));
-  const unsigned idx = gid / kFoldLanes;
-  const int g = (int)(idx / (unsigned)np);
-  const int i0 = g * R;
-  // groups of four lanes are whole within a wave, so a group leaves together
-  if (i0 >= numr) return;
   // lanes in l-major order, so that neighbours read the same rows
-  int l = 0, m = (int)(idx - (unsigned)g * (unsigned)np);
+  int l = 0, m = j;
   while (m > l) m -= ++l;
   const int p = m * (a.lmax + 1) - m * (m - 1) / 2 + l - m;
   const double mul = a.mul[p];
   const bool two = m > 0;
-  const double* c = f.coef + (size_t)set * f.coef_stride;
   const double* cc = c + (size_t)(l * l + (two ? 2 * m - 1 : 0)) * nmax;
   const double* cs = c + (size_t)(l * l + 2 * m) * nmax;
   const size_t plane = (size_t)(a.lmax + 1) * numr * nmax;
@@ -105,13 +100,11 @@ __device__ __forceinline__ void sl_fold_block(const SLFoldIn& f, const SLFoldArg
 #pragma unroll
     for (int k = 0; k < R + 2; ++k) w[k][h] = sum(w[k][h]);
   }
-  float4* o = reinterpret_cast<float4*>(f.out + (size_t)set * f.out_stride);
-  float4* od = o + (size_t)numr * np * 2;
 #pragma unroll
   for (int k = 0; k < R; ++k) {
     const int i = i0 + k;
     if (i >= numr) break;
-    const size_t at = (size_t)i * np + p;
+    const size_t at = (size_t)k * np + p;
     const bool last = i == numr - 1;
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
     if (q == 0) {
@@ -141,6 +134,21 @@ __device__ __forceinline__ void sl_fold_block(const SLFoldIn& f, const SLFoldArg
       od[at] = v;
     }
   }
+}
+
+__device__ __forceinline__ void sl_fold_block(const SLFoldIn& f, const SLFoldArgs& a, unsigned block,
+                                              int set) {
+  const int np = sl_npairs(a.lmax);
+  const unsigned gid = block * blockDim.x + threadIdx.x;
+  const unsigned idx = gid / kFoldLanes;
+  const int g = (int)(idx / (unsigned)np);
+  const int i0 = g * kFoldRows;
+  // groups of four lanes are whole within a wave, so a group leaves together
+  if (i0 >= f.numr) return;
+  float4* o = reinterpret_cast<float4*>(f.out + (size_t)set * f.out_stride);
+  sl_fold_nodes<kFoldRows>(f, a, i0, (int)(idx - (unsigned)g * (unsigned)np), (int)(gid & (kFoldLanes - 1)),
+                           f.coef + (size_t)set * f.coef_stride, o + (size_t)i0 * np * 2,
+                           o + (size_t)f.numr * np * 2 + (size_t)i0 * np);
 }
 
 __global__ __launch_bounds__(256) void sl_fold_kernel(SLFoldIn f, SLFoldArgs a) {
@@ -528,6 +536,104 @@ __global__ __launch_bounds__(256) void eof_eval_cyl_kernel(
   out[8 * n + i] = o.fz0;
 }
 
+// The point forms for few points: a block per point folds the coefficients into
+// the blocks of the point's own cell (the sums of the whole-table folds, in the
+// same order) and evaluates it from LDS.  A whole-table fold is 93 MB of table
+// reads and a launch of its own; a point needs 4 nodes of the disc's 33 153 and
+// one of the halo's 2 000.  Disc calls, whole-table fold / by cells: 24 points
+// 25.8 / 16.0 us, 512 31.1 / 16.8, 1 024 30.9 / 27.6, 2 048 31.0 / 48.9, hence
+// point_blocks = 512.
+template <bool DENS>
+__global__ __launch_bounds__(256) void sl_points_kernel(
+    SLFoldIn f, SLFoldArgs a, const double* __restrict__ pr, const double* __restrict__ pct,
+    const double* __restrict__ pph, int64_t n, SLGeom g, uint32_t flags, double densfac,
+    double* __restrict__ out) {
+  __shared__ float4 sA[2 * kMaxLM], sD[kMaxLM];
+  const int64_t p = blockIdx.x;
+  const double r = pr[p];
+  const SLCell cell = sl_locate(r, g.cmap, g.scale, g.xi, g.numr, g.idxi, g.xi0, g.xin);
+  const int lanes = sl_npairs(a.lmax) * kFoldLanes;
+  for (int t = threadIdx.x; t < lanes; t += 256)
+    sl_fold_nodes<1>(f, a, cell.i, t / kFoldLanes, t & (kFoldLanes - 1), f.coef, sA, sD);
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  double s1, c1;
+  sincos(pph[p], &s1, &c1);
+  SLOut o;
+  sl_eval_cell<DENS>(g, (const float4*)sA, sD, a.lmax, cell, pct[p], c1, s1, flags, o);
+  out[p] = DENS ? o.den0 * densfac : 0.0;
+  out[n + p] = DENS ? o.den1 * densfac : 0.0;
+  out[2 * n + p] = o.pot0;
+  out[3 * n + p] = o.pot1;
+  out[4 * n + p] = o.potr;
+  out[5 * n + p] = o.pott;
+  out[6 * n + p] = o.potp;
+}
+
+template <bool DENS>
+__global__ __launch_bounds__(256) void eof_points_kernel(
+    const float* __restrict__ T0, const float* __restrict__ T1, const float* __restrict__ T2,
+    const float* __restrict__ T3, const double* __restrict__ ccos, const double* __restrict__ csin,
+    const double* __restrict__ E, int64_t nodes, int64_t nedge, int norder, EOFFoldArgs a,
+    const double* __restrict__ pR, const double* __restrict__ pz, const double* __restrict__ pph,
+    int64_t n, EOFGeom g, double* __restrict__ out) {
+  __shared__ float4 sF[4][2 * (kMaxM + 1)];   // corner, (m, cos / sin): [pot, rf, zf, dens]
+  __shared__ double4 sE[4];                   // m = 0 in float64, last grid column or row
+  const int64_t i = blockIdx.x;
+  const EOFCell cell = eof_locate(pR[i], pz[i], g.cmap, g.ascale, g.ihscale, g.xmin, g.idx, g.ymin,
+                                  g.idy, g.numx, g.numy);
+  const bool edge = cell.ix == g.numx - 1 || cell.iy == g.numy - 1;
+  const int rows = 2 * g.mmax + 1;
+  // lane: value (pot, rf, zf, dens), corner (ix + c / 2, iy + c % 2), row group
+  for (int t = threadIdx.x; t < 16 * (rows + 1); t += 256) {
+    const int f = t & 3, c = (t >> 2) & 3, q = t >> 4;
+    const bool live = f < 3 || DENS;
+    const int x = cell.ix + (c >> 1), y = cell.iy + (c & 1);
+    if (q < rows) {
+      const bool sn = q > g.mmax;
+      const int m = sn ? q - g.mmax : q;
+      const double* cf = (sn ? csin : ccos) + (size_t)m * norder;
+      const float* T = (f == 0 ? T0 : f == 1 ? T1 : f == 2 ? T2 : T3) + (size_t)q * norder * nodes +
+                       (size_t)x * (g.numy + 1) + y;
+      double v = 0.0;
+      if (live) {
+#pragma unroll 6
+        for (int k = 0; k < a.nuse; ++k) v += cf[k] * T[(size_t)k * nodes];
+      }
+      reinterpret_cast<float*>(&sF[c][2 * m + (sn ? 1 : 0)])[f] = live ? (float)(v * a.mmul[m]) : 0.f;
+    } else if (edge) {
+      const double* e = E + (size_t)f * norder * nedge + eof_edge_index(x, y, g.numx, g.numy);
+      double v = 0.0;
+      if (live) {
+#pragma unroll 6
+        for (int k = 0; k < a.nuse; ++k) v += ccos[k] * e[(size_t)k * nedge];
+      }
+      reinterpret_cast<double*>(&sE[c])[f] = v * a.mmul[0];
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  auto wide = [](const float4& v) { return make_double4(v.x, v.y, v.z, v.w); };
+  EOFCorners0 q0;
+  q0.a = edge ? sE[0] : wide(sF[0][0]);
+  q0.b = edge ? sE[1] : wide(sF[1][0]);
+  q0.c = edge ? sE[2] : wide(sF[2][0]);
+  q0.e = edge ? sE[3] : wide(sF[3][0]);
+  double s1, c1;
+  sincos(pph[i], &s1, &c1);
+  EOFOut o;
+  eof_eval_corners<DENS>(cell, g.mmax, q0, sF[0], sF[1], sF[2], sF[3], c1, s1, o);
+  out[i] = o.p0;
+  out[n + i] = o.p;
+  out[2 * n + i] = o.fr;
+  out[3 * n + i] = o.fp;
+  out[4 * n + i] = o.fz;
+  out[5 * n + i] = DENS ? o.d0 : 0.0;
+  out[6 * n + i] = DENS ? o.d : 0.0;
+  out[7 * n + i] = o.fr0;
+  out[8 * n + i] = o.fz0;
+}
+
 // Fields.return_forces_cart at n points.  pts (may be NULL): the points in
 // table-cell order as float4 (x, y, z, input index bits), outputs scattered
 // back to input order; block b then takes logical block xcd_block(nb) so that
@@ -784,17 +890,31 @@ extern "C" int bfe_sl_eval_sph(bfe_ctx* h, const double* r, const double* costh,
   hipStream_t s = (hipStream_t)stream;
   const int ll = lmax_use < 0 ? c->lmax : std::min(lmax_use, c->lmax);
   const int nn = nmax_use < 0 ? c->nmax : std::min(nmax_use, c->nmax);
-  int rc = sl_fold(c, 0, coef, 1.0, ll, nn, -(1 << 30), 1 << 30, (flags & BFE_NO_ODD) != 0, s);
-  if (rc) return rc;
   if (n == 0) return 0;
+  const bool no_odd = (flags & BFE_NO_ODD) != 0;
+  const uint32_t pf = flags & (BFE_COMPAT_SL_EDGE | BFE_COMPAT_SL_COS_L);
+  if (n <= c->point_blocks) {
+    SLFoldIn in;
+    SLFoldArgs a;
+    sl_fold_args(c, coef, 1, 1.0, ll, nn, -(1 << 30), 1 << 30, no_odd, nullptr, &in, &a);
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)n), dim3(256), 0, s, in, a, r, costh, phi, n, sl_geom(c), pf,
+                         0.25 / kPi, out);
+    };
+    if (flags & BFE_EVAL_DENS) go(sl_points_kernel<true>);
+    else go(sl_points_kernel<false>);
+    BFE_HIP(c, hipGetLastError());
+    return 0;
+  }
+  int rc = sl_fold(c, 0, coef, 1.0, ll, nn, -(1 << 30), 1 << 30, no_odd, s);
+  if (rc) return rc;
   const SLFolded& f = c->slf[0];
-  const uint32_t ef = flags & (BFE_COMPAT_SL_EDGE | BFE_COMPAT_SL_COS_L);
   if (flags & BFE_EVAL_DENS)
     hipLaunchKernelGGL(sl_eval_sph_kernel<true>, dim3(nblocks256(n)), dim3(256), 0, s, r, costh,
-                       phi, n, sl_geom(c), f.d, c->lmax, ef, 0.25 / kPi, out);
+                       phi, n, sl_geom(c), f.d, c->lmax, pf, 0.25 / kPi, out);
   else
     hipLaunchKernelGGL(sl_eval_sph_kernel<false>, dim3(nblocks256(n)), dim3(256), 0, s, r, costh,
-                       phi, n, sl_geom(c), f.d, c->lmax, ef, 0.25 / kPi, out);
+                       phi, n, sl_geom(c), f.d, c->lmax, pf, 0.25 / kPi, out);
   BFE_HIP(c, hipGetLastError());
   return 0;
 }
@@ -816,10 +936,24 @@ extern "C" int bfe_eof_eval_cyl(bfe_ctx* h, const double* R, const double* z, co
   hipStream_t s = (hipStream_t)stream;
   const int mm = mmax_use < 0 ? c->mmax : std::min(mmax_use, c->mmax);
   const int nn = nmax_use < 0 ? c->norder : std::min(nmax_use, c->norder);
-  int rc = eof_fold(c, 0, cos_coef, sin_coef, mm, nn, 0, 1 << 30, (flags & BFE_NO_ODD) != 0,
-                    (flags & BFE_COMPAT_EOF_MASK) != 0, dens, s);
-  if (rc) return rc;
   if (n == 0) return 0;
+  const bool no_odd = (flags & BFE_NO_ODD) != 0, mask = (flags & BFE_COMPAT_EOF_MASK) != 0;
+  if (n <= c->point_blocks) {
+    EOFFoldIn in;
+    EOFFoldArgs a;
+    eof_fold_args(c, cos_coef, sin_coef, 1, 1, mm, nn, 0, 1 << 30, no_odd, mask, dens, nullptr, &in, &a);
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)n), dim3(256), 0, s, in.T[0], in.T[1], in.T[2], in.T[3],
+                         cos_coef, sin_coef, in.E, in.nodes, in.nedge, c->norder, a, R, z, phi, n,
+                         eof_geom(c), out);
+    };
+    if (dens) go(eof_points_kernel<true>);
+    else go(eof_points_kernel<false>);
+    BFE_HIP(c, hipGetLastError());
+    return 0;
+  }
+  int rc = eof_fold(c, 0, cos_coef, sin_coef, mm, nn, 0, 1 << 30, no_odd, mask, dens, s);
+  if (rc) return rc;
   const EOFFolded& f = c->eoff[0];
   if (dens)
     hipLaunchKernelGGL(eof_eval_cyl_kernel<true>, dim3(nblocks256(n)), dim3(256), 0, s, R, z, phi,

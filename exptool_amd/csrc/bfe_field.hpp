@@ -305,37 +305,24 @@ __device__ __forceinline__ SLRadial sl_radial(const SLGeom& g, const SLCell& cel
 // STAGED: node i's force blocks are read from the LDS copy Abase at
 // (i - ibase) * 2 np float4 (a block stages its nodes there); otherwise from
 // the folded table itself.
-template <bool DENS, bool STAGED = false>
-__device__ __forceinline__ void sl_eval_folded(const SLGeom& g, const float* __restrict__ F,
-                                               int L, double r, double costh, double c1,
-                                               double s1, uint32_t flags, SLOut& o,
-                                               const SLCell* pcell = nullptr,
-                                               const float4* Abase = nullptr, int ibase = 0) {
-  const SLCell cell = pcell ? *pcell : sl_locate(r, g.cmap, g.scale, g.xi, g.numr, g.idxi, g.xi0, g.xin);
+// The sums of sl_eval_folded in cell `cell` from its node's blocks: A (2 np
+// float4, in global memory or LDS) and the density block Nd.
+template <bool DENS, typename PA>
+__device__ __forceinline__ void sl_eval_cell(const SLGeom& g, PA A, const float4* __restrict__ Nd,
+                                             int L, const SLCell& cell, double costh, double c1,
+                                             double s1, uint32_t flags, SLOut& o) {
   const int i = cell.i;
   const double x1 = cell.x1, x2 = cell.x2;
   const SLRadial rad = sl_radial(g, cell, flags);
   const double P0 = rad.P0;
   const double D0 = DENS ? x1 * g.d0[i] + x2 * g.d0[i + 1] : 0.0;
   const float ps = rad.ps;
-  const int np = sl_npairs(L);
-  const float4* __restrict__ Nd =
-      reinterpret_cast<const float4*>(F + (size_t)g.numr * np * 8) + (size_t)i * np;
   const bool dq = (flags & BFE_COMPAT_SL_DENS) != 0;
   double acc[7];
-  if (STAGED) {
-    const LdsF4 A = (LdsF4)Abase + (size_t)(i - ibase) * 2 * np;
-    if (flags & BFE_COMPAT_SL_COS_L)
-      sl_angular_cosl<DENS>(g, A, Nd, L, (float)x1, (float)x2, ps, costh, c1, s1, dq, acc);
-    else
-      sl_angular<DENS>(g, A, Nd, L, (float)x1, (float)x2, ps, costh, c1, s1, dq, acc);
-  } else {
-    const float4* __restrict__ A = reinterpret_cast<const float4*>(F) + (size_t)i * 2 * np;
-    if (flags & BFE_COMPAT_SL_COS_L)
-      sl_angular_cosl<DENS>(g, A, Nd, L, (float)x1, (float)x2, ps, costh, c1, s1, dq, acc);
-    else
-      sl_angular<DENS>(g, A, Nd, L, (float)x1, (float)x2, ps, costh, c1, s1, dq, acc);
-  }
+  if (flags & BFE_COMPAT_SL_COS_L)
+    sl_angular_cosl<DENS>(g, A, Nd, L, (float)x1, (float)x2, ps, costh, c1, s1, dq, acc);
+  else
+    sl_angular<DENS>(g, A, Nd, L, (float)x1, (float)x2, ps, costh, c1, s1, dq, acc);
   o.pot0 = acc[0] * P0;
   o.pot = fma(acc[3], P0, acc[0] * P0);
   o.potr = acc[1] * rad.fac;
@@ -344,6 +331,26 @@ __device__ __forceinline__ void sl_eval_folded(const SLGeom& g, const float* __r
   o.pott = acc[4] * P0;
   o.potp = acc[5] * P0;
   o.den1 = acc[6] * D0;
+}
+
+template <bool DENS, bool STAGED = false>
+__device__ __forceinline__ void sl_eval_folded(const SLGeom& g, const float* __restrict__ F,
+                                               int L, double r, double costh, double c1,
+                                               double s1, uint32_t flags, SLOut& o,
+                                               const SLCell* pcell = nullptr,
+                                               const float4* Abase = nullptr, int ibase = 0) {
+  const SLCell cell = pcell ? *pcell : sl_locate(r, g.cmap, g.scale, g.xi, g.numr, g.idxi, g.xi0, g.xin);
+  const int i = cell.i;
+  const int np = sl_npairs(L);
+  const float4* __restrict__ Nd =
+      reinterpret_cast<const float4*>(F + (size_t)g.numr * np * 8) + (size_t)i * np;
+  if (STAGED) {
+    const LdsF4 A = (LdsF4)Abase + (size_t)(i - ibase) * 2 * np;
+    sl_eval_cell<DENS>(g, A, Nd, L, cell, costh, c1, s1, flags, o);
+  } else {
+    const float4* __restrict__ A = reinterpret_cast<const float4*>(F) + (size_t)i * 2 * np;
+    sl_eval_cell<DENS>(g, A, Nd, L, cell, costh, c1, s1, flags, o);
+  }
 }
 
 // m = 0 corner values [pot, rforce, zforce, dens] of a cell: from the float64
@@ -399,32 +406,15 @@ __device__ __forceinline__ void eof_term(const EOFWeights32& v, const float4& a,
   t[3] = cs_sum(sm, pc, -cm, ps);
 }
 
-// EOF evaluation at planar radius R, height z, angle phi from the folded
-// table (8-float block per m).  Bilinear weights as eof.py:443-451; sums as
-// force_eval (eof.py:842-870) and accumulated_eval_particles (:1092-1138):
-// fp = sum m (C sin m phi potC - S cos m phi potS) = -dPhi/dphi.  MU: unroll
-// count of the m loop (2 measured 7 % faster in the RK4 kernel, slower in
-// the leapfrog one).  Cells of the last grid column or row take their m = 0
-// corner values from the float64 edge blocks that follow the float32 table:
-// past the outer edges the weights extrapolate linearly (eof.py:414-415) and
-// grow without bound, and with them the rounding of the table values; the
-// m = 0 terms carry the largest values.  The m > 0 terms stay float32.
+// The sums of eof_eval_folded from the cell's four node blocks A (ix, iy), B (ix,
+// iy + 1), C (ix + 1, iy), D (ix + 1, iy + 1).
 template <bool DENS, int MU = 1>
-__device__ __forceinline__ void eof_eval_folded(const EOFGeom& g, const float* __restrict__ F,
-                                                double R, double z, double c1, double s1,
-                                                EOFOut& o) {
-  const EOFCell cell = eof_locate(R, z, g.cmap, g.ascale, g.ihscale, g.xmin, g.idx, g.ymin, g.idy,
-                                  g.numx, g.numy);
-  const int ny1 = g.numy + 1;
-  const int M = g.mmax;
-  const int ns4 = 2 * (M + 1);
-  const size_t n00 = (size_t)cell.ix * ny1 + cell.iy;
-  const float4* __restrict__ A = reinterpret_cast<const float4*>(F) + n00 * ns4;  // (ix, iy)
-  const float4* __restrict__ B = A + ns4;                                          // (ix, iy+1)
-  const float4* __restrict__ C = A + (size_t)ny1 * ns4;                            // (ix+1, iy)
-  const float4* __restrict__ D = C + ns4;                                          // (ix+1, iy+1)
-  // m = 0: [pot, rforce, zforce, dens] of the four corners
-  const EOFCorners0 q0 = eof_corners0(g, F, cell, A[0], B[0], C[0], D[0]);
+__device__ __forceinline__ void eof_eval_corners(const EOFCell& cell, int M, const EOFCorners0& q0,
+                                                 const float4* __restrict__ A,
+                                                 const float4* __restrict__ B,
+                                                 const float4* __restrict__ C,
+                                                 const float4* __restrict__ D, double c1, double s1,
+                                                 EOFOut& o) {
   const double p0 = eof_bil0(cell, q0.a.x, q0.c.x, q0.b.x, q0.e.x);
   const double fr0 = eof_bil0(cell, q0.a.y, q0.c.y, q0.b.y, q0.e.y);
   const double fz0 = eof_bil0(cell, q0.a.z, q0.c.z, q0.b.z, q0.e.z);
@@ -457,6 +447,34 @@ __device__ __forceinline__ void eof_eval_folded(const EOFGeom& g, const float* _
   o.d = d;
   o.fr0 = fr0;
   o.fz0 = fz0;
+}
+
+// EOF evaluation at planar radius R, height z, angle phi from the folded
+// table (8-float block per m).  Bilinear weights as eof.py:443-451; sums as
+// force_eval (eof.py:842-870) and accumulated_eval_particles (:1092-1138):
+// fp = sum m (C sin m phi potC - S cos m phi potS) = -dPhi/dphi.  MU: unroll
+// count of the m loop (2 measured 7 % faster in the RK4 kernel, slower in
+// the leapfrog one).  Cells of the last grid column or row take their m = 0
+// corner values from the float64 edge blocks that follow the float32 table:
+// past the outer edges the weights extrapolate linearly (eof.py:414-415) and
+// grow without bound, and with them the rounding of the table values; the
+// m = 0 terms carry the largest values.  The m > 0 terms stay float32.
+template <bool DENS, int MU = 1>
+__device__ __forceinline__ void eof_eval_folded(const EOFGeom& g, const float* __restrict__ F,
+                                                double R, double z, double c1, double s1,
+                                                EOFOut& o) {
+  const EOFCell cell = eof_locate(R, z, g.cmap, g.ascale, g.ihscale, g.xmin, g.idx, g.ymin, g.idy,
+                                  g.numx, g.numy);
+  const int ny1 = g.numy + 1;
+  const int ns4 = 2 * (g.mmax + 1);
+  const size_t n00 = (size_t)cell.ix * ny1 + cell.iy;
+  const float4* __restrict__ A = reinterpret_cast<const float4*>(F) + n00 * ns4;  // (ix, iy)
+  const float4* __restrict__ B = A + ns4;                                          // (ix, iy+1)
+  const float4* __restrict__ C = A + (size_t)ny1 * ns4;                            // (ix+1, iy)
+  const float4* __restrict__ D = C + ns4;                                          // (ix+1, iy+1)
+  // m = 0: [pot, rforce, zforce, dens] of the four corners
+  const EOFCorners0 q0 = eof_corners0(g, F, cell, A[0], B[0], C[0], D[0]);
+  eof_eval_corners<DENS, MU>(cell, g.mmax, q0, A, B, C, D, c1, s1, o);
 }
 
 // The SL radial cell field_eval_point locates for the point (x, y, z).

@@ -162,6 +162,7 @@ struct Context {
                                    // evaluate in it from twice as many points
   int64_t split_max = 36864;       // orbits up to which the split integrators run
   int64_t split_eval_max = 131072; // points up to which the split evaluation runs
+  int64_t point_blocks = 512;      // points up to which the point evaluators fold only their cells
   int64_t sl_acc_path = 0;         // SL accumulate: 0 auto (vector ALU), 1 MFMA, 2 vector ALU
   int64_t eof_dep_shape = -1;      // cell-ordered EOF accumulate lane shape (index), -1 auto
   int64_t sl_dep_shape = -1;       // cell-ordered SL accumulate lane shape (index), -1 auto

@@ -160,3 +160,40 @@ def test_small_dump_in_one_stream(nd, nh, lmax, nmax, mmax, norder):
     ref = s.field_forces(*(np.concatenate([a, b]) for a, b in zip(d[:3], h[:3])), rotpos=0.2)
     for k, v in zip(("fx", "fy", "fz", "pot"), ref):
         assert torch.equal(out[k], v), k
+
+
+@pytest.mark.parametrize("density", [False, True])
+@pytest.mark.parametrize("lmax,mmax,numr,numx,numy", [(0, 0, 4, 8, 6), (6, 6, 201, 20, 15), (9, 16, 64, 31, 17)])
+def test_point_forms_by_cells_equal_whole_folds(lmax, mmax, numr, numx, numy, density):
+    """The point evaluators' fold of the points' own cells against the
+    whole-table folds: the same bits, in the first, last and middle cells, past
+    the tables, at r = 0, at NaN, with truncations, masks and options."""
+    import torch
+    from exptool_amd.bfe import BFESystem
+    from exptool_amd.utils import workloads as W
+    st, et = W.disc_halo_tables(seed=2, n_eof_sample=3000, lmax_s=16, nmax_s=8,
+                                eof=dict(mmax=mmax, norder=7, numx=numx, numy=numy),
+                                sl=dict(lmax=lmax, nmax=7, numr=numr))
+    s = BFESystem(sl=st, eof=et)
+    d, h = W.disc_halo_particles(500, 500, seed=3)
+    c, sn = s.eof_accumulate(*d)
+    hl = s.sl_accumulate(*h)
+    g = np.random.default_rng(5)
+    r = np.concatenate([[0.0, 1e-9, 1e-3, 1e6, np.nan, 1.0], 10 ** g.uniform(-3, 2, 95)])
+    z = np.concatenate([[0.0, 1e-9, -30.0, 1e6, 0.5, np.nan], g.normal(0, 0.5, 95)])
+    t = np.concatenate([[1.0, -1.0, 0.0, np.nan, 0.3, 0.1], g.uniform(-1, 1, 95)])
+    ph = g.uniform(-4, 4, r.size)
+    runs = [lambda n: s.sl_eval_sph(r[:n], t[:n], ph[:n], hl, density=density),
+            lambda n: s.sl_eval_sph(r[:n], t[:n], ph[:n], hl, lmax_use=2, nmax_use=3, no_odd=True,
+                                    density=density, edge=True),
+            lambda n: s.sl_eval_sph(r[:n], t[:n], ph[:n], hl, density=density, cos_l=True),
+            lambda n: s.eof_eval_cyl(r[:n], z[:n], ph[:n], c, sn, density=density),
+            lambda n: s.eof_eval_cyl(r[:n], z[:n], ph[:n], c, sn, mmax_use=2, nmax_use=3, no_odd=True,
+                                     compat_mask=True, density=density)]
+    for run in runs:
+        for n in (0, 1, r.size):
+            out = []
+            for pb in (0, 512):
+                s.set_tuning("point_blocks", pb)
+                out.append(run(n))
+            assert torch.equal(torch.nan_to_num(out[0], nan=7.5), torch.nan_to_num(out[1], nan=7.5))
