@@ -523,11 +523,15 @@ __device__ __forceinline__ void eof_to_run(float (&G)[PPT][4], double (&GD)[PPT]
 // of the sorted input gives its row weights -4 pi m {1, cos k phi, sin k phi}
 // (rows 0, k, mmax + k of sW), its four bilinear corner weights (sE, 64 per
 // corner: c00, c10, c01, c11) and its cell's first node (sB, also returned).
-__device__ __forceinline__ int eof_dep_setup(const float4* __restrict__ P, int64_t p, bool live,
+// pm: NULL when P holds the masses, else the masses by the input indices in P
+// (an order that the evaluation then shares).
+__device__ __forceinline__ int eof_dep_setup(const float4* __restrict__ P,
+                                             const float* __restrict__ pm, int64_t p, bool live,
                                              const EOFGeom& g, int ny1, int lane, float* sW,
                                              float* sE, int* sB) {
   const float4 q4 = live ? P[p] : make_float4(1.f, 0.f, 0.f, 0.f);
-  const double x = q4.x, y = q4.y, z = q4.z, mass = live ? (double)q4.w : 0.0;
+  const double x = q4.x, y = q4.y, z = q4.z;
+  const double mass = live ? (double)(pm ? pm[__float_as_int(q4.w)] : q4.w) : 0.0;
   const double R = sqrt(x * x + y * y + 1.e-10);
   double c1, s1v;
   planar_angle(x, y, c1, s1v);
@@ -581,8 +585,8 @@ __device__ __forceinline__ void eof_group(const float4 (&wv)[PPT], float4 e00, f
 // Body of the cell-ordered EOF accumulate; dsm is the block's dynamic LDS.
 template <int PPT, int CH>
 __device__ __forceinline__ void eof_deposit_body(
-    unsigned char* dsm, const float4* __restrict__ P, Segments S, EOFGeom g,
-    const float* __restrict__ T, int rp, int K, double* __restrict__ partials) {
+    unsigned char* dsm, const float4* __restrict__ P, const float* __restrict__ pm, Segments S,
+    EOFGeom g, const float* __restrict__ T, int rp, int K, double* __restrict__ partials) {
   // rp: padded row length of T, norder rounded up to a multiple of CH
   const int rowlen = (2 * g.mmax + 1) * rp;
   const int J = 2 * g.mmax + 1;
@@ -622,7 +626,7 @@ __device__ __forceinline__ void eof_deposit_body(
     for (int64_t t0 = s0 + 64 * wave; t0 < s1; t0 += 256) {
       const int64_t p = t0 + lane;
       const bool live = p < s1;
-      const int node = eof_dep_setup(P, p, live, g, ny1, lane, sW, sE, sB);
+      const int node = eof_dep_setup(P, pm, p, live, g, ny1, lane, sW, sE, sB);
       wave_sync();
       const int64_t left = s1 - t0;
       const int np = left < 64 ? (int)left : 64;
@@ -741,10 +745,10 @@ __device__ __forceinline__ void eof_deposit_body(
 template <int PPT, int CH>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(PPT == 1 && CH <= 8 ? 3 : 1))) void eof_deposit_kernel(
-    const float4* __restrict__ P, Segments S, EOFGeom g, const float* __restrict__ T, int rp,
-    int K, double* __restrict__ partials) {
+    const float4* __restrict__ P, const float* __restrict__ pm, Segments S, EOFGeom g,
+    const float* __restrict__ T, int rp, int K, double* __restrict__ partials) {
   extern __shared__ __align__(16) unsigned char dsm[];
-  eof_deposit_body<PPT, CH>(dsm, P, S, g, T, rp, K, partials);
+  eof_deposit_body<PPT, CH>(dsm, P, pm, S, g, T, rp, K, partials);
 }
 
 template <int PPT, int CH>
@@ -753,7 +757,7 @@ eof_deposit_alone_kernel(const float4* __restrict__ P, Segments S, EOFGeom g,
                          const float* __restrict__ T, int rp, int K,
                          double* __restrict__ partials) {
   extern __shared__ __align__(16) unsigned char dsm[];
-  eof_deposit_body<PPT, CH>(dsm, P, S, g, T, rp, K, partials);
+  eof_deposit_body<PPT, CH>(dsm, P, nullptr, S, g, T, rp, K, partials);
 }
 
 // eof_dep32[node][j][n < norder] = eof_pot32[node][j norder + n], zero for
@@ -822,8 +826,8 @@ __device__ __forceinline__ void sl_to_run(float (&A1)[PPT], float (&A2)[PPT], do
 // LM > 0: g.lmax == LM, known at compile time; LM = 0: any lmax.
 template <int PPT, int CH, int LM>
 __device__ __forceinline__ void sl_deposit_body(
-    unsigned char* dsm, const float4* __restrict__ P, Segments S, SLGeom g,
-    const float* __restrict__ E, const double* __restrict__ lmc, int no_odd,
+    unsigned char* dsm, const float4* __restrict__ P, const float* __restrict__ pm, Segments S,
+    SLGeom g, const float* __restrict__ E, const double* __restrict__ lmc, int no_odd,
     double* __restrict__ partials) {
   const int R = (g.lmax + 1) * (g.lmax + 1);
   const int K = R * g.nmax;
@@ -870,7 +874,8 @@ __device__ __forceinline__ void sl_deposit_body(
       float w1 = 0.f, w2 = 0.f;
       {
         const float4 q4 = live ? P[p] : make_float4(1.f, 0.f, 0.f, 0.f);
-        const double x = q4.x, y = q4.y, z = q4.z, mass = live ? (double)q4.w : 0.0;
+        const double x = q4.x, y = q4.y, z = q4.z;
+        const double mass = live ? (double)(pm ? pm[__float_as_int(q4.w)] : q4.w) : 0.0;
         double r = sqrt(x * x + y * y + z * z);
         r = (r == r) ? (r > 1.0e-10 ? r : 1.0e-10) : 1.0e-10;   // np.nanmax([r, 1e-10])
         const double costh = z / r;
@@ -1041,10 +1046,11 @@ __device__ __forceinline__ void sl_deposit_body(
 // nmax 20; beside the EOF accumulate the two-wave form gave the shorter call.
 template <int PPT, int CH, int LM>
 __global__ __launch_bounds__(256) void sl_deposit_kernel(
-    const float4* __restrict__ P, Segments S, SLGeom g, const float* __restrict__ E,
-    const double* __restrict__ lmc, int no_odd, double* __restrict__ partials) {
+    const float4* __restrict__ P, const float* __restrict__ pm, Segments S, SLGeom g,
+    const float* __restrict__ E, const double* __restrict__ lmc, int no_odd,
+    double* __restrict__ partials) {
   extern __shared__ __align__(16) unsigned char dsm[];
-  sl_deposit_body<PPT, CH, LM>(dsm, P, S, g, E, lmc, no_odd, partials);
+  sl_deposit_body<PPT, CH, LM>(dsm, P, pm, S, g, E, lmc, no_odd, partials);
 }
 
 template <int PPT, int CH, int LM>
@@ -1053,7 +1059,7 @@ sl_deposit_alone_kernel(const float4* __restrict__ P, Segments S, SLGeom g,
                         const float* __restrict__ E, const double* __restrict__ lmc, int no_odd,
                         double* __restrict__ partials) {
   extern __shared__ __align__(16) unsigned char dsm[];
-  sl_deposit_body<PPT, CH, LM>(dsm, P, S, g, E, lmc, no_odd, partials);
+  sl_deposit_body<PPT, CH, LM>(dsm, P, nullptr, S, g, E, lmc, no_odd, partials);
 }
 
 // ---------------------------------------------------------------------------
@@ -1702,6 +1708,9 @@ int eof_dep_prepare(Context* c) {
 }
 
 // beside: another accumulate runs concurrently (selects the deposit kernel).
+// order_out (beside only): receives the particles in cell order as (x, y, z,
+// input index), NULL when they are summed in input order; the masses are then
+// read by index, so the order serves the evaluation as well.
 // bf16 pieces of the potential table for the MFMA mode (once per table set).
 static int eof_mfma_prepare(Context* c, hipStream_t s) {
   if (c->eof_mfmaT) return 0;
@@ -1807,7 +1816,7 @@ static int eof_accumulate_mfma_run(Context* c, const float* x, const float* y, c
 static int eof_accumulate_run(Context* c, const float* x, const float* y, const float* z,
                               const float* m, int64_t n, const int64_t* off, int nsnap,
                               double* cos_out, double* sin_out, hipStream_t s,
-                              bool beside = false) {
+                              bool beside = false, const float4** order_out = nullptr) {
   const int K = c->eof_K;
   // cell-ordered form: (2 mmax + 1) rows x chunks of radial orders per lane,
   // LDS for the per-wave weights and the float64 wave reduction
@@ -1834,8 +1843,9 @@ static int eof_accumulate_run(Context* c, const float* x, const float* y, const 
   const float4* sorted = nullptr;
   if (ordered) {
     if ((rc = eof_dep_prepare(c))) return rc;
-    rc = order_particles(c, 0, x, y, z, m, n, off_dev, nsnap, s, &sorted, off);
+    rc = order_particles(c, 0, x, y, z, order_out ? nullptr : m, n, off_dev, nsnap, s, &sorted, off);
     if (rc) return rc;
+    if (order_out) *order_out = sorted;
   }
   timer_begin(c, "eof_accumulate", s);
   if (sorted) {
@@ -1843,7 +1853,7 @@ static int eof_accumulate_run(Context* c, const float* x, const float* y, const 
   else if (dsh.ppt == PP && dsh.ch == CC) {                                                   \
     if (beside)                                                                               \
       hipLaunchKernelGGL((eof_deposit_kernel<PP, CC>), dim3(P.grid), dim3(256), dlds, s,       \
-                         sorted, P.S, g, c->eof_dep32, c->eof_dep_rp, K, partials);           \
+                         sorted, order_out ? m : nullptr, P.S, g, c->eof_dep32, c->eof_dep_rp, K, partials);           \
     else                                                                                      \
       hipLaunchKernelGGL((eof_deposit_alone_kernel<PP, CC>), dim3(P.grid), dim3(256), dlds, s, \
                          sorted, P.S, g, c->eof_dep32, c->eof_dep_rp, K, partials);           \
@@ -1868,9 +1878,13 @@ static int eof_accumulate_run(Context* c, const float* x, const float* y, const 
 }
 
 // beside: another accumulate runs concurrently (selects the deposit kernel).
+// order_out (beside only): receives the particles in cell order as (x, y, z,
+// input index), NULL when they are summed in input order; the masses are then
+// read by index, so the order serves the evaluation as well.
 static int sl_accumulate_run(Context* c, const float* x, const float* y, const float* z,
                              const float* m, int64_t n, const int64_t* off, int nsnap, uint32_t flags,
-                             double* coef_out, hipStream_t s, bool beside = false) {
+                             double* coef_out, hipStream_t s, bool beside = false,
+                             const float4** order_out = nullptr) {
   const int R = (c->lmax + 1) * (c->lmax + 1);
   const int LN = (c->lmax + 1) * c->nmax;
   const int K = R * c->nmax;
@@ -1930,15 +1944,16 @@ static int sl_accumulate_run(Context* c, const float* x, const float* y, const f
   // LDS for the per-wave Y rows and the float64 wave reduction
   const float4* sorted = nullptr;
   if (ordered) {
-    rc = order_particles(c, 1, x, y, z, m, n, off_dev, nsnap, s, &sorted, off);
+    rc = order_particles(c, 1, x, y, z, order_out ? nullptr : m, n, off_dev, nsnap, s, &sorted, off);
     if (rc) return rc;
+    if (order_out) *order_out = sorted;
   }
   timer_begin(c, "sl_accumulate", s);
   if (sorted) {
 #define BFE_SL_DEP_LM(PP, CC, LL)                                                              \
   if (beside)                                                                                  \
     hipLaunchKernelGGL((sl_deposit_kernel<PP, CC, LL>), dim3(P.grid), dim3(256), dlds, s, sorted, \
-                       P.S, g, c->sl_dep32, c->sl_lmc, no_odd, partials);                      \
+                       order_out ? m : nullptr, P.S, g, c->sl_dep32, c->sl_lmc, no_odd, partials);                      \
   else                                                                                         \
     hipLaunchKernelGGL((sl_deposit_alone_kernel<PP, CC, LL>), dim3(P.grid), dim3(256), dlds, s,  \
                        sorted, P.S, g, c->sl_dep32, c->sl_lmc, no_odd, partials);
@@ -2077,13 +2092,17 @@ static int eof_accumulate_noalloc_run(Context* c, const float* x, const float* y
 }
 
 int eof_accumulate_one(Context* c, const float* x, const float* y, const float* z,
-                       const float* m, int64_t n, double* cos_out, double* sin_out, hipStream_t s) {
-  return eof_accumulate_run(c, x, y, z, m, n, nullptr, 1, cos_out, sin_out, s, true);
+                       const float* m, int64_t n, double* cos_out, double* sin_out, hipStream_t s,
+                       const float4** order_out) {
+  *order_out = nullptr;
+  return eof_accumulate_run(c, x, y, z, m, n, nullptr, 1, cos_out, sin_out, s, true, order_out);
 }
 
 int sl_accumulate_one(Context* c, const float* x, const float* y, const float* z, const float* m,
-                      int64_t n, uint32_t flags, double* coef_out, hipStream_t s) {
-  return sl_accumulate_run(c, x, y, z, m, n, nullptr, 1, flags, coef_out, s, true);
+                      int64_t n, uint32_t flags, double* coef_out, hipStream_t s,
+                      const float4** order_out) {
+  *order_out = nullptr;
+  return sl_accumulate_run(c, x, y, z, m, n, nullptr, 1, flags, coef_out, s, true, order_out);
 }
 
 }  // namespace bfe

@@ -640,15 +640,25 @@ __global__ __launch_bounds__(256) void eof_points_kernel(
 // each XCD evaluates a contiguous range of cells.  Without pts, point j of
 // px/py/pz.  In cell order a block's points usually share a few SL radial
 // nodes: when their force blocks fit in kStageFloat4, the block copies them
-// to LDS and the SL sums read them there.
+// to LDS and the SL sums read them there.  pts2 (may be NULL): a second set of n2
+// points in its own cell order, numbered after the first.
 __global__ __launch_bounds__(256) void field_eval_kernel(
     const float* __restrict__ px, const float* __restrict__ py, const float* __restrict__ pz,
-    int64_t n, const float4* __restrict__ pts, FieldTables T, float* fx, float* fy, float* fz,
-    float* pot, float* comp, float4* __restrict__ quad) {
+    int64_t n, const float4* __restrict__ pts, const float4* __restrict__ pts2, int64_t n2,
+    FieldTables T, float* fx, float* fy, float* fz, float* pot, float* comp,
+    float4* __restrict__ quad, int64_t total) {
   __shared__ float4 stage[kStageFloat4];
   __shared__ int smin[4], smax[4];
-  const int64_t nb = (n + 255) / 256;
-  const int64_t j = (pts ? xcd_block(nb) : (int64_t)blockIdx.x) * 256 + threadIdx.x;
+  // the second set's blocks follow the first's, whose number is a multiple of eight
+  const unsigned b1 = 8 * (unsigned)((n + 2047) / 2048);
+  const bool second = pts2 && blockIdx.x >= b1;
+  const int64_t base = second ? n : 0;
+  const unsigned b = second ? blockIdx.x - b1 : blockIdx.x;
+  if (second) {
+    pts = pts2;
+    n = n2;
+  }
+  const int64_t j = (pts ? xcd_block((n + 255) / 256, b) : (int64_t)b) * 256 + threadIdx.x;
   if (pts && (j - threadIdx.x) >= n) return;   // whole block past the end (XCD mapping)
   const bool live = j < n;
   float qx = 0.f, qy = 0.f, qz = 0.f;
@@ -657,7 +667,7 @@ __global__ __launch_bounds__(256) void field_eval_kernel(
     if (pts) {
       const float4 q = pts[j];
       qx = q.x; qy = q.y; qz = q.z;
-      i = (int64_t)__float_as_int(q.w);
+      i = base + (int64_t)__float_as_int(q.w);
     } else {
       qx = px[j]; qy = py[j]; qz = pz[j];
       i = j;
@@ -688,7 +698,7 @@ __global__ __launch_bounds__(256) void field_eval_kernel(
   if (pot) pot[i] = (float)(cv[6] + cv[7]);
   if (comp) {
 #pragma unroll
-    for (int k = 0; k < 8; ++k) comp[(size_t)k * n + i] = (float)cv[k];
+    for (int k = 0; k < 8; ++k) comp[(size_t)k * total + i] = (float)cv[k];
   }
 }
 
@@ -1018,7 +1028,8 @@ __global__ __launch_bounds__(256) void quad_split_kernel(const float4* __restric
 // pass splits it into fx, fy, fz, pot.
 static int field_eval_run(Context* c, const FieldTables& T, const float* x, const float* y,
                           const float* z, int64_t n, const float4* pts, float* fx, float* fy,
-                          float* fz, float* pot, float* comp, hipStream_t s) {
+                          float* fz, float* pot, float* comp, hipStream_t s,
+                          const float4* pts2 = nullptr, int64_t n1 = 0) {
   if (n == 0) return 0;
   float4* quad = nullptr;
   if (pts && !comp && (fx || fy || fz || pot)) {
@@ -1026,10 +1037,11 @@ static int field_eval_run(Context* c, const FieldTables& T, const float* x, cons
     if (rc) return rc;
     quad = (float4*)c->scratch;
   }
-  const unsigned grid = pts ? xcd_grid(nblocks256(n)) : nblocks256(n);
+  const unsigned grid = pts2 ? xcd_grid(nblocks256(n1)) + xcd_grid(nblocks256(n - n1))
+                        : pts ? xcd_grid(nblocks256(n)) : nblocks256(n);
   timer_begin(c, "field_eval", s);
-  hipLaunchKernelGGL(field_eval_kernel, dim3(grid), dim3(256), 0, s, x, y, z, n, pts, T, fx, fy,
-                     fz, pot, comp, quad);
+  hipLaunchKernelGGL(field_eval_kernel, dim3(grid), dim3(256), 0, s, x, y, z, pts2 ? n1 : n, pts, pts2,
+                     n - n1, T, fx, fy, fz, pot, comp, quad, n);
   timer_end(c, "field_eval", s);
   BFE_HIP(c, hipGetLastError());
   if (quad) {
@@ -1104,12 +1116,13 @@ extern "C" int bfe_field_eval_cart(bfe_ctx* h, const float* x, const float* y, c
 // Fields.total_coefficients followed by Fields.return_forces_cart at the
 // same particles (potential.py:98-252, :445-497).  Two concurrent branches,
 // each folding its coefficients as soon as they are reduced:
-//   caller stream  disc EOF accumulate, the EOF fold, then the evaluation
-//                  order of all nd + nh points taken as one set (it needs
-//                  only positions and table geometry; the disc branch is
-//                  the shorter one, so the sort fills its idle tail);
+//   caller stream  disc EOF accumulate, then the EOF fold (the longer branch,
+//                  launched first);
 //   internal       halo SL accumulate (second buffer set), then the SL fold;
-// then, after the join, the evaluation.  Few particles take one stream with
+// then, after the join, the evaluation: in the two orders that the accumulates
+// sorted their particles to (ordering all points once more for it took 80 us of
+// 427 at 1M + 1M), or, where one of them sums in input order, in an order of
+// all points made on the caller's stream.  Few particles take one stream with
 // both accumulates, reductions and folds each in one launch.  Results equal
 // bfe_accumulate_disc_halo + bfe_field_set + bfe_field_eval_cart over the
 // concatenated points.
@@ -1138,7 +1151,7 @@ extern "C" int bfe_forces_disc_halo(bfe_ctx* h, const float* dx, const float* dy
                                  coef_out, s, &done);
   if (rc) return rc;
   // the two inputs are evaluated as one set: by split blocks, or ordered
-  const float4* pts = nullptr;
+  const float4 *pts = nullptr, *pts2 = nullptr;
   FieldTables G;
   G.slg = sl_geom(c);
   G.eg = eof_geom(c);
@@ -1158,16 +1171,24 @@ extern "C" int bfe_forces_disc_halo(bfe_ctx* h, const float* dx, const float* dy
     const bool no_odd = (field_flags & BFE_NO_ODD) != 0;
     rc = fork_begin(c, s, &s1);
     if (rc) return rc;
-    // halo: accumulate and fold on the first internal stream
-    swap_work(c);
-    int r1 = sl_accumulate_one(c, hx, hy, hz, hm, nh, acc_flags, coef_out, s1);
-    swap_work(c);
-    if (!r1) r1 = sl_fold(c, 1, coef_out, halofac, ll, hn, -(1 << 30), 1 << 30, no_odd, s1);
-    // disc: accumulate and fold on the caller's stream
-    int r0 = eof_accumulate_one(c, dx, dy, dz, dm, nd, cos_out, sin_out, s);
+    const float4 *dpts = nullptr, *hpts = nullptr;
+    // disc: accumulate and fold on the caller's stream, the longer branch first
+    int r0 = eof_accumulate_one(c, dx, dy, dz, dm, nd, cos_out, sin_out, s, &dpts);
     if (!r0) r0 = eof_fold(c, 1, cos_out, sin_out, mm, nn, 0, 1 << 30, no_odd,
                            (field_flags & BFE_COMPAT_EOF_MASK) != 0, false, s);
-    if (!r0 && n > 0 && !split) r0 = order_points2(c, G, dx, dy, dz, nd, hx, hy, hz, nh, s, &pts);
+    // halo: accumulate and fold on the first internal stream
+    swap_work(c);
+    int r1 = sl_accumulate_one(c, hx, hy, hz, hm, nh, acc_flags, coef_out, s1, &hpts);
+    swap_work(c);
+    if (!r1) r1 = sl_fold(c, 1, coef_out, halofac, ll, hn, -(1 << 30), 1 << 30, no_odd, s1);
+    if (dpts && hpts) {
+      // both orders are there: the disc's EOF cells (few SL nodes and EOF cells a
+      // block) and the halo's evaluation cells
+      pts = dpts;
+      pts2 = hpts;
+    } else if (!r0 && n > 0 && !split) {
+      r0 = order_points2(c, G, dx, dy, dz, nd, hx, hy, hz, nh, s, &pts);
+    }
     rc = fork_end(c, s);
     if (r0 || r1 || rc) return r0 ? r0 : (r1 ? r1 : rc);
   }
@@ -1178,7 +1199,7 @@ extern "C" int bfe_forces_disc_halo(bfe_ctx* h, const float* dx, const float* dy
   if (rc || n == 0) return rc;
   if (split)
     return field_eval_split_run(c, T, dx, dy, dz, nd, hx, hy, hz, n, fx, fy, fz, pot, comp, s);
-  return field_eval_run(c, T, nullptr, nullptr, nullptr, n, pts, fx, fy, fz, pot, comp, s);
+  return field_eval_run(c, T, nullptr, nullptr, nullptr, n, pts, fx, fy, fz, pot, comp, s, pts2, nd);
 }
 
 extern "C" int bfe_field_set_batch(bfe_ctx* h, const double* eof_cos, const double* eof_sin,

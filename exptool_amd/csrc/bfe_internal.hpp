@@ -293,11 +293,15 @@ int order_particles(Context* c, int kind, const float* x, const float* y, const 
 // Single-snapshot accumulates (bfe_eof_accumulate / bfe_sl_accumulate
 // without the argument checks), enqueued on s with the current buffer set.
 // Both are for callers that run them side by side (they take the deposit
-// kernels sized for sharing the GPU).
+// kernels sized for sharing the GPU).  order_out receives the particles in
+// cell order as (x, y, z, input index) in the order buffer, NULL when they were
+// summed in input order.
 int eof_accumulate_one(Context* c, const float* x, const float* y, const float* z,
-                       const float* m, int64_t n, double* cos_out, double* sin_out, hipStream_t s);
+                       const float* m, int64_t n, double* cos_out, double* sin_out, hipStream_t s,
+                       const float4** order_out);
 int sl_accumulate_one(Context* c, const float* x, const float* y, const float* z, const float* m,
-                      int64_t n, uint32_t flags, double* coef_out, hipStream_t s);
+                      int64_t n, uint32_t flags, double* coef_out, hipStream_t s,
+                      const float4** order_out);
 int accumulate_both_small(Context* c, const float* dx, const float* dy, const float* dz,
                           const float* dm, int64_t nd, const float* hx, const float* hy,
                           const float* hz, const float* hm, int64_t nh, uint32_t flags,
@@ -317,10 +321,11 @@ void batch_free(Context* c);
 // cell-ordered points), keeping each XCD's L2 on its own part of the tables.
 // Launch with xcd_grid(nb) blocks; logical blocks >= nb do nothing.
 inline unsigned xcd_grid(int64_t nb) { return (unsigned)(8 * ((nb + 7) / 8)); }
-__device__ __forceinline__ int64_t xcd_block(int64_t nb) {
+__device__ __forceinline__ int64_t xcd_block(int64_t nb, unsigned b) {
   const int64_t per = (nb + 7) / 8;
-  return (int64_t)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  return (int64_t)(b & 7) * per + (b >> 3);
 }
+__device__ __forceinline__ int64_t xcd_block(int64_t nb) { return xcd_block(nb, blockIdx.x); }
 
 // With kernel_timing on, record HIP events around a compute kernel launch on
 // stream s (read back by bfe_kernel_times).

@@ -197,3 +197,33 @@ def test_point_forms_by_cells_equal_whole_folds(lmax, mmax, numr, numx, numy, de
                 s.set_tuning("point_blocks", pb)
                 out.append(run(n))
             assert torch.equal(torch.nan_to_num(out[0], nan=7.5), torch.nan_to_num(out[1], nan=7.5))
+
+
+@pytest.mark.parametrize("comp", [False, True])
+@pytest.mark.parametrize("nd,nh", [(1, 1), (255, 257), (2048, 2049), (4099, 300), (3, 5000)])
+def test_dump_evaluated_in_the_accumulate_orders(big, particles, nd, nh, comp):  # noqa: F811
+    """Both accumulates in cell order: the evaluation takes their two orders (and
+    the deposits read masses by index).  Coefficients as the separate calls'
+    within the float32 sums, field bits as the separate evaluation's; with one
+    side in input order the points are ordered together."""
+    import torch
+    s, _, _ = big
+    d, h = ([torch.tensor(a[:n], dtype=torch.float32, device="cuda") for a in p]
+            for p, n in zip(particles, (nd, nh)))
+    for omin in (1, min(nd, nh) + 1):
+        s.set_tuning("order_min", omin)
+        s.set_tuning("split_eval_max", 0)
+        out = s.forces_disc_halo(d, h, rotpos=0.2, components=comp)
+        c, sn = s.eof_accumulate(*d)
+        hl = s.sl_accumulate(*h)
+        s.set_tuning("order_min", 1 << 40)
+        s.set_field(out["cos"], out["sin"], out["coef"])
+        ref = s.field_forces(*(torch.cat([a, b]) for a, b in zip(d[:3], h[:3])), rotpos=0.2,
+                             components=comp)
+        s.set_tuning("order_min", 65536)
+        s.set_tuning("split_eval_max", 131072)
+        assert block_rel_eof(out["cos"].cpu().numpy(), c.cpu().numpy()) <= TOL
+        assert block_rel_eof(out["sin"].cpu().numpy()[1:], sn.cpu().numpy()[1:]) <= TOL
+        assert block_rel_sl(out["coef"].cpu().numpy(), hl.cpu().numpy(), 6) <= TOL
+        for k, v in zip(("fx", "fy", "fz", "pot", "comp"), ref):
+            assert torch.equal(out[k], v), k
