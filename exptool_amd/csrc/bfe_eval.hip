@@ -642,7 +642,7 @@ __global__ __launch_bounds__(256) void eof_points_kernel(
 // nodes: when their force blocks fit in kStageFloat4, the block copies them
 // to LDS and the SL sums read them there.  pts2 (may be NULL): a second set of n2
 // points in its own cell order, numbered after the first.
-__global__ __launch_bounds__(256) void field_eval_kernel(
+__global__ __launch_bounds__(256, 4) void field_eval_kernel(
     const float* __restrict__ px, const float* __restrict__ py, const float* __restrict__ pz,
     int64_t n, const float4* __restrict__ pts, const float4* __restrict__ pts2, int64_t n2,
     FieldTables T, float* fx, float* fy, float* fz, float* pot, float* comp,
