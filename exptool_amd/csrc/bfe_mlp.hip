@@ -61,7 +61,9 @@ constexpr int kBlockInf = BFE_MLP_BLOCK;
 constexpr int kInfPts = kWaveTile * kBlockInf / 64;   // points per block
 // The conservative-field kernels carry three tangent operand sets beside the
 // activations: four waves per block, one per SIMD, keep them in registers.
-constexpr int kBlockGrad = 256;
+constexpr int kBlockGrad = 512;
+constexpr int kBlockGradStep = 256;
+constexpr int kGradBlocks = 256;
 // LDS copy of the three hidden weight matrices: rows of kH bf16 padded to
 // kLdsRow.  A lane reads 16 bytes of row 16 mt + c; unpadded (256-byte)
 // rows put the rows that one read cycle serves on the same four banks, with
@@ -279,62 +281,85 @@ __device__ __forceinline__ void mlp_tile_forward(const __bf16* __restrict__ sW,
 // accumulation, tangents rounded to bf16 as the activations are), and
 // dy0/df_k = W4[0] . t_4^k.  Layout as mlp_tile_forward; NT 16-point tiles.
 //
-// One hidden layer W of it: the value pass (activations into B, or LAST: the
-// potential row of the output layer into ys) and the three tangent passes
-// (into T, or LAST: into ds).
+// One hidden layer W of it, 32 output neurons (one operand of the next layer) at
+// a time: each A fragment is read from LDS once and multiplied into the
+// activations (acc[0], from the bias) and the three tangents (acc[1..3], from
+// zero).  The activations of one group (B2, T2; LAST: into the sums ys, ds of the
+// potential row) run on the vector ALUs while the products of the next are on the
+// matrix cores: the scheduling groups place three vector instructions behind each
+// product, which is about what both units take.
 template <int NT, bool LAST>
 __device__ __forceinline__ void grad_layer(const __bf16* __restrict__ W, const float* bias,
-                                           const float* __restrict__ sW4, bf16x8 (&B)[4][NT],
-                                           bf16x8 (&T)[3][4][NT], float (&ys)[NT],
-                                           float (&ds)[NT][3], int g, int c) {
-  // One sweep over W: each A fragment is read from LDS once and multiplied
-  // into the activations (acc[0], from the bias) and the three tangents
-  // (acc[1..3], from zero), 4 NT independent products per fragment.
-  floatx4 acc[4][8][NT];
+                                           const float* __restrict__ sW4,
+                                           const bf16x8 (&B)[4][NT], const bf16x8 (&T)[3][4][NT],
+                                           bf16x8 (&B2)[4][NT], bf16x8 (&T2)[3][4][NT],
+                                           float (&ys)[NT], float (&ds)[NT][3], int g, int c) {
+  floatx4 acc[2][4][2][NT];
   const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+  auto products = [&](int mp, floatx4 (&ac)[4][2][NT]) {
 #pragma unroll
-  for (int kk = 0; kk < 4; ++kk) {
-    // one K-step's operand loads in flight at a time (register budget)
+    for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int mt = 2 * mp + h;
+        const bf16x8 a = *reinterpret_cast<const bf16x8*>(W + (16 * mt + c) * kLdsRow + 32 * kk + 8 * g);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+          if (kk == 0) {
+            floatx4 b0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) b0[i] = bias[16 * mt + 4 * g + i];
+            ac[0][h][nt] = mfma16(a, B[0][nt], b0);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) ac[1 + k][h][nt] = mfma16(a, T[k][0][nt], zero);
+          } else {
+            ac[0][h][nt] = mfma16(a, B[kk][nt], ac[0][h][nt]);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) ac[1 + k][h][nt] = mfma16(a, T[k][kk][nt], ac[1 + k][h][nt]);
+          }
+        }
+      }
+  };
+  auto activate = [&](int mp, const floatx4 (&ac)[4][2][NT]) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int mt = 2 * mp + h;
+          const float zz = ac[0][h][nt][i];
+          const float sg = sigmoid(zz);
+          const float hh = zz * sg;
+          const float dsl = sg * (1.f + zz * (1.f - sg));
+          if (LAST) ys[nt] = fmaf(sW4[16 * mt + 4 * g + i], hh, ys[nt]);
+          else B2[mp][nt][h * 4 + i] = (__bf16)hh;
+#pragma unroll
+          for (int k = 0; k < 3; ++k) {
+            const float tt = dsl * ac[1 + k][h][nt][i];
+            if (LAST) ds[nt][k] = fmaf(sW4[16 * mt + 4 * g + i], tt, ds[nt][k]);
+            else T2[k][mp][nt][h * 4 + i] = (__bf16)tt;
+          }
+        }
+  };
+  products(0, acc[0]);
+#pragma unroll
+  for (int mp = 0; mp < 4; ++mp) {
     __builtin_amdgcn_sched_barrier(0);
+    if (mp < 3) products(mp + 1, acc[(mp + 1) & 1]);
+    activate(mp, acc[mp & 1]);
+    if (mp < 3) {
 #pragma unroll
-    for (int mt = 0; mt < 8; ++mt) {
-      const bf16x8 a = *reinterpret_cast<const bf16x8*>(W + (16 * mt + c) * kLdsRow + 32 * kk + 8 * g);
+      for (int i = 0; i < 8; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // an LDS read
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        if (kk == 0) {
-          floatx4 b0;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) b0[i] = bias[16 * mt + 4 * g + i];
-          acc[0][mt][nt] = mfma16(a, B[0][nt], b0);
-#pragma unroll
-          for (int k = 0; k < 3; ++k) acc[1 + k][mt][nt] = mfma16(a, T[k][0][nt], zero);
-        } else {
-          acc[0][mt][nt] = mfma16(a, B[kk][nt], acc[0][mt][nt]);
-#pragma unroll
-          for (int k = 0; k < 3; ++k) acc[1 + k][mt][nt] = mfma16(a, T[k][kk][nt], acc[1 + k][mt][nt]);
+        for (int k = 0; k < 4 * NT; ++k) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // a product
+          __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);   // three vector instructions
         }
       }
     }
   }
-#pragma unroll
-  for (int mt = 0; mt < 8; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float zz = acc[0][mt][nt][i];
-        const float sg = sigmoid(zz);
-        const float hh = zz * sg;
-        const float dsl = sg * (1.f + zz * (1.f - sg));
-        if (LAST) ys[nt] = fmaf(sW4[16 * mt + 4 * g + i], hh, ys[nt]);
-        else B[mt >> 1][nt][(mt & 1) * 4 + i] = (__bf16)hh;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          const float tt = dsl * acc[1 + k][mt][nt][i];
-          if (LAST) ds[nt][k] = fmaf(sW4[16 * mt + 4 * g + i], tt, ds[nt][k]);
-          else T[k][mt >> 1][nt][(mt & 1) * 4 + i] = (__bf16)tt;
-        }
-      }
 }
 
 template <int NT>
@@ -372,12 +397,11 @@ __device__ __forceinline__ void mlp_tile_grad(const __bf16* __restrict__ sW,
     ys[nt] = 0.f;
     ds[nt][0] = ds[nt][1] = ds[nt][2] = 0.f;
   }
-  // layers 1 and 2 feed the next layer's operands; the last layer is peeled
-  // so that no activation carries a branch on the layer
-#pragma unroll 1
-  for (int layer = 0; layer < 2; ++layer)
-    grad_layer<NT, false>(sW + layer * kLdsLayer, sBh + layer * kH, sW4, B, T, ys, ds, g, c);
-  grad_layer<NT, true>(sW + 2 * kLdsLayer, sBh + 2 * kH, sW4, B, T, ys, ds, g, c);
+  bf16x8 B2[4][NT];
+  bf16x8 T2[3][4][NT];
+  grad_layer<NT, false>(sW, sBh, sW4, B, T, B2, T2, ys, ds, g, c);
+  grad_layer<NT, false>(sW + kLdsLayer, sBh + kH, sW4, B2, T2, B, T, ys, ds, g, c);
+  grad_layer<NT, true>(sW + 2 * kLdsLayer, sBh + 2 * kH, sW4, B, T, B2, T2, ys, ds, g, c);
   // sums over the four lane groups that hold the same point column
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
@@ -453,9 +477,12 @@ __global__ __launch_bounds__(kBlockInf) void mlp_fwd_kernel(MLPKArgs a) {
 }
 
 // Inference of the conservative field: out = Phi, F_R, F_phi, F_z with
-// F = -grad Phi (mlp_tile_grad, 16-point tiles per wave).
-__global__ __launch_bounds__(kBlockGrad) void mlp_fwd_grad_kernel(MLPKArgs a) {
-  constexpr int NT = 1, kBlockPts = 16 * NT * (kBlockGrad / 64);
+// F = -grad Phi (mlp_tile_grad).  A wave takes `per` 16-point tiles (1 or 4) at a
+// time: the features and the force of the base model, a fifth of the vector work
+// when every lane group of a tile repeats them, are then evaluated one point per
+// lane, and the tiles' features and results pass through the lanes.
+__global__ __launch_bounds__(kBlockGrad) void mlp_fwd_grad_kernel(MLPKArgs a, int per) {
+  constexpr int NT = 1;
   extern __shared__ __align__(16) unsigned char smem[];
   __bf16* sW = reinterpret_cast<__bf16*>(smem);
   float* sS = reinterpret_cast<float*>(smem + kLdsWBytes);
@@ -464,19 +491,30 @@ __global__ __launch_bounds__(kBlockGrad) void mlp_fwd_grad_kernel(MLPKArgs a) {
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int g = lane >> 4, c = lane & 15;
-  const int64_t ntiles = (a.n + kBlockPts - 1) / kBlockPts;
-  for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int64_t p = tile * kBlockPts + wave * 16 * NT + c;
-    const bool valid = p < a.n;
-    const int64_t q = valid ? p : 0;
+  const int pts = 16 * per;            // points of a wave
+  for (int64_t base = ((int64_t)blockIdx.x * (kBlockGrad / 64) + wave) * pts; base < a.n;
+       base += (int64_t)gridDim.x * (kBlockGrad / 64) * pts) {
+    const int64_t p = base + lane;
+    const bool valid = lane < pts && p < a.n;
+    const int64_t q = valid ? p : base;
     const float x = a.x[q], y = a.y[q], z = a.z[q];
-    float f[NT][3];
-    mlp_features(a.cfg, x, y, z, f[0]);
-    float y0[NT], dy[NT][3];
-    mlp_tile_grad<NT>(sW, sS, f, y0, dy, g, c);
-    if (valid && g == 0) {
+    float fl[3], y0 = 0.f, dy[3] = {0.f, 0.f, 0.f};
+    mlp_features(a.cfg, x, y, z, fl);
+#pragma unroll 1
+    for (int t = 0; t < per; ++t) {
+      float f[NT][3], yt[NT], dt[NT][3];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) f[0][k] = __shfl(fl[k], 16 * t + c, 64);
+      mlp_tile_grad<NT>(sW, sS, f, yt, dt, g, c);
+      if (g == t) {   // all four lane groups hold the tile's results
+        y0 = yt[0];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) dy[k] = dt[0][k];
+      }
+    }
+    if (valid) {
       float fx, fy, fz, pot;
-      conservative_field(a.cfg, x, y, z, y0[0], dy[0], fx, fy, fz, pot);
+      conservative_field(a.cfg, x, y, z, y0, dy, fx, fy, fz, pot);
       const float R = sqrtf(x * x + y * y);
       const float cp = R > 0.f ? x / R : 1.f, sp = R > 0.f ? y / R : 0.f;
       a.out[p] = pot;
@@ -1034,10 +1072,10 @@ __device__ __forceinline__ void surrogate_accel(const MLPLeapArgs& a, FieldTable
 }
 
 template <bool GRAD>
-__global__ __launch_bounds__(GRAD ? kBlockGrad : kBlockInf) void mlp_leapfrog_kernel(MLPLeapArgs a) {
+__global__ __launch_bounds__(GRAD ? kBlockGradStep : kBlockInf) void mlp_leapfrog_kernel(MLPLeapArgs a) {
   // GRAD: conservative forces from mlp_tile_grad, 16-point tiles
   constexpr int NT = GRAD ? 1 : kNT;
-  constexpr int kBlock = GRAD ? kBlockGrad : kBlockInf, kBlockPts = 16 * NT * (kBlock / 64);
+  constexpr int kBlock = GRAD ? kBlockGradStep : kBlockInf, kBlockPts = 16 * NT * (kBlock / 64);
   extern __shared__ __align__(16) unsigned char smem[];
   __bf16* sW = reinterpret_cast<__bf16*>(smem);
   float* sS = reinterpret_cast<float*>(smem + kLdsWBytes);
@@ -1409,9 +1447,12 @@ extern "C" int bfe_mlp_forward(bfe_ctx* h, const float* x, const float* y, const
   MLPKArgs a = base_args(c);
   a.x = x; a.y = y; a.z = z; a.n = n; a.out = out;
   if (c->mlp.conservative) {
-    const int64_t ntiles = (n + 16 * (kBlockGrad / 64) - 1) / (16 * (kBlockGrad / 64));
-    const int nb = (int)(ntiles < 2048 ? ntiles : 2048);
-    hipLaunchKernelGGL(mlp_fwd_grad_kernel, dim3(nb), dim3(kBlockGrad), kLdsBytes, s, a);
+    // four tiles a wave once every wave of the device has them
+    constexpr int kWaves = kBlockGrad / 64;
+    const int per = n > (int64_t)kGradBlocks * kWaves * 16 ? 4 : 1;
+    const int64_t blocks = (n + 16 * per * kWaves - 1) / (16 * per * kWaves);
+    const int nb = (int)(blocks < kGradBlocks ? blocks : kGradBlocks);
+    hipLaunchKernelGGL(mlp_fwd_grad_kernel, dim3(nb), dim3(kBlockGrad), kLdsBytes, s, a, per);
     BFE_HIP(c, hipGetLastError());
     return 0;
   }
@@ -1506,7 +1547,7 @@ extern "C" int bfe_mlp_leapfrog(bfe_ctx* h, float* x, float* y, float* z, float*
   a.partE = energy_log ? partE : nullptr;
   a.check_index = 0;
   if (a.cfg.conservative)
-    hipLaunchKernelGGL(mlp_leapfrog_kernel<true>, dim3(nb), dim3(kBlockGrad), kLdsBytes, s, a);
+    hipLaunchKernelGGL(mlp_leapfrog_kernel<true>, dim3(nb), dim3(kBlockGradStep), kLdsBytes, s, a);
   else
     hipLaunchKernelGGL(mlp_leapfrog_kernel<false>, dim3(nb), dim3(kBlockInf), kLdsBytes, s, a);
   BFE_HIP(c, hipGetLastError());
@@ -1518,7 +1559,7 @@ extern "C" int bfe_mlp_leapfrog(bfe_ctx* h, float* x, float* y, float* z, float*
     a.partE = (energy_log && a.energy_check) ? partE : nullptr;
     a.check_index = (int)ci + 1;
     if (a.cfg.conservative)
-    hipLaunchKernelGGL(mlp_leapfrog_kernel<true>, dim3(nb), dim3(kBlockGrad), kLdsBytes, s, a);
+    hipLaunchKernelGGL(mlp_leapfrog_kernel<true>, dim3(nb), dim3(kBlockGradStep), kLdsBytes, s, a);
   else
     hipLaunchKernelGGL(mlp_leapfrog_kernel<false>, dim3(nb), dim3(kBlockInf), kLdsBytes, s, a);
     BFE_HIP(c, hipGetLastError());
