@@ -822,6 +822,8 @@ __device__ __forceinline__ void sl_to_run(float (&A1)[PPT], float (&A2)[PPT], do
   }
 }
 
+constexpr int kWarmRuns = 16;   // cells of a 64-particle tile
+
 // Body of the cell-ordered SL accumulate; dsm is the block's dynamic LDS.
 // LM > 0: g.lmax == LM, known at compile time; LM = 0: any lmax.
 template <int PPT, int CH, int LM>
@@ -884,6 +886,15 @@ __device__ __forceinline__ void sl_deposit_body(
         const SLCell cell = sl_locate(r, g.cmap, g.scale, g.xi, g.numr, g.idxi, g.xi0, g.xin);
         const double P0 = cell.x1 * g.p0[cell.i] + cell.x2 * g.p0[cell.i + 1];
         ci = cell.i;
+        // a tile of many cells waits for two table rows at each: touch them all
+        // at once here (100 000 particles at lmax 4, nmax 10, whose outer tiles
+        // set the time: 32 -> 28 us)
+        if (__popcll(__ballot(live && ci != __shfl_up(ci, 1))) >= kWarmRuns) {
+          float warm = 0.f;
+          for (int l = 0; l <= g.lmax; ++l)
+            warm += E[(size_t)ci * rowlen + l * rp] + E[(size_t)(ci + 1) * rowlen + l * rp];
+          asm volatile("" ::"v"(warm));
+        }
         w1 = live ? (float)(cell.x1 * P0) : 0.f;
         w2 = live ? (float)(cell.x2 * P0) : 0.f;
         const int pad = (lane >> 2) * kDepStride + (lane & 3);
