@@ -173,7 +173,7 @@ struct Context {
 
   // ---- a second set of work buffers and an internal stream, for the two
   // independent halves of a call that runs them concurrently (disc and
-  // halo accumulate, EOF and SL folds); see fork_begin / fork_end
+  // halo accumulate and fold); see fork_begin / fork_end
   void* alt_scratch = nullptr;
   size_t alt_scratch_bytes = 0;
   void* alt_order = nullptr;

@@ -60,9 +60,15 @@ constexpr int kWaveTile = 16 * kNT;              // points per wave
 constexpr int kBlockInf = BFE_MLP_BLOCK;
 constexpr int kInfPts = kWaveTile * kBlockInf / 64;   // points per block
 // The conservative-field kernels carry three tangent operand sets beside the
-// activations: four waves per block, one per SIMD, keep them in registers.
+// activations (192 registers).  Inference: eight waves per block, two per SIMD
+// without spills, so that one wave's activations cover the other's products
+// (1M points 667 -> 458 us against four waves; 422 with the point work once per
+// point).  The integrator holds its state as well and spills 500 B a lane that
+// way: four waves, one per SIMD.
 constexpr int kBlockGrad = 512;
 constexpr int kBlockGradStep = 256;
+// Blocks of the inference kernel: one per CU loads the weights (104 KB) once
+// (523 us under the profiler, 537 with 2 048 blocks).
 constexpr int kGradBlocks = 256;
 // LDS copy of the three hidden weight matrices: rows of kH bf16 padded to
 // kLdsRow.  A lane reads 16 bytes of row 16 mt + c; unpadded (256-byte)
