@@ -60,13 +60,12 @@ constexpr int kWaveTile = 16 * kNT;              // points per wave
 constexpr int kBlockInf = BFE_MLP_BLOCK;
 constexpr int kInfPts = kWaveTile * kBlockInf / 64;   // points per block
 // The conservative-field kernels carry three tangent operand sets beside the
-// activations (192 registers).  Inference: eight waves per block, two per SIMD
-// without spills, so that one wave's activations cover the other's products
-// (1M points 667 -> 458 us against four waves; 422 with the point work once per
-// point).  The integrator holds its state as well and spills 500 B a lane that
-// way: four waves, one per SIMD.
+// activations (192 registers): eight waves per block, two per SIMD, so that one
+// wave's activations cover the other's products.  Inference of 1M points 667 ->
+// 458 us against four waves (no spills; 422 with the point work once per point);
+// the integrator, which holds its state as well and spills 500 B a lane, 55.7 ->
+// 37.5 ms per 100 steps of 1M orbits.
 constexpr int kBlockGrad = 512;
-constexpr int kBlockGradStep = 256;
 // Blocks of the inference kernel: one per CU loads the weights (104 KB) once
 // (523 us under the profiler, 537 with 2 048 blocks).
 constexpr int kGradBlocks = 256;
@@ -1078,10 +1077,10 @@ __device__ __forceinline__ void surrogate_accel(const MLPLeapArgs& a, FieldTable
 }
 
 template <bool GRAD>
-__global__ __launch_bounds__(GRAD ? kBlockGradStep : kBlockInf) void mlp_leapfrog_kernel(MLPLeapArgs a) {
+__global__ __launch_bounds__(GRAD ? kBlockGrad : kBlockInf) void mlp_leapfrog_kernel(MLPLeapArgs a) {
   // GRAD: conservative forces from mlp_tile_grad, 16-point tiles
   constexpr int NT = GRAD ? 1 : kNT;
-  constexpr int kBlock = GRAD ? kBlockGradStep : kBlockInf, kBlockPts = 16 * NT * (kBlock / 64);
+  constexpr int kBlock = GRAD ? kBlockGrad : kBlockInf, kBlockPts = 16 * NT * (kBlock / 64);
   extern __shared__ __align__(16) unsigned char smem[];
   __bf16* sW = reinterpret_cast<__bf16*>(smem);
   float* sS = reinterpret_cast<float*>(smem + kLdsWBytes);
@@ -1553,7 +1552,7 @@ extern "C" int bfe_mlp_leapfrog(bfe_ctx* h, float* x, float* y, float* z, float*
   a.partE = energy_log ? partE : nullptr;
   a.check_index = 0;
   if (a.cfg.conservative)
-    hipLaunchKernelGGL(mlp_leapfrog_kernel<true>, dim3(nb), dim3(kBlockGradStep), kLdsBytes, s, a);
+    hipLaunchKernelGGL(mlp_leapfrog_kernel<true>, dim3(nb), dim3(kBlockGrad), kLdsBytes, s, a);
   else
     hipLaunchKernelGGL(mlp_leapfrog_kernel<false>, dim3(nb), dim3(kBlockInf), kLdsBytes, s, a);
   BFE_HIP(c, hipGetLastError());
@@ -1565,7 +1564,7 @@ extern "C" int bfe_mlp_leapfrog(bfe_ctx* h, float* x, float* y, float* z, float*
     a.partE = (energy_log && a.energy_check) ? partE : nullptr;
     a.check_index = (int)ci + 1;
     if (a.cfg.conservative)
-    hipLaunchKernelGGL(mlp_leapfrog_kernel<true>, dim3(nb), dim3(kBlockGradStep), kLdsBytes, s, a);
+    hipLaunchKernelGGL(mlp_leapfrog_kernel<true>, dim3(nb), dim3(kBlockGrad), kLdsBytes, s, a);
   else
     hipLaunchKernelGGL(mlp_leapfrog_kernel<false>, dim3(nb), dim3(kBlockInf), kLdsBytes, s, a);
     BFE_HIP(c, hipGetLastError());
