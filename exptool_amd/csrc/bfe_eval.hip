@@ -5,6 +5,7 @@
 #include <vector>
 
 #include "bfe_field.hpp"
+#include "bfe_rules.hpp"
 
 namespace bfe {
 
@@ -642,9 +643,12 @@ __global__ __launch_bounds__(256) void eof_points_kernel(
 // nodes: when their force blocks fit in kStageFloat4, the block copies them
 // to LDS and the SL sums read them there.  pts2 (may be NULL): a second set of n2
 // points in its own cell order, numbered after the first.  Bound by vector ALU
-// issue (77 % busy) and address units (71 %); four waves a SIMD (128 registers,
-// 20 B spilled) 149 us for 2M points, three 155.
-__global__ __launch_bounds__(256, 4) void field_eval_kernel(
+// issue (77 % busy) and address units (71 %) where the chip is full: 2M points 149
+// us with WAVES = 4 a SIMD (128 registers, 20 B spilled), 155 with three (144);
+// fewer points by one wave's own latency, where three are faster
+// (eval_four_waves).
+template <int WAVES>
+__global__ __launch_bounds__(256, WAVES) void field_eval_kernel(
     const float* __restrict__ px, const float* __restrict__ py, const float* __restrict__ pz,
     int64_t n, const float4* __restrict__ pts, const float4* __restrict__ pts2, int64_t n2,
     FieldTables T, float* fx, float* fy, float* fz, float* pot, float* comp,
@@ -1042,8 +1046,12 @@ static int field_eval_run(Context* c, const FieldTables& T, const float* x, cons
   const unsigned grid = pts2 ? xcd_grid(nblocks256(n1)) + xcd_grid(nblocks256(n - n1))
                         : pts ? xcd_grid(nblocks256(n)) : nblocks256(n);
   timer_begin(c, "field_eval", s);
-  hipLaunchKernelGGL(field_eval_kernel, dim3(grid), dim3(256), 0, s, x, y, z, pts2 ? n1 : n, pts, pts2,
-                     n - n1, T, fx, fy, fz, pot, comp, quad, n);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, s, x, y, z, pts2 ? n1 : n, pts, pts2, n - n1, T,
+                       fx, fy, fz, pot, comp, quad, n);
+  };
+  if (eval_four_waves(n)) go(field_eval_kernel<4>);
+  else go(field_eval_kernel<3>);
   timer_end(c, "field_eval", s);
   BFE_HIP(c, hipGetLastError());
   if (quad) {
