@@ -5,7 +5,6 @@
 #include <vector>
 
 #include "bfe_field.hpp"
-#include "bfe_rules.hpp"
 
 namespace bfe {
 
@@ -1071,7 +1070,7 @@ static int field_eval_split_run(Context* c, const FieldTables& T, const float* x
   const unsigned grid = (unsigned)((n + kSplitPts - 1) / kSplitPts);
   const size_t lds = (size_t)split_lds_doubles(c->mmax, c->lmax) * sizeof(double);
   timer_begin(c, "field_eval", s);
-  if (c->lmax == 6 && c->mmax == 6)
+  if (split_fixed(c->lmax, c->mmax))
     hipLaunchKernelGGL((field_eval_split_kernel<6, 6>), dim3(grid), dim3(kSplitThreads), lds, s, x, y,
                        z, n1, x2, y2, z2, n, T, fx, fy, fz, pot, comp);
   else

@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "bfe_math.hpp"
+#include "bfe_rules.hpp"
 #include "../../include/exptool_bfe.h"
 
 namespace bfe {
@@ -160,7 +161,7 @@ struct Context {
   int64_t sl_seg_tiles = 0;
   int64_t order_min = 65536;       // accumulate in cell order from this many particles,
                                    // evaluate in it from twice as many points
-  int64_t split_max = 36864;       // orbits up to which the split integrators run
+  int64_t split_max = kSplitMax;   // orbits up to which the split integrators run (split_orbits_max)
   int64_t split_eval_max = 131072; // points up to which the split evaluation runs
   int64_t point_blocks = 512;      // points up to which the point evaluators fold only their cells
   int64_t sl_acc_path = 0;         // SL accumulate: 0 auto (vector ALU), 1 MFMA, 2 vector ALU

@@ -185,9 +185,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void l
 
 // The same steps with the field evaluated by split blocks (field_eval_split:
 // 64 orbits, eight waves sharing the orders) for orbit counts that leave the
-// one-lane kernel latency-bound (up to split_max: one orbit 7.9 -> 2.8 us a
-// step, 12 800 orbits 14.6 -> 4.5, 36k orbits 12.4 and 12.4; RK4 of 20 000
-// orbits 15.5 -> 8.4 us an evaluation).  A block's eight waves fill a CU at
+// one-lane kernel latency-bound (split_orbits_max; at lmax = mmax = 6 one orbit
+// 6.9 -> 3.0 us a step, 12 800 orbits 13 -> 4.8, 36 864 orbits 12.7 -> 11.1; RK4
+// of 20 000 orbits 15.5 -> 7.0 us an evaluation).  A block's eight waves fill a CU at
 // 156 registers; at four waves per SIMD (128, 120 B spilled) one orbit took
 // 3.3 us.  Every wave carries the state of the block's
 // orbits and advances it alike; wave w writes component w of the records.
@@ -528,7 +528,7 @@ static int leapfrog_run(bfe_ctx* h, float* x, float* y, float* z, float* vx, flo
   BFE_HIP(c, hipSetDevice(c->device));
   hipStream_t s = (hipStream_t)stream;
   const int nb = (int)((n + 255) / 256);
-  const bool split = n <= c->split_max && split_ok(T);
+  const bool split = n <= split_orbits_max(c->split_max, c->lmax, c->mmax, false) && split_ok(T);
   const int64_t plain = split ? kSplitChunkSteps : 100;
   const int chunk = energy_every > 0 ? energy_every : (int)std::min<int64_t>(nsteps > 0 ? nsteps : 1, plain);
   const int nchecks = energy_every > 0 ? (int)(nsteps / energy_every) + 1 : 1;
@@ -572,7 +572,7 @@ static int leapfrog_run(bfe_ctx* h, float* x, float* y, float* z, float* vx, flo
       hipLaunchKernelGGL(kernel, dim3(grid), dim3(kSplitThreads), slds, s, x, y, z, vx, vy, vz, perm,
                          T, b, init, aux, eb, traj);
     };
-    const bool fixed = c->lmax == 6 && c->mmax == 6;
+    const bool fixed = split_fixed(c->lmax, c->mmax);
     if (dtv && fixed) go(leapfrog_split_kernel<true, 6, 6>);
     else if (dtv) go(leapfrog_split_kernel<true, -1, -1>);
     else if (fixed) go(leapfrog_split_kernel<false, 6, 6>);
@@ -687,7 +687,7 @@ extern "C" int bfe_rk4(bfe_ctx* h, float* x, float* y, float* z, float* vx, floa
   if (n == 0) return 0;
   BFE_HIP(c, hipSetDevice(c->device));
   hipStream_t s = (hipStream_t)stream;
-  const bool split = n <= c->split_max && split_ok(T);
+  const bool split = n <= split_orbits_max(c->split_max, c->lmax, c->mmax, true) && split_ok(T);
   const bool ordered = !split || n >= kSplitOrderMin;
   const int nb = (int)((n + 255) / 256);
   const int sb = (int)((n + kSplitPts - 1) / kSplitPts);
@@ -712,7 +712,7 @@ extern "C" int bfe_rk4(bfe_ctx* h, float* x, float* y, float* z, float* vx, floa
     }
     a.k0 = k0;
     a.k1 = std::min<int64_t>(nsteps, k0 + chunk);
-    if (split && c->lmax == 6 && c->mmax == 6)
+    if (split && split_fixed(c->lmax, c->mmax))
       hipLaunchKernelGGL((rk4_split_kernel<6, 6>), dim3(grid), dim3(kSplitThreads), slds, s, x, y, z,
                          vx, vy, vz, perm, T, a, traj);
     else if (split)

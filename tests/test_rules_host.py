@@ -19,6 +19,8 @@ int main() {
   long long a[6];
   while (std::scanf("%63s %lld %lld %lld %lld %lld %lld", f, a, a + 1, a + 2, a + 3, a + 4, a + 5) == 7) {
     if (!std::strcmp(f, "eval_four_waves")) std::printf("%d\n", (int)bfe::eval_four_waves(a[0]));
+    else if (!std::strcmp(f, "split_orbits_max"))
+      std::printf("%lld\n", (long long)bfe::split_orbits_max(a[0], a[1], a[2], a[3] != 0));
     else return 1;
   }
   return 0;
@@ -50,3 +52,30 @@ def test_four_waves_only_where_the_chip_is_full(rule):
     ns = [1, 256, 65_536, 131_072, 196_608, 262_144, 500_000, 1_000_000, 2_000_000]
     got = [bool(v[0]) for v in rule("eval_four_waves", [(n,) for n in ns])]
     assert got == [False] * 7 + [True] * 2
+
+
+# us of the one-lane and the split integrators on MI355X at (lmax, mmax), orbits
+LEAPFROG = [((0, 0), 16_384, 321, 342), ((0, 0), 32_768, 303, 614), ((2, 2), 16_384, 552, 436),
+            ((2, 2), 16_385, 555, 742), ((2, 2), 32_768, 578, 779), ((3, 3), 24_000, 762, 965),
+            ((4, 4), 16_384, 833, 514), ((4, 4), 32_768, 814, 909), ((4, 4), 36_864, 812, 1285),
+            ((4, 6), 32_768, 909, 905), ((4, 6), 36_864, 908, 1315), ((4, 8), 24_000, 1000, 939),
+            ((4, 8), 32_769, 1007, 1320), ((6, 0), 32_768, 1006, 859), ((6, 4), 24_000, 1136, 1029),
+            ((6, 4), 36_864, 1167, 1485), ((6, 6), 32_768, 1279, 804), ((6, 6), 36_864, 1274, 1112),
+            ((8, 8), 32_768, 1629, 1312), ((8, 8), 36_864, 1614, 1905), ((10, 6), 16_384, 1927, 854),
+            ((10, 6), 36_864, 1903, 2260), ((12, 12), 32_768, 2812, 1928)]
+RK4 = [((2, 2), 16_384, 603, 418), ((2, 2), 24_000, 576, 747), ((3, 3), 32_768, 876, 956),
+       ((2, 6), 32_768, 776, 838), ((4, 2), 32_768, 860, 820), ((4, 4), 24_000, 937, 869),
+       ((4, 4), 36_864, 949, 1262), ((5, 5), 32_768, 1233, 986), ((5, 5), 36_864, 1229, 1391),
+       ((6, 0), 36_864, 1254, 1164), ((6, 6), 36_864, 1535, 1076), ((8, 8), 36_864, 2069, 1896),
+       ((10, 6), 36_864, 2603, 2276), ((12, 12), 36_864, 3805, 2796)]
+
+
+def test_split_orbits_where_they_are_the_faster(rule):
+    """At its default the limit takes, of the two forms, the one measured faster
+    (within 8 %: the table's own spread, and the fixed cost at the smallest
+    basis), for every basis; any other value is the limit."""
+    for rk4, table in ((0, LEAPFROG), (1, RK4)):
+        lim = rule("split_orbits_max", [(36_864, *b, rk4) for b, *_ in table])
+        for (basis, n, one, split), (m,) in zip(table, lim):
+            assert (split if n <= m else one) <= 1.08 * min(one, split), (rk4, basis, n, m)
+    assert rule("split_orbits_max", [(0, 4, 4, 0), (1 << 40, 2, 2, 1), (5000, 10, 6, 0)]) == [[0], [1 << 40], [5000]]
