@@ -1108,14 +1108,11 @@ extern "C" int bfe_field_eval_cart(bfe_ctx* h, const float* x, const float* y, c
   if (n == 0) return 0;
   BFE_HIP(c, hipSetDevice(c->device));
   hipStream_t s = (hipStream_t)stream;
-  // 40k unordered points: 14 us by split blocks against 17 one lane a point;
-  // from about 131k points the sort pays (200k: 68 us ordered with the sort,
-  // 74 split, 82 one lane a point in input order)
-  const bool ordered = n / 2 >= c->order_min;
-  if (!ordered && n <= c->split_eval_max && split_ok(T))
+  const EvalForm form = eval_form(n, c->lmax, c->mmax, split_ok(T), c->order_min, c->split_eval_max);
+  if (form == kEvalSplit)
     return field_eval_split_run(c, T, x, y, z, n, x, y, z, n, fx, fy, fz, pot, comp, s);
   const float4* pts = nullptr;
-  if (ordered) {
+  if (form == kEvalOrdered) {
     rc = order_points(c, T, x, y, z, n, s, nullptr, nullptr, 1, nullptr, &pts);
     if (rc) return rc;
   }
@@ -1166,7 +1163,7 @@ extern "C" int bfe_forces_disc_halo(bfe_ctx* h, const float* dx, const float* dy
   G.eg = eof_geom(c);
   G.lmax = c->lmax;
   G.flags = field_flags & (BFE_COMPAT_SL_COS_L | BFE_COMPAT_SL_EDGE);
-  const bool split = n / 2 < c->order_min && n <= c->split_eval_max && split_ok(G);
+  const bool split = eval_split_two(n, c->lmax, c->mmax, split_ok(G), c->order_min, c->split_eval_max);
   if (done) {
     rc = field_set_run(c, cos_out, sin_out, coef_out, halofac, disk_m, disk_n, halo_l, halo_n,
                        field_flags, s);

@@ -159,10 +159,10 @@ struct Context {
   int64_t sl_acc_blocks_beside = 1024;
   int64_t eof_seg_tiles = 0;       // batch accumulate: tiles per segment, 0 = from the budget
   int64_t sl_seg_tiles = 0;
-  int64_t order_min = 65536;       // accumulate in cell order from this many particles,
-                                   // evaluate in it from twice as many points
+  int64_t order_min = 65536;       // accumulate in cell order from this many particles; the
+                                   // evaluation's line follows it (eval_form)
   int64_t split_max = kSplitMax;   // orbits up to which the split integrators run (split_orbits_max)
-  int64_t split_eval_max = 131072; // points up to which the split evaluation runs
+  int64_t split_eval_max = kSplitEvalMax;   // points up to which the split evaluation does (eval_form)
   int64_t point_blocks = 512;      // points up to which the point evaluators fold only their cells
   int64_t sl_acc_path = 0;         // SL accumulate: 0 auto (vector ALU), 1 MFMA, 2 vector ALU
   int64_t eof_dep_shape = -1;      // cell-ordered EOF accumulate lane shape (index), -1 auto

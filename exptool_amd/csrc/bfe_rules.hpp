@@ -43,4 +43,54 @@ inline int64_t split_orbits_max(int64_t knob, int lmax, int mmax, bool rk4) {
   return terms >= (rk4 ? 15 : 21) ? 32768 : 16384;
 }
 
+// The form of a field evaluation of n points: one lane a point in input order,
+// split blocks (64 points a block of eight waves) or one lane a point in cell order
+// (sorted first).
+//
+// One lane in input order is flat up to 65 536 points (a block of 256 a CU), then
+// doubles.  The sort costs about 25 us, so it pays from the second round on where a
+// point has many terms, from the third otherwise.  Split blocks cost with every
+// round of theirs and win while one lane's latency is longer.  us in input order /
+// split / cell order at (lmax, mmax) and points:
+//   (2, 2)    16 384  7.7 / 10.1 / 29    65 536  9.0 / 32 / 31    131 072  14 / 57 / 36
+//   (4, 4)    8 192 10.2 / 9.8 / 32    16 384 10.4 / 11.4 / 32    65 536 13 / 36 / 33
+//             131 072  25 / 66 / 39
+//   (4, 8)    16 384 14.2 / 13.7 / 34    24 576 17 / 23 / 34    131 072 42 / 76 / 46
+//   (6, 6)    49 152  22 / 20.5 / 37    65 536  22.6 / 26.6 / 37    98 304 42 / 38 / 42
+//             131 072  44 / 49 / 43
+//   (8, 8)    32 768  33 / 29 / 40    65 536  33 / 52 / 41    80 000  60 / 63 / 48
+//   (10, 6)   32 768  33 / 31 / 41    65 536  33 / 54 / 41    100 000  63 / 77 / 49
+//   (12, 12)  32 768  48 / 40 / 52    65 536  48 / 72 / 58    100 000  102 / 104 / 69
+//   without split blocks (cos(l phi)): (4, 4) 100 000 23 / - / 39, (6, 6) 42 / - / 45,
+//   (10, 6) 62 / - / 58, (12, 12) 106 / - / 92
+// (6, 6) is the split kernels' instance with its orders at compile time.
+// At any other value than its default split_knob takes split blocks for every
+// unordered call up to it.
+enum EvalForm { kEvalInput = 0, kEvalSplit = 1, kEvalOrdered = 2 };
+constexpr int64_t kSplitEvalMax = 131072;
+constexpr int64_t kEvalRound = 65536;
+inline EvalForm eval_form(int64_t n, int lmax, int mmax, bool split_ok, int64_t order_min,
+                          int64_t split_knob) {
+  const int terms = field_terms(lmax, mmax);
+  const bool explicit_max = split_knob != kSplitEvalMax;
+  if (!explicit_max && terms >= 45 ? n > order_min : n / 2 >= order_min) return kEvalOrdered;
+  int64_t most = split_knob;
+  if (!explicit_max) {
+    if (split_fixed(lmax, mmax)) most = n <= kEvalRound ? 49152 : 98304;
+    else most = terms >= 45 ? 32768 : terms >= 20 ? 16384 : 0;
+  }
+  return split_ok && n <= most ? kEvalSplit : kEvalInput;
+}
+// Whether the n points of two inputs are evaluated by split blocks or else ordered
+// together (they have no one-lane form in input order): split / cell order at
+// 49 152 | 57 344 points (0, 0) 20 / 28 | 25 / 28, (4, 4) 28 / 33 | 35 / 33, (6, 4) 31 /
+// 36 | 39 / 36, (10, 6) 43 / 43 | 53 / 44, (12, 12) 57 / 63 | 71 / 62; (6, 6) at 114 688
+// 44 / 46.
+inline bool eval_split_two(int64_t n, int lmax, int mmax, bool split_ok, int64_t order_min,
+                           int64_t split_knob) {
+  if (!split_ok || n / 2 >= order_min) return false;
+  if (split_knob != kSplitEvalMax) return n <= split_knob;
+  return n <= (split_fixed(lmax, mmax) ? 114688 : 49152);
+}
+
 }  // namespace bfe

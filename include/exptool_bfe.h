@@ -291,11 +291,11 @@ int bfe_field_eval_batch(bfe_ctx* ctx, const float* x, const float* y, const flo
  * (lane shape of the cell-ordered accumulate kernels, -1 = automatic; a
  * shape that does not fit the tables falls back to the automatic one),
  * "order_min" (particles from which the accumulates run in table-cell order,
- * and half the points from which evaluation does, 65536), "split_max" and
- * "split_eval_max" (orbits, unordered points up to which the field is
- * evaluated by split blocks, several waves per 64 points; 36864, 131072; at that
- * default "split_max" is lmax = mmax = 6's limit and other bases take their own,
- * any other value holds for every basis),
+ * 65536; evaluations from the next point on where a point has many terms, else
+ * from twice as many), "split_max" and "split_eval_max" (orbits, unordered
+ * points up to which the field is evaluated by split blocks, several waves per
+ * 64 points; 36864, 131072: at these defaults the limits follow the basis, any
+ * other value holds for every basis),
  * "point_blocks" (points up to which bfe_sl_eval_sph and bfe_eof_eval_cyl fold
  * only the points' own cells; 512).
  * Evaluation and orbits do not depend on these; accumulate sums depend on

@@ -21,6 +21,10 @@ int main() {
     if (!std::strcmp(f, "eval_four_waves")) std::printf("%d\n", (int)bfe::eval_four_waves(a[0]));
     else if (!std::strcmp(f, "split_orbits_max"))
       std::printf("%lld\n", (long long)bfe::split_orbits_max(a[0], a[1], a[2], a[3] != 0));
+    else if (!std::strcmp(f, "eval_form"))
+      std::printf("%d\n", (int)bfe::eval_form(a[0], a[1], a[2], a[3] != 0, a[4], a[5]));
+    else if (!std::strcmp(f, "eval_split_two"))
+      std::printf("%d\n", (int)bfe::eval_split_two(a[0], a[1], a[2], a[3] != 0, a[4], a[5]));
     else return 1;
   }
   return 0;
@@ -38,7 +42,7 @@ def rule(tmp_path_factory):
 
     def ask(name, calls):
         """The rule's answers (lists of integers) to a list of argument tuples."""
-        text = "\n".join(" ".join([name] + [str(v) for v in c] + ["0"] * (6 - len(c))) for c in calls)
+        text = "\n".join(" ".join([name] + [str(int(v)) for v in c] + ["0"] * (6 - len(c))) for c in calls)
         r = subprocess.run([exe], input=text + "\n", capture_output=True, text=True, check=True)
         out = [[int(v) for v in line.split()] for line in r.stdout.splitlines()]
         assert len(out) == len(calls)
@@ -79,3 +83,46 @@ def test_split_orbits_where_they_are_the_faster(rule):
         for (basis, n, one, split), (m,) in zip(table, lim):
             assert (split if n <= m else one) <= 1.08 * min(one, split), (rk4, basis, n, m)
     assert rule("split_orbits_max", [(0, 4, 4, 0), (1 << 40, 2, 2, 1), (5000, 10, 6, 0)]) == [[0], [1 << 40], [5000]]
+
+
+# us of an evaluation on MI355X in input order, by split blocks (None: not taken by
+# them, cos(l phi)) and in cell order at (lmax, mmax), points
+EVALUATION = [((0, 0), 1000, 5.0, 7.4, 26), ((0, 0), 131_000, 6.6, 45, 33), ((2, 2), 16_384, 7.7, 10.1, 29),
+              ((2, 2), 65_536, 9.0, 32, 31), ((4, 4), 16_384, 10.4, 11.4, 32), ((4, 4), 40_000, 11.7, 27, 33),
+              ((4, 4), 65_536, 13, 36, 33), ((4, 4), 100_000, 23, 51, 37), ((4, 4), 131_071, 25, 66, 39),
+              ((4, 8), 4096, 12.9, 9.7, 34), ((4, 8), 24_576, 16.7, 22.5, 34), ((4, 8), 98_304, 41, 59, 45),
+              ((6, 4), 8192, 15, 10.9, 36), ((6, 4), 32_768, 17.7, 22.6, 36), ((6, 4), 131_071, 36, 73, 42),
+              ((6, 6), 16_384, 16.7, 8.6, 37), ((6, 6), 49_152, 22, 20.5, 37), ((6, 6), 65_536, 22.6, 26.6, 37),
+              ((6, 6), 80_000, 42, 32, 39), ((6, 6), 131_071, 44, 49, 43), ((8, 8), 16_384, 28, 18.7, 40),
+              ((8, 8), 65_536, 31, 52, 41), ((8, 8), 98_304, 59, 73, 51), ((8, 8), 131_071, 59, 95, 57),
+              ((10, 6), 16_384, 32, 20, 42), ((10, 6), 40_000, 33, 42, 43), ((10, 6), 65_536, 33, 54, 41),
+              ((10, 6), 100_000, 63, 77, 49), ((12, 12), 20_000, 48, 39, 54), ((12, 12), 49_152, 48, 57, 58),
+              ((12, 12), 80_000, 104, 88, 69), ((12, 12), 131_071, 98, 137, 69),
+              ((4, 4), 100_000, 22.6, None, 39), ((6, 6), 65_536, 25.2, None, 40), ((6, 6), 131_071, 42.5, None, 47),
+              ((10, 6), 65_536, 45, None, 53), ((10, 6), 100_000, 62, None, 58), ((12, 12), 65_536, 72, None, 76),
+              ((12, 12), 100_000, 104, None, 90)]
+TWO_INPUTS = [((0, 0), 49_152, 20.5, 28.2), ((2, 2), 80_000, 38, 32.5), ((4, 4), 49_152, 28, 33), ((4, 4), 57_344, 35, 33),
+              ((4, 4), 131_071, 66, 39), ((6, 4), 65_536, 40, 36.5), ((6, 6), 65_536, 26.6, 37), ((6, 6), 114_688, 44, 46),
+              ((6, 6), 131_071, 49, 43), ((10, 6), 40_000, 42, 43), ((10, 6), 65_536, 54, 41), ((12, 12), 130_000, 136, 69)]
+
+
+def test_evaluation_takes_the_fastest_form(rule):
+    """At the default limits the form taken is the one measured fastest, within
+    10 % (the spread of the figures and the steps of the limits)."""
+    got = rule("eval_form", [(n, *b, s is not None, 65_536, 131_072) for b, n, _, s, _ in EVALUATION])
+    for (basis, n, *us), (form,) in zip(EVALUATION, got):
+        assert us[form] is not None and us[form] <= 1.10 * min(u for u in us if u), (basis, n, form)
+    got = rule("eval_split_two", [(n, *b, 1, 65_536, 131_072) for b, n, _, _ in TWO_INPUTS])
+    for (basis, n, split, ordered), (yes,) in zip(TWO_INPUTS, got):
+        assert (split if yes else ordered) <= 1.10 * min(split, ordered), (basis, n, yes)
+
+
+def test_evaluation_form_follows_explicit_knobs(rule):
+    """Other values than the defaults hold for every basis: split up to the knob
+    where it can be, cell order from twice order_min points."""
+    calls = [(5000, 2, 2, 1, 1 << 40, 1 << 40), (5000, 2, 2, 0, 1 << 40, 1 << 40), (5000, 12, 12, 1, 1 << 40, 0),
+             (5000, 12, 12, 1, 1, 0), (1, 6, 6, 1, 1, 0), (131_071, 6, 6, 1, 65_536, 0), (131_072, 6, 6, 1, 65_536, 0)]
+    assert [v[0] for v in rule("eval_form", calls)] == [1, 0, 0, 2, 0, 0, 2]
+    calls = [(5000, 2, 2, 1, 1 << 40, 1 << 40), (5000, 2, 2, 0, 1 << 40, 1 << 40), (5000, 2, 2, 1, 1, 1 << 40),
+             (5000, 2, 2, 1, 1 << 40, 4999), (131_072, 6, 6, 1, 65_536, 131_072)]
+    assert [v[0] for v in rule("eval_split_two", calls)] == [1, 0, 0, 0, 0]
