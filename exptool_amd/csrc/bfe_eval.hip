@@ -1049,7 +1049,7 @@ static int field_eval_run(Context* c, const FieldTables& T, const float* x, cons
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, s, x, y, z, pts2 ? n1 : n, pts, pts2, n - n1, T,
                        fx, fy, fz, pot, comp, quad, n);
   };
-  if (eval_four_waves(n)) go(field_eval_kernel<4>);
+  if (eval_four_waves(n, (T.flags & BFE_COMPAT_SL_COS_L) != 0)) go(field_eval_kernel<4>);
   else go(field_eval_kernel<3>);
   timer_end(c, "field_eval", s);
   BFE_HIP(c, hipGetLastError());

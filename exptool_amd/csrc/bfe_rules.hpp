@@ -12,9 +12,13 @@ namespace bfe {
 // about eight blocks of 256 a CU.  Three / four, in cell order: 262 144 points
 // 63.5 / 65.8 us at lmax = mmax = 6 and 90.2 / 95.0 at 12, 500 000 90.0 / 91.6 and
 // 128.7 / 130.5, 800 000 115.6 / 113.9 and 173.7 / 168.3, 2M 218 / 214 and 342 /
-// 320; in input order 65 536 points 22.6 / 24.0 and 47.9 / 56.6.
-constexpr int64_t kEvalFourWaves = 524288;
-inline bool eval_four_waves(int64_t n) { return n >= kEvalFourWaves; }
+// 320; in input order 65 536 points 22.6 / 24.0 and 47.9 / 56.6.  With cos(l phi)
+// factors from three blocks a CU: 196 608 points on, (10, 6) 200 000 84.0 / 78.6, 500 000
+// 128 / 122; 65 536 52.7 / 51.3 and (12, 12) 75.6 / 78.4.
+constexpr int64_t kEvalFourWaves = 524288, kEvalFourWavesCosL = 196608;
+inline bool eval_four_waves(int64_t n, bool cos_l) {
+  return n >= (cos_l ? kEvalFourWavesCosL : kEvalFourWaves);
+}
 
 // Terms of one field evaluation: SL (l, m) pairs and EOF orders.
 inline int field_terms(int lmax, int mmax) { return (lmax + 1) * (lmax + 2) / 2 + mmax; }

@@ -18,7 +18,7 @@ int main() {
   char f[64];
   long long a[6];
   while (std::scanf("%63s %lld %lld %lld %lld %lld %lld", f, a, a + 1, a + 2, a + 3, a + 4, a + 5) == 7) {
-    if (!std::strcmp(f, "eval_four_waves")) std::printf("%d\n", (int)bfe::eval_four_waves(a[0]));
+    if (!std::strcmp(f, "eval_four_waves")) std::printf("%d\n", (int)bfe::eval_four_waves(a[0], a[1] != 0));
     else if (!std::strcmp(f, "split_orbits_max"))
       std::printf("%lld\n", (long long)bfe::split_orbits_max(a[0], a[1], a[2], a[3] != 0));
     else if (!std::strcmp(f, "eval_form"))
@@ -52,10 +52,13 @@ def rule(tmp_path_factory):
 
 def test_four_waves_only_where_the_chip_is_full(rule):
     """Up to three blocks of 256 points a CU (256 CUs) are resident with three
-    waves a SIMD, so the four-wave build has nothing to give there."""
+    waves a SIMD, so the four-wave build has nothing to give there; with
+    cos(l phi) factors it gives from there on, without from 524 288 points."""
     ns = [1, 256, 65_536, 131_072, 196_608, 262_144, 500_000, 1_000_000, 2_000_000]
     got = [bool(v[0]) for v in rule("eval_four_waves", [(n,) for n in ns])]
     assert got == [False] * 7 + [True] * 2
+    got = [bool(v[0]) for v in rule("eval_four_waves", [(n, 1) for n in ns])]
+    assert got == [False] * 4 + [True] * 5
 
 
 # us of the one-lane and the split integrators on MI355X at (lmax, mmax), orbits
