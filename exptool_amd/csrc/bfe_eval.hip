@@ -157,14 +157,18 @@ __global__ __launch_bounds__(256) void sl_fold_kernel(SLFoldIn f, SLFoldArgs a) 
 
 struct EOFFoldArgs {
   double mmul[kMaxM + 1];  // per-m multiplier (range / no_odd mask)
-  int nuse, dens;
+  int nuse;
   int numx, numy;          // grid, for the float64 edge blocks
 };
 
 // The float64 edge blocks of the folded field (after the float32 blocks of
 // each set): the m = 0 cos sums [pot, rforce, zforce, dens] of edge node e
 // (eof_edge_index) from its float64 fold inputs E[f][n][edge], as the float32
-// blocks sum them for m = 0.
+// blocks sum them for m = 0.  One serial chain of norder reads a lane, so the
+// reads of six orders go out together; with the density a test inside the loop
+// each order waited for its own (density fold at mmax 2, 257 x 129 nodes, 24.2 ->
+// 20.1 us).
+template <bool DENS>
 __device__ __forceinline__ void eof_fold_edge(const double* __restrict__ E, int64_t nedge,
                                               int64_t e, const double* __restrict__ cf, int mmax,
                                               int norder, const EOFFoldArgs& a,
@@ -174,8 +178,7 @@ __device__ __forceinline__ void eof_fold_edge(const double* __restrict__ E, int6
   for (int n = 0; n < a.nuse; ++n) {
     const double c = cf[n];
 #pragma unroll
-    for (int f = 0; f < 4; ++f)
-      if (f < 3 || a.dens) s[f] += c * E[((size_t)f * norder + n) * nedge + e];
+    for (int f = 0; f < (DENS ? 4 : 3); ++f) s[f] += c * E[((size_t)f * norder + n) * nedge + e];
   }
   const double mul = a.mmul[0];
   double4* o = reinterpret_cast<double4*>(out_set + eof_fold32_floats(a.numx, a.numy, mmax)) + e;
@@ -209,10 +212,12 @@ struct EOFFoldIn {
   float* out;
   int64_t coef_stride, out_stride;
 };
-template <int SETS, bool DENS>
+// The pointers come as arguments of their own: read from the struct they lose
+// __restrict__, and with it the scalar loads of the coefficients (six sets 69 -> 115 us).
+template <int SETS>
 __device__ __forceinline__ void eof_fold_block(
     const float* __restrict__ T0, const float* __restrict__ T1, const float* __restrict__ T2,
-    const float* __restrict__ T3, const double* __restrict__ ccos, const double* __restrict__ csin,
+    const double* __restrict__ ccos, const double* __restrict__ csin,
     const double* __restrict__ E, float* __restrict__ out, const EOFFoldIn& f, const EOFFoldArgs& a,
     unsigned block, int set0) {
   __shared__ float4 s_fold[SETS][kFoldNodes][2 * kFoldM];
@@ -223,8 +228,8 @@ __device__ __forceinline__ void eof_fold_block(
     const int k = set0 + (int)(block % SETS);
     const int64_t e = (int64_t)(block / SETS) * kFoldThreads + threadIdx.x;
     if (k < nset && e < nedge)
-      eof_fold_edge(E, nedge, e, ccos + (size_t)k * coef_stride, mmax, norder, a,
-                    out + (size_t)k * out_stride);
+      eof_fold_edge<false>(E, nedge, e, ccos + (size_t)k * coef_stride, mmax, norder, a,
+                           out + (size_t)k * out_stride);
     return;
   }
   const unsigned b = block - eblocks;
@@ -248,21 +253,20 @@ __device__ __forceinline__ void eof_fold_block(
       const float* t0 = T0 + row;
       const float* t1 = T1 + row;
       const float* t2 = T2 + row;
-      const float* t3 = T3 + row;
-      double v[SETS][DENS ? 4 : 3];
+      double v[SETS][3];
 #pragma unroll
       for (int k = 0; k < SETS; ++k)
 #pragma unroll
-        for (int f = 0; f < (DENS ? 4 : 3); ++f) v[k][f] = 0.0;
+        for (int f = 0; f < 3; ++f) v[k][f] = 0.0;
 #pragma unroll 6
       for (int n = 0; n < a.nuse; ++n) {
         const size_t o = (size_t)n * nodes;
-        const float t[4] = {t0[o], t1[o], t2[o], DENS ? t3[o] : 0.f};
+        const float t[3] = {t0[o], t1[o], t2[o]};
 #pragma unroll
         for (int k = 0; k < SETS; ++k) {
           const double c = cf[k][n];
 #pragma unroll
-          for (int f = 0; f < (DENS ? 4 : 3); ++f) v[k][f] += c * t[f];
+          for (int f = 0; f < 3; ++f) v[k][f] += c * t[f];
         }
       }
       // slot j of a node at j ^ (node & 7): eight lanes' stores on eight bank groups
@@ -270,8 +274,7 @@ __device__ __forceinline__ void eof_fold_block(
 #pragma unroll
       for (int k = 0; k < SETS; ++k) {
         s_fold[k][lane][j ^ sw] =
-            make_float4((float)(v[k][0] * mul), (float)(v[k][1] * mul), (float)(v[k][2] * mul),
-                        DENS ? (float)(v[k][DENS ? 3 : 0] * mul) : 0.f);
+            make_float4((float)(v[k][0] * mul), (float)(v[k][1] * mul), (float)(v[k][2] * mul), 0.f);
         if (m == 0) s_fold[k][lane][1 ^ sw] = make_float4(0.f, 0.f, 0.f, 0.f);
       }
     }
@@ -291,9 +294,50 @@ __device__ __forceinline__ void eof_fold_block(
   }
 }
 
-template <int SETS, bool DENS>
+template <int SETS>
 __global__ __launch_bounds__(kFoldThreads) void eof_fold_kernel(EOFFoldIn f, EOFFoldArgs a) {
-  eof_fold_block<SETS, DENS>(f.T[0], f.T[1], f.T[2], f.T[3], f.ccos, f.csin, f.E, f.out, f, a, blockIdx.x, blockIdx.y * SETS);
+  eof_fold_block<SETS>(f.T[0], f.T[1], f.T[2], f.ccos, f.csin, f.E, f.out, f, a, blockIdx.x, blockIdx.y * SETS);
+}
+
+// One set with the density: one thread per (row group, node), the row groups one
+// after the other (q as above), so that a block reads 1 KB of a table row and the
+// grid streams the rows in turn.  Bound by those reads (124 MB at mmax 6, 257 x
+// 129 nodes): tables not in the cache 70 us, by blocks of 64 nodes 73 - 77; in the
+// cache, where the 16-byte stores cost, 38.4 and 36.2.  mmax 12: 124 / 136 and 69.8 /
+// 67.6, mmax 2: 31.5 / 35.8 and 19.0 / 19.8.
+__global__ __launch_bounds__(256) void eof_fold_rows_kernel(
+    const float* __restrict__ T0, const float* __restrict__ T1, const float* __restrict__ T2,
+    const float* __restrict__ T3, const double* __restrict__ ccos, const double* __restrict__ csin,
+    const double* __restrict__ E, float* __restrict__ out, EOFFoldIn f, EOFFoldArgs a, unsigned chunks) {
+  const unsigned eblocks = (unsigned)((f.nedge + 255) / 256);
+  if (blockIdx.x < eblocks) {
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e < f.nedge) eof_fold_edge<true>(E, f.nedge, e, ccos, f.mmax, f.norder, a, out);
+    return;
+  }
+  const unsigned b = blockIdx.x - eblocks;
+  const int q = (int)(b / chunks);
+  const int64_t nodes = f.nodes, node = (int64_t)(b - (unsigned)q * chunks) * 256 + threadIdx.x;
+  if (node >= nodes) return;
+  const bool sn = q > f.mmax;
+  const int m = sn ? q - f.mmax : q;
+  const double* cf = (sn ? csin : ccos) + (size_t)m * f.norder;
+  const double mul = a.mmul[m];
+  const size_t row = (size_t)q * f.norder * nodes + node;
+  const float *t0 = T0 + row, *t1 = T1 + row, *t2 = T2 + row, *t3 = T3 + row;
+  double v[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 6
+  for (int n = 0; n < a.nuse; ++n) {
+    const double c = cf[n];
+    const size_t o = (size_t)n * nodes;
+    v[0] += c * t0[o];
+    v[1] += c * t1[o];
+    v[2] += c * t2[o];
+    v[3] += c * t3[o];
+  }
+  float4* o = reinterpret_cast<float4*>(out) + ((size_t)node * (f.mmax + 1) + m) * 2;
+  o[sn ? 1 : 0] = make_float4((float)(v[0] * mul), (float)(v[1] * mul), (float)(v[2] * mul), (float)(v[3] * mul));
+  if (q == 0) o[1] = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
 // Both folds of one frozen field in one launch: the SL fold waits on its own
@@ -303,8 +347,8 @@ __global__ __launch_bounds__(kFoldThreads) void field_fold_kernel(SLFoldIn sf, S
                                                                      unsigned slblocks, EOFFoldIn ef,
                                                                      EOFFoldArgs ea) {
   if (blockIdx.x < slblocks) sl_fold_block(sf, sa, blockIdx.x, 0);
-  else eof_fold_block<1, false>(ef.T[0], ef.T[1], ef.T[2], ef.T[3], ef.ccos, ef.csin, ef.E, ef.out, ef, ea,
-                                blockIdx.x - slblocks, 0);
+  else eof_fold_block<1>(ef.T[0], ef.T[1], ef.T[2], ef.ccos, ef.csin, ef.E, ef.out, ef, ea,
+                         blockIdx.x - slblocks, 0);
 }
 
 static int ensure_folded(Context* c, float** d, size_t* have, size_t floats, hipStream_t s) {
@@ -395,7 +439,6 @@ static unsigned eof_fold_args(Context* c, const double* ccos, const double* csin
     a.mmul[m] = mul;
   }
   a.nuse = nuse;
-  a.dens = dens ? 1 : 0;
   a.numx = c->numx;
   a.numy = c->numy;
   const int64_t nedge = eof_edge_count(c->numx, c->numy);
@@ -415,12 +458,20 @@ static int eof_fold_into(Context* c, const double* ccos, const double* csin, int
   EOFFoldArgs a;
   auto go = [&](auto kernel, int sets) {
     const unsigned grid = eof_fold_args(c, ccos, csin, nset, sets, mmax_use, nuse, m1, m2, no_odd,
-                                        compat_mask, dens, out, &f, &a);
+                                        compat_mask, false, out, &f, &a);
     hipLaunchKernelGGL(kernel, dim3(grid, (unsigned)((nset + sets - 1) / sets)), dim3(kFoldThreads), 0, s, f, a);
   };
-  if (nset > 1 && !dens) go(eof_fold_kernel<kEofFoldSets, false>, kEofFoldSets);
-  else if (dens) go(eof_fold_kernel<1, true>, 1);
-  else go(eof_fold_kernel<1, false>, 1);
+  if (dens) {   // one set
+    eof_fold_args(c, ccos, csin, 1, 1, mmax_use, nuse, m1, m2, no_odd, compat_mask, true, out, &f, &a);
+    const unsigned chunks = (unsigned)((f.nodes + 255) / 256);
+    const unsigned grid = (unsigned)((f.nedge + 255) / 256) + (2u * (unsigned)f.mmax + 1) * chunks;
+    hipLaunchKernelGGL(eof_fold_rows_kernel, dim3(grid), dim3(256), 0, s, f.T[0], f.T[1], f.T[2], f.T[3], ccos,
+                       csin, f.E, out, f, a, chunks);
+  } else if (nset > 1) {
+    go(eof_fold_kernel<kEofFoldSets>, kEofFoldSets);
+  } else {
+    go(eof_fold_kernel<1>, 1);
+  }
   BFE_HIP(c, hipGetLastError());
   return 0;
 }
