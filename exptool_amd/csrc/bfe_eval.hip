@@ -13,17 +13,16 @@ struct SLFoldArgs {
   int lmax, nmax_use;
 };
 
-// Four lanes per (kFoldRows radial nodes from i0, (l, m) pair p in m-major
-// order), lane q summing radial orders q, q + 4, ...: the sums of a table row are
-// shared by the nodes that read it (a node takes rows i and i + 1 of E and D and
-// three rows of G), so kFoldRows nodes cost 3 kFoldRows + 4 rows instead of
-// 7 kFoldRows.  The four partial sums are combined across the lanes, D1/D2 formed,
-// and the blocks rounded once to float32 (layout in bfe_field.hpp; the last node,
-// never a cell start, is zero).  What bounds it is the latency and number of the
-// row gathers: lmax 6, nmax 20, numr 2000, one set / 12 sets, with one node a
-// group of lanes and seven rows each 12.3 / 75 us, one, two and four nodes with
-// shared rows 15.6 / 91, 10.5 / 55 and 10.3 / 47; smaller tables (lmax 4, numr
-// 1000) 6.4, then 8.0, 6.2 and 7.8.
+// Four lanes per (R radial nodes from i0, (l, m) pair p in m-major order), lane q
+// summing radial orders q, q + 4, ...: the sums of a table row are shared by the
+// nodes that read it (a node takes rows i and i + 1 of E and D and three rows of G),
+// so R nodes cost 3 R + 4 rows instead of 7 R.  The four partial sums are combined
+// across the lanes, D1/D2 formed, and the blocks rounded once to float32 (layout in
+// bfe_field.hpp; the last node, never a cell start, is zero).  What bounds it is the
+// latency and number of the row gathers: lmax 6, nmax 20, numr 2000, one set / 12
+// sets, with one node a group of lanes and seven rows each 12.3 / 75 us, one, two and
+// four nodes with shared rows 15.6 / 91, 10.5 / 55 and 10.3 / 47; small tables take
+// one (sl_fold_rows).
 struct SLFoldIn {
   const double* S;       // fold inputs
   const double* coef;
@@ -32,7 +31,6 @@ struct SLFoldIn {
   int64_t coef_stride, out_stride;
 };
 constexpr int kFoldLanes = 4;
-constexpr int kFoldRows = 2;
 // Nodes i0 .. i0 + R - 1 of the pair at place j of the l-major order, into the
 // node blocks at o (2 np float4 a node) and the density blocks at od.
 template <int R>
@@ -136,23 +134,25 @@ __device__ __forceinline__ void sl_fold_nodes(const SLFoldIn& f, const SLFoldArg
   }
 }
 
+template <int R>
 __device__ __forceinline__ void sl_fold_block(const SLFoldIn& f, const SLFoldArgs& a, unsigned block,
                                               int set) {
   const int np = sl_npairs(a.lmax);
   const unsigned gid = block * blockDim.x + threadIdx.x;
   const unsigned idx = gid / kFoldLanes;
   const int g = (int)(idx / (unsigned)np);
-  const int i0 = g * kFoldRows;
+  const int i0 = g * R;
   // groups of four lanes are whole within a wave, so a group leaves together
   if (i0 >= f.numr) return;
   float4* o = reinterpret_cast<float4*>(f.out + (size_t)set * f.out_stride);
-  sl_fold_nodes<kFoldRows>(f, a, i0, (int)(idx - (unsigned)g * (unsigned)np), (int)(gid & (kFoldLanes - 1)),
-                           f.coef + (size_t)set * f.coef_stride, o + (size_t)i0 * np * 2,
-                           o + (size_t)f.numr * np * 2 + (size_t)i0 * np);
+  sl_fold_nodes<R>(f, a, i0, (int)(idx - (unsigned)g * (unsigned)np), (int)(gid & (kFoldLanes - 1)),
+                   f.coef + (size_t)set * f.coef_stride, o + (size_t)i0 * np * 2,
+                   o + (size_t)f.numr * np * 2 + (size_t)i0 * np);
 }
 
+template <int R>
 __global__ __launch_bounds__(256) void sl_fold_kernel(SLFoldIn f, SLFoldArgs a) {
-  sl_fold_block(f, a, blockIdx.x, blockIdx.y);
+  sl_fold_block<R>(f, a, blockIdx.x, blockIdx.y);
 }
 
 struct EOFFoldArgs {
@@ -343,10 +343,11 @@ __global__ __launch_bounds__(256) void eof_fold_rows_kernel(
 // Both folds of one frozen field in one launch: the SL fold waits on its own
 // gathers and runs in the shadow of the EOF fold's table reads (23 us; as two
 // launches on two streams 21 and 12 us and 15 us of events between them).
+template <int R>
 __global__ __launch_bounds__(kFoldThreads) void field_fold_kernel(SLFoldIn sf, SLFoldArgs sa,
-                                                                     unsigned slblocks, EOFFoldIn ef,
-                                                                     EOFFoldArgs ea) {
-  if (blockIdx.x < slblocks) sl_fold_block(sf, sa, blockIdx.x, 0);
+                                                                  unsigned slblocks, EOFFoldIn ef,
+                                                                  EOFFoldArgs ea) {
+  if (blockIdx.x < slblocks) sl_fold_block<R>(sf, sa, blockIdx.x, 0);
   else eof_fold_block<1>(ef.T[0], ef.T[1], ef.T[2], ef.ccos, ef.csin, ef.E, ef.out, ef, ea,
                          blockIdx.x - slblocks, 0);
 }
@@ -398,7 +399,8 @@ static int64_t sl_fold_args(Context* c, const double* coef, int nset, double hal
     }
   *f = SLFoldIn{c->sl_fold64, coef, c->nmax, c->numr, nset, out,
                 (int64_t)(c->lmax + 1) * (c->lmax + 1) * c->nmax, (int64_t)sl_fold_floats(c)};
-  return (int64_t)((c->numr + kFoldRows - 1) / kFoldRows) * sl_npairs(c->lmax) * kFoldLanes;
+  const int rows = sl_fold_rows(c->numr, c->lmax);
+  return (int64_t)((c->numr + rows - 1) / rows) * sl_npairs(c->lmax) * kFoldLanes;
 }
 
 static int sl_fold_into(Context* c, const double* coef, int nset, double halofac, int lmax_use,
@@ -406,8 +408,11 @@ static int sl_fold_into(Context* c, const double* coef, int nset, double halofac
   SLFoldIn f;
   SLFoldArgs a;
   const int64_t lanes = sl_fold_args(c, coef, nset, halofac, lmax_use, nmax_use, L1, L2, no_odd, out, &f, &a);
-  hipLaunchKernelGGL(sl_fold_kernel, dim3((unsigned)((lanes + 255) / 256), (unsigned)nset), dim3(256), 0, s,
-                     f, a);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((lanes + 255) / 256), (unsigned)nset), dim3(256), 0, s, f, a);
+  };
+  if (sl_fold_rows(c->numr, c->lmax) == 2) go(sl_fold_kernel<2>);
+  else go(sl_fold_kernel<1>);
   BFE_HIP(c, hipGetLastError());
   return 0;
 }
@@ -1054,7 +1059,11 @@ static int field_set_run(Context* c, const double* eof_cos, const double* eof_si
   const unsigned eb = eof_fold_args(c, eof_cos, eof_sin, 1, 1, mm, nn, 0, 1 << 30, no_odd,
                                     (flags & BFE_COMPAT_EOF_MASK) != 0, false, c->eoff[1].d, &ef, &ea);
   const unsigned sb = (unsigned)((lanes + kFoldThreads - 1) / kFoldThreads);
-  hipLaunchKernelGGL(field_fold_kernel, dim3(sb + eb), dim3(kFoldThreads), 0, s, sf, sa, sb, ef, ea);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(sb + eb), dim3(kFoldThreads), 0, s, sf, sa, sb, ef, ea);
+  };
+  if (sl_fold_rows(c->numr, c->lmax) == 2) go(field_fold_kernel<2>);
+  else go(field_fold_kernel<1>);
   BFE_HIP(c, hipGetLastError());
   c->slf[1].valid = c->eoff[1].valid = true;
   c->field_halofac = halofac;

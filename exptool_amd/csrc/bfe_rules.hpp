@@ -97,4 +97,13 @@ inline bool eval_split_two(int64_t n, int lmax, int mmax, bool split_ok, int64_t
   return n <= (split_fixed(lmax, mmax) ? 114688 : 49152);
 }
 
+// Nodes a group of four lanes folds in the whole-table SL fold: one until the lanes
+// of two a group fill 128 blocks, then two, which share rows.  Whole calls, one / two,
+// us at lmax, numr (nmax 20): 0, 2000 7.8 / 8.5; 2, 2000 10.3 / 11.0; 4, 1000 (30 000
+// lanes) 13.2 / 13.8; 3, 2000 (40 000) 12.9 / 12.4; 6, 2000 22.1 / 20.4; 8, 4000 41.0 /
+// 36.9.
+inline int sl_fold_rows(int numr, int lmax) {
+  return (int64_t)numr * (lmax + 1) * (lmax + 2) >= 32768 ? 2 : 1;
+}
+
 }  // namespace bfe

@@ -1,5 +1,6 @@
-"""The forms an evaluation chooses between give the same bits per point: whole
+"""The forms a fold or an evaluation chooses between give the same bits per point: whole
 calls against the same points in slices that take another build or form."""
+import numpy as np
 import pytest
 
 from tests.test_gpu_split import _points, _same, system  # noqa: F401
@@ -46,3 +47,23 @@ def test_default_form_agrees_with_input_order(system, n):  # noqa: F811
     for a, b in zip(got, ref):
         for u, v in zip(a, b):
             _same(u, v)
+
+
+@pytest.mark.parametrize("density", [False, True])
+@pytest.mark.parametrize("lmax,numr", [(3, 1638), (3, 1639), (9, 601), (16, 108)])
+def test_sl_fold_of_one_and_two_nodes(lmax, numr, density):
+    """Whole-table SL folds on either side of the line (32 768 lanes), odd and even
+    numr, against the points' own cells: the same bits in every part of the table."""
+    import torch
+    from exptool_amd.basis import tablegen
+    from exptool_amd.bfe import BFESystem
+    s = BFESystem(sl=tablegen.make_sl_tables(lmax=lmax, nmax=5, numr=numr, rmin=1e-3, rmax=50.0, cmap=1, scale=1.0))
+    g = np.random.default_rng(lmax)
+    r = np.concatenate([[0.0, 1e-9, 1e-3, 49.9, 1e6], 10 ** g.uniform(-3, 1.7, 400)])
+    t, ph = g.uniform(-1, 1, r.size), g.uniform(-4, 4, r.size)
+    c = g.normal(size=((lmax + 1) ** 2, 5))
+    out = []
+    for pb in (0, 512):
+        s.set_tuning("point_blocks", pb)
+        out.append(s.sl_eval_sph(r, t, ph, c, density=density))
+    assert torch.equal(out[0], out[1])

@@ -25,6 +25,7 @@ int main() {
       std::printf("%d\n", (int)bfe::eval_form(a[0], a[1], a[2], a[3] != 0, a[4], a[5]));
     else if (!std::strcmp(f, "eval_split_two"))
       std::printf("%d\n", (int)bfe::eval_split_two(a[0], a[1], a[2], a[3] != 0, a[4], a[5]));
+    else if (!std::strcmp(f, "sl_fold_rows")) std::printf("%d\n", bfe::sl_fold_rows(a[0], a[1]));
     else return 1;
   }
   return 0;
@@ -129,3 +130,15 @@ def test_evaluation_form_follows_explicit_knobs(rule):
     calls = [(5000, 2, 2, 1, 1 << 40, 1 << 40), (5000, 2, 2, 0, 1 << 40, 1 << 40), (5000, 2, 2, 1, 1, 1 << 40),
              (5000, 2, 2, 1, 1 << 40, 4999), (131_072, 6, 6, 1, 65_536, 131_072)]
     assert [v[0] for v in rule("eval_split_two", calls)] == [1, 0, 0, 0, 0]
+
+
+# us of a whole-table SL evaluation on MI355X with one and two nodes a group of lanes
+# at numr, lmax (nmax 20)
+SL_FOLD = [(300, 0, 7.6, 8.3), (300, 8, 21.1, 21.7), (1000, 1, 8.9, 9.6), (1000, 4, 13.2, 13.8), (1000, 6, 19.0, 18.2),
+           (2000, 0, 7.8, 8.5), (2000, 2, 10.3, 11.0), (2000, 3, 12.9, 12.4), (2000, 6, 22.1, 20.4),
+           (4000, 1, 9.2, 10.0), (4000, 2, 11.8, 11.2), (4000, 8, 41.0, 36.9)]
+
+
+def test_sl_fold_shares_rows_where_it_is_the_faster(rule):
+    for (numr, lmax, *us), (rows,) in zip(SL_FOLD, rule("sl_fold_rows", [v[:2] for v in SL_FOLD])):
+        assert us[rows - 1] == min(us), (numr, lmax, rows)
