@@ -66,9 +66,6 @@ constexpr int kInfPts = kWaveTile * kBlockInf / 64;   // points per block
 // the integrator, which holds its state as well and spills 500 B a lane, 55.7 ->
 // 37.5 ms per 100 steps of 1M orbits.
 constexpr int kBlockGrad = 512;
-// Blocks of the inference kernel: one per CU loads the weights (104 KB) once
-// (523 us under the profiler, 537 with 2 048 blocks).
-constexpr int kGradBlocks = 256;
 // LDS copy of the three hidden weight matrices: rows of kH bf16 padded to
 // kLdsRow.  A lane reads 16 bytes of row 16 mt + c; unpadded (256-byte)
 // rows put the rows that one read cycle serves on the same four banks, with
@@ -482,11 +479,11 @@ __global__ __launch_bounds__(kBlockInf) void mlp_fwd_kernel(MLPKArgs a) {
 }
 
 // Inference of the conservative field: out = Phi, F_R, F_phi, F_z with
-// F = -grad Phi (mlp_tile_grad).  A wave takes `per` 16-point tiles (1 or 4) at a
-// time: the features and the force of the base model, a fifth of the vector work
+// F = -grad Phi (mlp_tile_grad).  The first `waves` waves of a block take `per`
+// 16-point tiles (1 to 4) each at a time (mlp_grad_launch): the features and the force of the base model, a fifth of the vector work
 // when every lane group of a tile repeats them, are then evaluated one point per
 // lane, and the tiles' features and results pass through the lanes.
-__global__ __launch_bounds__(kBlockGrad) void mlp_fwd_grad_kernel(MLPKArgs a, int per) {
+__global__ __launch_bounds__(kBlockGrad) void mlp_fwd_grad_kernel(MLPKArgs a, int waves, int per) {
   constexpr int NT = 1;
   extern __shared__ __align__(16) unsigned char smem[];
   __bf16* sW = reinterpret_cast<__bf16*>(smem);
@@ -497,8 +494,9 @@ __global__ __launch_bounds__(kBlockGrad) void mlp_fwd_grad_kernel(MLPKArgs a, in
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int g = lane >> 4, c = lane & 15;
   const int pts = 16 * per;            // points of a wave
-  for (int64_t base = ((int64_t)blockIdx.x * (kBlockGrad / 64) + wave) * pts; base < a.n;
-       base += (int64_t)gridDim.x * (kBlockGrad / 64) * pts) {
+  if (wave >= waves) return;
+  for (int64_t base = ((int64_t)blockIdx.x * waves + wave) * pts; base < a.n;
+       base += (int64_t)gridDim.x * waves * pts) {
     const int64_t p = base + lane;
     const bool valid = lane < pts && p < a.n;
     const int64_t q = valid ? p : base;
@@ -1452,12 +1450,8 @@ extern "C" int bfe_mlp_forward(bfe_ctx* h, const float* x, const float* y, const
   MLPKArgs a = base_args(c);
   a.x = x; a.y = y; a.z = z; a.n = n; a.out = out;
   if (c->mlp.conservative) {
-    // four tiles a wave once every wave of the device has them
-    constexpr int kWaves = kBlockGrad / 64;
-    const int per = n > (int64_t)kGradBlocks * kWaves * 16 ? 4 : 1;
-    const int64_t blocks = (n + 16 * per * kWaves - 1) / (16 * per * kWaves);
-    const int nb = (int)(blocks < kGradBlocks ? blocks : kGradBlocks);
-    hipLaunchKernelGGL(mlp_fwd_grad_kernel, dim3(nb), dim3(kBlockGrad), kLdsBytes, s, a, per);
+    const GradLaunch g = mlp_grad_launch(n);
+    hipLaunchKernelGGL(mlp_fwd_grad_kernel, dim3(g.blocks), dim3(kBlockGrad), kLdsBytes, s, a, g.waves, g.per);
     BFE_HIP(c, hipGetLastError());
     return 0;
   }

@@ -106,4 +106,25 @@ inline int sl_fold_rows(int numr, int lmax) {
   return (int64_t)numr * (lmax + 1) * (lmax + 2) >= 32768 ? 2 : 1;
 }
 
+// Launch of the conservative surrogate's inference: the first `waves` of a block's
+// eight take `per` 16-point tiles each at a time; at most one block a CU (its LDS
+// holds the weights, loaded once by all eight: 1M points 523 us under a profiler,
+// 537 with 2 048 blocks).  Up to 16 384 points four waves a block give every tile a
+// SIMD to itself (14.8 us; eight on half the CUs 19.5); from there eight, and as many
+// tiles a wave at a time as the waves of the whole device leave it, at most four
+// (one point load and one base model a lane then serve four tiles), in rounds of
+// nearly equal length.  32 769 points: two tiles a wave 30.8 us, four on a quarter of
+// the CUs 54; 65 537: three 42.6, four 55.
+struct GradLaunch {
+  int waves, per, blocks;
+};
+inline GradLaunch mlp_grad_launch(int64_t n) {
+  const int64_t tiles = (n + 15) / 16;
+  const int waves = tiles <= 256 * 4 ? 4 : 8;
+  const int64_t steps = (tiles + 256 * 8 - 1) / (256 * 8), rounds = (steps + 3) / 4;
+  const int per = (int)((steps + rounds - 1) / rounds);
+  const int64_t blocks = (tiles + (int64_t)per * waves - 1) / ((int64_t)per * waves);
+  return GradLaunch{waves, per, (int)(blocks < 256 ? blocks : 256)};
+}
+
 }  // namespace bfe

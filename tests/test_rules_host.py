@@ -26,7 +26,10 @@ int main() {
     else if (!std::strcmp(f, "eval_split_two"))
       std::printf("%d\n", (int)bfe::eval_split_two(a[0], a[1], a[2], a[3] != 0, a[4], a[5]));
     else if (!std::strcmp(f, "sl_fold_rows")) std::printf("%d\n", bfe::sl_fold_rows(a[0], a[1]));
-    else return 1;
+    else if (!std::strcmp(f, "mlp_grad_launch")) {
+      const bfe::GradLaunch g = bfe::mlp_grad_launch(a[0]);
+      std::printf("%d %d %d\n", g.waves, g.per, g.blocks);
+    } else return 1;
   }
   return 0;
 }
@@ -142,3 +145,18 @@ SL_FOLD = [(300, 0, 7.6, 8.3), (300, 8, 21.1, 21.7), (1000, 1, 8.9, 9.6), (1000,
 def test_sl_fold_shares_rows_where_it_is_the_faster(rule):
     for (numr, lmax, *us), (rows,) in zip(SL_FOLD, rule("sl_fold_rows", [v[:2] for v in SL_FOLD])):
         assert us[rows - 1] == min(us), (numr, lmax, rows)
+
+
+def test_surrogate_inference_fills_the_device(rule):
+    """No size makes a wave take more tiles in sequence than the device's waves
+    leave it (plus the rounding to rounds of equal length), one wave a SIMD where
+    that is enough, every point covered."""
+    ns = [1, 15, 16, 17, 64, 65, 1000, 16_383, 16_384, 16_385, 20_000, 32_768, 32_769, 40_000, 49_152, 65_536, 65_537,
+          80_000, 98_305, 131_072, 131_073, 200_000, 262_145, 524_289, 1_000_000, 10_000_001]
+    for n, (waves, per, blocks) in zip(ns, rule("mlp_grad_launch", [(n,) for n in ns])):
+        tiles = -(-n // 16)
+        assert waves == (4 if n <= 16_384 else 8) and 1 <= per <= 4 and 1 <= blocks <= 256
+        sweep = blocks * waves * per
+        steps = -(-tiles // sweep) * per          # tiles of the busiest wave
+        ideal = -(-tiles // (256 * waves))
+        assert steps <= ideal * 1.25, (n, waves, per, blocks)
