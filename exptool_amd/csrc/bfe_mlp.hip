@@ -58,14 +58,17 @@ constexpr int kWaveTile = 16 * kNT;              // points per wave
 // Threads per block of the inference and integrator kernels: 8 waves on one
 // copy of the LDS weights (two waves per SIMD hide the SiLU latency).
 constexpr int kBlockInf = BFE_MLP_BLOCK;
+static_assert(kBlockInf == 512 && kNT == 2, "mlp_leap_launch");
 constexpr int kInfPts = kWaveTile * kBlockInf / 64;   // points per block
 // The conservative-field kernels carry three tangent operand sets beside the
 // activations (192 registers): eight waves per block, two per SIMD, so that one
 // wave's activations cover the other's products.  Inference of 1M points 667 ->
 // 458 us against four waves (no spills; 422 with the point work once per point);
 // the integrator, which holds its state as well and spills 500 B a lane, 55.7 ->
-// 37.5 ms per 100 steps of 1M orbits.
+// 37.5 ms per 100 steps of 1M orbits.  Few orbits take four waves, one per SIMD, with
+// nothing spilled (mlp_leap_launch).
 constexpr int kBlockGrad = 512;
+constexpr int kBlockGradSmall = 256;
 // LDS copy of the three hidden weight matrices: rows of kH bf16 padded to
 // kLdsRow.  A lane reads 16 bytes of row 16 mt + c; unpadded (256-byte)
 // rows put the rows that one read cycle serves on the same four banks, with
@@ -1074,11 +1077,11 @@ __device__ __forceinline__ void surrogate_accel(const MLPLeapArgs& a, FieldTable
   pot = a.cfg.os[0] * yv[0] + a.cfg.ob[0] + bv[0];
 }
 
-template <bool GRAD>
-__global__ __launch_bounds__(GRAD ? kBlockGrad : kBlockInf) void mlp_leapfrog_kernel(MLPLeapArgs a) {
+template <bool GRAD, int kBlock>
+__global__ __launch_bounds__(kBlock) void mlp_leapfrog_kernel(MLPLeapArgs a) {
   // GRAD: conservative forces from mlp_tile_grad, 16-point tiles
   constexpr int NT = GRAD ? 1 : kNT;
-  constexpr int kBlock = GRAD ? kBlockGrad : kBlockInf, kBlockPts = 16 * NT * (kBlock / 64);
+  constexpr int kBlockPts = 16 * NT * (kBlock / 64);
   extern __shared__ __align__(16) unsigned char smem[];
   __bf16* sW = reinterpret_cast<__bf16*>(smem);
   float* sS = reinterpret_cast<float*>(smem + kLdsWBytes);
@@ -1373,9 +1376,11 @@ extern "C" int bfe_mlp_set_params(bfe_ctx* h, const float* params, int64_t count
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes));
     BFE_HIP(c, hipFuncSetAttribute((const void*)mlp_train_kernel,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTrainLds));
-    BFE_HIP(c, hipFuncSetAttribute((const void*)mlp_leapfrog_kernel<false>,
+    BFE_HIP(c, hipFuncSetAttribute((const void*)mlp_leapfrog_kernel<false, kBlockInf>,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes));
-    BFE_HIP(c, hipFuncSetAttribute((const void*)mlp_leapfrog_kernel<true>,
+    BFE_HIP(c, hipFuncSetAttribute((const void*)mlp_leapfrog_kernel<true, kBlockGradSmall>,
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes));
+    BFE_HIP(c, hipFuncSetAttribute((const void*)mlp_leapfrog_kernel<true, kBlockGrad>,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes));
     BFE_HIP(c, hipFuncSetAttribute((const void*)mlp_fwd_grad_kernel,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes));
@@ -1515,8 +1520,8 @@ extern "C" int bfe_mlp_leapfrog(bfe_ctx* h, float* x, float* y, float* z, float*
   if (n == 0) return 0;
   BFE_HIP(c, hipSetDevice(c->device));
   hipStream_t s = (hipStream_t)stream;
-  const int64_t ntiles = (n + kInfPts - 1) / kInfPts;
-  const int nb = (int)(ntiles < 2048 ? ntiles : 2048);
+  const LeapLaunch shape = mlp_leap_launch(n, c->mlp.conservative != 0);
+  const int nb = shape.blocks;
   const int chunk = energy_every > 0 ? energy_every : (int)(nsteps < 100 ? (nsteps > 0 ? nsteps : 1) : 100);
   const int nchecks = energy_every > 0 ? (int)(nsteps / energy_every) + 1 : 1;
   const size_t aux_bytes = (size_t)n * sizeof(MLPOrbitAux);
@@ -1545,10 +1550,15 @@ extern "C" int bfe_mlp_leapfrog(bfe_ctx* h, float* x, float* y, float* z, float*
   a.energy_check = 1;
   a.partE = energy_log ? partE : nullptr;
   a.check_index = 0;
-  if (a.cfg.conservative)
-    hipLaunchKernelGGL(mlp_leapfrog_kernel<true>, dim3(nb), dim3(kBlockGrad), kLdsBytes, s, a);
-  else
-    hipLaunchKernelGGL(mlp_leapfrog_kernel<false>, dim3(nb), dim3(kBlockInf), kLdsBytes, s, a);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(nb), dim3(64 * shape.waves), kLdsBytes, s, a);
+  };
+  auto go = [&]() {
+    if (!a.cfg.conservative) launch(mlp_leapfrog_kernel<false, kBlockInf>);
+    else if (shape.waves == kBlockGradSmall / 64) launch(mlp_leapfrog_kernel<true, kBlockGradSmall>);
+    else launch(mlp_leapfrog_kernel<true, kBlockGrad>);
+  };
+  go();
   BFE_HIP(c, hipGetLastError());
   a.init = 0;
   for (int64_t k0 = 0, ci = 0; k0 < nsteps; k0 += chunk, ++ci) {
@@ -1557,10 +1567,7 @@ extern "C" int bfe_mlp_leapfrog(bfe_ctx* h, float* x, float* y, float* z, float*
     a.energy_check = (energy_every > 0 && a.k1 - a.k0 == energy_every) ? 1 : 0;
     a.partE = (energy_log && a.energy_check) ? partE : nullptr;
     a.check_index = (int)ci + 1;
-    if (a.cfg.conservative)
-    hipLaunchKernelGGL(mlp_leapfrog_kernel<true>, dim3(nb), dim3(kBlockGrad), kLdsBytes, s, a);
-  else
-    hipLaunchKernelGGL(mlp_leapfrog_kernel<false>, dim3(nb), dim3(kBlockInf), kLdsBytes, s, a);
+    go();
     BFE_HIP(c, hipGetLastError());
   }
   if (drift_out || maxerr_out || counts_out)

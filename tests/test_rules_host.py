@@ -29,6 +29,9 @@ int main() {
     else if (!std::strcmp(f, "mlp_grad_launch")) {
       const bfe::GradLaunch g = bfe::mlp_grad_launch(a[0]);
       std::printf("%d %d %d\n", g.waves, g.per, g.blocks);
+    } else if (!std::strcmp(f, "mlp_leap_launch")) {
+      const bfe::LeapLaunch g = bfe::mlp_leap_launch(a[0], a[1] != 0);
+      std::printf("%d %d\n", g.waves, g.blocks);
     } else return 1;
   }
   return 0;
@@ -160,3 +163,12 @@ def test_surrogate_inference_fills_the_device(rule):
         steps = -(-tiles // sweep) * per          # tiles of the busiest wave
         ideal = -(-tiles // (256 * waves))
         assert steps <= ideal * 1.25, (n, waves, per, blocks)
+
+
+@pytest.mark.parametrize("conservative,per_wave", [(1, 16), (0, 32)])
+def test_surrogate_orbits_take_one_tile_a_block(rule, conservative, per_wave):
+    """A block walks several tiles of orbits only once eight blocks a CU are there."""
+    ns = [1, 64, 65, 128, 129, 1000, 16_384, 16_385, 20_000, 65_536, 100_000, 262_144, 262_145, 1_000_000]
+    for n, (waves, blocks) in zip(ns, rule("mlp_leap_launch", [(n, conservative) for n in ns])):
+        assert waves == (4 if conservative and n <= 16_384 else 8)
+        assert blocks == min(2048, -(-n // (waves * per_wave))), n
