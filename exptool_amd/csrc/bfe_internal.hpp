@@ -80,7 +80,7 @@ struct MLPState {
   __bf16* Wp = nullptr;
   __bf16* Wt = nullptr;
   float* dwpart = nullptr;       // per 128-point tile: partial sums of dW1..dW3
-  float* small_wave = nullptr;   // per tile and wave: of the other gradients
+  double* small_wave = nullptr;  // per training block and wave: of the other gradients
   double* small_part = nullptr;  // per training block: these and the loss
   int64_t bcap = 0;              // tiles these hold
   int64_t step = 0;

@@ -549,8 +549,8 @@ __global__ __launch_bounds__(kBlockGrad) void mlp_fwd_grad_kernel(MLPKArgs a, in
 // neuron l of four points).  Wave w makes output rows 16 w .. 16 w + 15.  The
 // k order of the products is point 4 g + j, then 16 + 4 g + j, for lane group
 // g, in both operands.  The sums run in float32 over a tile and in float64
-// over tiles.  b0..b3, W0 and W4 gradients: float32 sums over the wave's 16
-// points by pairs (reduce_rows), float64 beyond.
+// over tiles.  b0..b3, W0 and W4 gradients: products and sums over points in
+// float64 throughout (reduce_rows).
 // Measured for 65 536 points: 910 us as separate forward, backward, weight
 // gradient and reduction kernels (72 + 200 + 337 + 63 + 197 + 41), 90 us for
 // this one and 16 for the reduction (100 MB of partial sums); about half of a
@@ -578,7 +578,7 @@ struct MLPTrainArgs {
   const __bf16* Wp;
   const __bf16* Wt;
   float* dwpart;         // [tile][3][128][128]
-  float* small_wave;     // [tile][8 waves][11][128]
+  double* small_wave;    // [block][8 waves][11][128]
   double* small_part;    // [block][kSmallRow]: dW0[d][nr], db0..db3, dW4, db4, loss
   MLPCfg cfg;
 };
@@ -696,33 +696,54 @@ __device__ __forceinline__ void forget(floatx4 (&z)[8]) {
 }
 
 template <int CTRL>
+__device__ __forceinline__ int dpp_get(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
 __device__ __forceinline__ float dpp_get(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+  return __int_as_float(dpp_get<CTRL>(__float_as_int(v)));
 }
 
-// Sums of the 32 values over the 16 lanes of a row (one point each): each
-// exchange halves the values a lane keeps; lane c ends with the sums of
-// values 2 c and 2 c + 1.
-__device__ __forceinline__ void reduce_rows(float (&v)[32], int c, float (&s)[2]) {
-  const bool b3 = c & 8, b2 = c & 4, b1 = c & 2, b0 = c & 1;
+template <int CTRL>
+__device__ __forceinline__ double dpp_get(double v) {
+  return __hiloint2double(dpp_get<CTRL>(__double2hiint(v)), dpp_get<CTRL>(__double2loint(v)));
+}
+
+// Sums of a lane's 32 values over the 16 lanes of a row (one point each), products
+// and sums in float64.  Each exchange halves the values a lane keeps; lane c ends
+// with the sums of values 2 c and 2 c + 1.  The first exchange passes the float32
+// values, kept in v[0..15] and received in v[16..31], once for several factors.
+__device__ __forceinline__ void rows_exchange(float (&v)[32], int c) {
+  const bool b3 = c & 8;
 #pragma unroll
   for (int k = 0; k < 16; ++k) {
     const float keep = b3 ? v[k + 16] : v[k], send = b3 ? v[k] : v[k + 16];
-    v[k] = keep + dpp_get<0x140>(send);   // row_mirror: lane 15 - c
+    v[k] = keep;
+    v[k + 16] = dpp_get<0x140>(send);   // row_mirror: lane 15 - c
   }
+}
+// The sums of the exchanged values times the lanes' factors m (MUL).
+template <bool MUL>
+__device__ __forceinline__ void reduce_rows(const float (&v)[32], float m, int c, double (&s)[2]) {
+  const bool b2 = c & 4, b1 = c & 2, b0 = c & 1;
+  const double mk = m, mo = dpp_get<0x140>(m);
+  double t[16];
+#pragma unroll
+  for (int k = 0; k < 16; ++k)
+    t[k] = MUL ? fma((double)v[k], mk, (double)v[k + 16] * mo) : (double)v[k] + (double)v[k + 16];
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
-    const float keep = b2 ? v[k + 8] : v[k], send = b2 ? v[k] : v[k + 8];
-    v[k] = keep + dpp_get<0x141>(send);   // row_half_mirror
+    const double keep = b2 ? t[k + 8] : t[k], send = b2 ? t[k] : t[k + 8];
+    t[k] = keep + dpp_get<0x141>(send);   // row_half_mirror
   }
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const float keep = b1 ? v[k + 4] : v[k], send = b1 ? v[k] : v[k + 4];
-    v[k] = keep + dpp_get<0x4E>(send);    // lanes 2 apart
+    const double keep = b1 ? t[k + 4] : t[k], send = b1 ? t[k] : t[k + 4];
+    t[k] = keep + dpp_get<0x4E>(send);    // lanes 2 apart
   }
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
-    const float keep = b0 ? v[k + 2] : v[k], send = b0 ? v[k] : v[k + 2];
+    const double keep = b0 ? t[k + 2] : t[k], send = b0 ? t[k] : t[k + 2];
     s[k] = keep + dpp_get<0xB1>(send);    // neighbours
   }
 }
@@ -748,15 +769,17 @@ __device__ __forceinline__ float pick4(const float (&v)[4], int k) {
   return k == 0 ? v[0] : k == 1 ? v[1] : k == 2 ? v[2] : v[3];
 }
 
-// Sums over the wave's 16 points of m v, to the wave's row of small sums:
-// lane c of group g has neurons 16 (c / 2) + 4 g + 2 (c & 1) + {0, 1}.
-__device__ __forceinline__ void small_sums(const float (&v)[32], float m, float* __restrict__ row,
-                                           int g, int c) {
-  float u[32], s[2];
-#pragma unroll
-  for (int j = 0; j < 32; ++j) u[j] = m * v[j];
-  reduce_rows(u, c, s);
-  *reinterpret_cast<float2*>(row + 16 * (c >> 1) + 4 * g + 2 * (c & 1)) = make_float2(s[0], s[1]);
+// Sums over the wave's 16 points of m v (MUL) or v, v exchanged (rows_exchange), to
+// the wave's row of small sums, added to what an earlier tile left there: lane c of
+// group g has neurons 16 (c / 2) + 4 g + 2 (c & 1) + {0, 1}.
+template <bool MUL>
+__device__ __forceinline__ void small_sums(const float (&v)[32], float m, double* __restrict__ row,
+                                           bool first, int g, int c) {
+  double2* o = reinterpret_cast<double2*>(row + 16 * (c >> 1) + 4 * g + 2 * (c & 1));
+  const double2 old = first ? make_double2(0.0, 0.0) : *o;
+  double s[2];
+  reduce_rows<MUL>(v, m, c, s);
+  *o = make_double2(old.x + s[0], old.y + s[1]);
 }
 
 __global__ __launch_bounds__(kTrainThreads) void mlp_train_kernel(MLPTrainArgs a) {
@@ -777,15 +800,13 @@ __global__ __launch_bounds__(kTrainThreads) void mlp_train_kernel(MLPTrainArgs a
   train_load(a.Wp, buf, wave, lane);
   load_small(a.params, sS);
   if (lane < 5) s_loss[wave][lane] = 0.0;          // the wave's loss and db4
-  int tiles = 0;
+  double* rows = a.small_wave + ((size_t)blockIdx.x * 8 + wave) * 11 * kH;   // dW0 (3), db0..3, dW4 (4)
 #pragma unroll 1
   for (int t = 0; t < a.tiles; ++t) {
     const int64_t tile = (int64_t)blockIdx.x * a.tiles + t;
     const int64_t p0 = tile * kTrainPts;
     if (p0 >= a.n) break;
-    ++tiles;
     float* part = a.dwpart + (size_t)tile * 3 * kH * kH;
-    float* rows = a.small_wave + ((size_t)tile * 8 + wave) * 11 * kH;   // dW0 (3), db0..3, dW4 (4)
     const int row = 16 * wave + c;   // the lane's point in the tile
     const int64_t p = p0 + row;
     const bool valid = p < a.n;
@@ -860,8 +881,9 @@ __global__ __launch_bounds__(kTrainThreads) void mlp_train_kernel(MLPTrainArgs a
         s_loss[wave][1 + k] += bs;
       }
     }
+    rows_exchange(v, c);
 #pragma unroll 1
-    for (int k = 0; k < 4; ++k) small_sums(v, pick4(gy, k), rows + (7 + k) * kH, g, c);
+    for (int k = 0; k < 4; ++k) small_sums<true>(v, pick4(gy, k), rows + (7 + k) * kH, t == 0, g, c);
     // gZ_4, and down the chain gZ_l = (W_l^T gZ_{l+1}) silu'(Z_l)
     asm volatile("" ::: "memory");   // W4 is read again, not kept
     forget(z);
@@ -885,7 +907,8 @@ __global__ __launch_bounds__(kTrainThreads) void mlp_train_kernel(MLPTrainArgs a
 #pragma unroll
       for (int j = 0; j < 32; ++j) B[j >> 3][j & 7] = (__bf16)v[j];
       train_stage(sG, row, g, v);
-      small_sums(v, 1.f, rows + (4 + l) * kH, g, c);
+      rows_exchange(v, c);
+      small_sums<false>(v, 1.f, rows + (4 + l) * kH, t == 0, g, c);
       layer_get(Z, l, z);
 #pragma unroll
       for (int j = 0; j < 32; ++j) v[j] = silu(z[j >> 2][j & 3]);
@@ -901,19 +924,20 @@ __global__ __launch_bounds__(kTrainThreads) void mlp_train_kernel(MLPTrainArgs a
       for (int j = 0; j < 32; ++j) v[j] = acc[j >> 2][j & 3] * dsilu(z[j >> 2][j & 3]);
       __syncthreads();   // every wave has read the stages
     }
+    rows_exchange(v, c);
 #pragma unroll 1
-    for (int d = 0; d < 4; ++d) small_sums(v, pick4(f, d), rows + d * kH, g, c);
+    for (int d = 0; d < 4; ++d) small_sums<true>(v, pick4(f, d), rows + d * kH, t == 0, g, c);
   }
-  // the small sums over the block's tiles and waves, the waves' loss and db4
+  // the small sums over the block's waves, the waves' loss and db4
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
   __threadfence_block();
   __syncthreads();
-  const float* rows = a.small_wave + (size_t)blockIdx.x * a.tiles * 8 * 11 * kH;
+  const double* block = a.small_wave + (size_t)blockIdx.x * 8 * 11 * kH;
   double* out = a.small_part + (size_t)blockIdx.x * kSmallRow;
   for (int e = threadIdx.x; e < 11 * kH; e += kTrainThreads) {
     double s = 0.0;
-#pragma unroll 8
-    for (int w = 0; w < 8 * tiles; ++w) s += (double)rows[(size_t)w * 11 * kH + e];
+#pragma unroll
+    for (int w = 0; w < 8; ++w) s += block[(size_t)w * 11 * kH + e];
     out[e] = s;
   }
   if (threadIdx.x < 5) {
@@ -1290,7 +1314,7 @@ int mlp_batch_buffers(Context* c, int64_t tiles, hipStream_t s) {
   M.small_part = nullptr;
   M.bcap = 0;
   BFE_HIP(c, hipMalloc(&M.dwpart, sizeof(float) * 3 * kH * kH * (size_t)tiles));
-  BFE_HIP(c, hipMalloc(&M.small_wave, sizeof(float) * 8 * 11 * kH * (size_t)tiles));
+  BFE_HIP(c, hipMalloc(&M.small_wave, sizeof(double) * 8 * 11 * kH * 256));
   BFE_HIP(c, hipMalloc(&M.small_part, sizeof(double) * kSmallRow * 256));
   M.bcap = tiles;
   return 0;
@@ -1345,12 +1369,13 @@ int mlp_sync(Context* c, hipStream_t s) {
 namespace bfe {
 void mlp_free(Context* c) {
   MLPState& M = c->mlp;
-  for (float** p : {&M.params, &M.grads, &M.m, &M.v, &M.dwpart, &M.small_wave}) {
+  for (float** p : {&M.params, &M.grads, &M.m, &M.v, &M.dwpart}) {
     if (*p) (void)hipFree(*p);
     *p = nullptr;
   }
   if (M.Wp) (void)hipFree(M.Wp);
   if (M.Wt) (void)hipFree(M.Wt);
+  if (M.small_wave) (void)hipFree(M.small_wave);
   if (M.small_part) (void)hipFree(M.small_part);
   M = MLPState();
 }
