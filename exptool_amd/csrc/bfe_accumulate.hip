@@ -1718,10 +1718,6 @@ int eof_dep_prepare(Context* c) {
   return 0;
 }
 
-// beside: another accumulate runs concurrently (selects the deposit kernel).
-// order_out (beside only): receives the particles in cell order as (x, y, z,
-// input index), NULL when they are summed in input order; the masses are then
-// read by index, so the order serves the evaluation as well.
 // bf16 pieces of the potential table for the MFMA mode (once per table set).
 static int eof_mfma_prepare(Context* c, hipStream_t s) {
   if (c->eof_mfmaT) return 0;
@@ -1824,6 +1820,10 @@ static int eof_accumulate_mfma_run(Context* c, const float* x, const float* y, c
   return 0;
 }
 
+// beside: another accumulate runs concurrently (selects the deposit kernel).
+// order_out (beside only): receives the particles in cell order as (x, y, z,
+// input index), NULL when they are summed in input order; the masses are then
+// read by index, so the order serves the evaluation as well.
 static int eof_accumulate_run(Context* c, const float* x, const float* y, const float* z,
                               const float* m, int64_t n, const int64_t* off, int nsnap,
                               double* cos_out, double* sin_out, hipStream_t s,

@@ -395,9 +395,12 @@ extern "C" int bfe_set_tuning(bfe_ctx* h, const char* name, int64_t value) {
   } else if (!strcmp(name, "point_blocks")) {
     if (value < 0 || value > 65535) return set_error(c, BFE_EINVAL, "point_blocks outside [0, 65535]");
     c->point_blocks = value;
-  } else if (!strcmp(name, "split_max") || !strcmp(name, "split_eval_max")) {
-    if (value < 0) return set_error(c, BFE_EINVAL, "%s < 0", name);
-    (name[5] == '_' && name[6] == 'm' ? c->split_max : c->split_eval_max) = value;
+  } else if (!strcmp(name, "split_max")) {
+    if (value < 0) return set_error(c, BFE_EINVAL, "split_max < 0");
+    c->split_max = value;
+  } else if (!strcmp(name, "split_eval_max")) {
+    if (value < 0) return set_error(c, BFE_EINVAL, "split_eval_max < 0");
+    c->split_eval_max = value;
   } else if (!strcmp(name, "kernel_timing")) {
     c->kernel_timing = value != 0;
   } else if (!strcmp(name, "sl_acc_path")) {

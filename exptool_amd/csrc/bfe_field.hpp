@@ -301,10 +301,6 @@ __device__ __forceinline__ SLRadial sl_radial(const SLGeom& g, const SLCell& cel
   return q;
 }
 
-// pcell: the radial cell of r when the caller has located it already.
-// STAGED: node i's force blocks are read from the LDS copy Abase at
-// (i - ibase) * 2 np float4 (a block stages its nodes there); otherwise from
-// the folded table itself.
 // The sums of sl_eval_folded in cell `cell` from its node's blocks: A (2 np
 // float4, in global memory or LDS) and the density block Nd.
 template <bool DENS, typename PA>
@@ -333,6 +329,10 @@ __device__ __forceinline__ void sl_eval_cell(const SLGeom& g, PA A, const float4
   o.den1 = acc[6] * D0;
 }
 
+// pcell: the radial cell of r when the caller has located it already.
+// STAGED: node i's force blocks are read from the LDS copy Abase at
+// (i - ibase) * 2 np float4 (a block stages its nodes there); otherwise from
+// the folded table itself.
 template <bool DENS, bool STAGED = false>
 __device__ __forceinline__ void sl_eval_folded(const SLGeom& g, const float* __restrict__ F,
                                                int L, double r, double costh, double c1,

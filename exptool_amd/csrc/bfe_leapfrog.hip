@@ -355,8 +355,9 @@ __device__ __forceinline__ void rk4_frame(const RK4Args& a, float px, float py, 
   fy = fmaf(s, fmaf(w2, py, -(tw * ux)), fy);
 }
 
-// Three waves per SIMD (168 registers, about 300 B per lane spilled):
-// 1.94e9 against 1.73e9 steps/s at the two waves 255 registers allowed.
+// Three waves per SIMD: 1.94e9 against 1.73e9 steps/s at the two waves 255 registers
+// allowed, both before the build without machine LICM (159 registers, nothing
+// spilled).
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void rk4_chunk_kernel(
     float* __restrict__ x, float* __restrict__ y, float* __restrict__ z, float* __restrict__ vx,
     float* __restrict__ vy, float* __restrict__ vz, const int* __restrict__ perm, FieldTables T,

@@ -64,7 +64,7 @@ constexpr int kInfPts = kWaveTile * kBlockInf / 64;   // points per block
 // activations (192 registers): eight waves per block, two per SIMD, so that one
 // wave's activations cover the other's products.  Inference of 1M points 667 ->
 // 458 us against four waves (no spills; 422 with the point work once per point);
-// the integrator, which holds its state as well and spills 500 B a lane, 55.7 ->
+// the integrator, which holds its state as well and spills 39 registers, 55.7 ->
 // 37.5 ms per 100 steps of 1M orbits.  Few orbits take four waves, one per SIMD, with
 // nothing spilled (mlp_leap_launch).
 constexpr int kBlockGrad = 512;

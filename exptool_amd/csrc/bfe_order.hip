@@ -285,7 +285,7 @@ __device__ __forceinline__ uint32_t block_scan_incl(uint32_t v, uint32_t* wsum) 
 
 // Items [t0, end) of tile b: b kSortThreads IPT and on, or the bounds tb[2b], tb[2b + 1]
 // (at most kSortThreads IPT items) of a segmented sort.  Slot i of thread (w, l)
-// holds item t0 + (w kSortIPT + i) 64 + l.
+// holds item t0 + (w IPT + i) 64 + l.
 struct TileRange {
   int64_t t0, end;
 };
