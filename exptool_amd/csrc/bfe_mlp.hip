@@ -552,9 +552,9 @@ __global__ __launch_bounds__(kBlockGrad) void mlp_fwd_grad_kernel(MLPKArgs a, in
 // over tiles.  b0..b3, W0 and W4 gradients: products and sums over points in
 // float64 throughout (reduce_rows).
 // Measured for 65 536 points: 910 us as separate forward, backward, weight
-// gradient and reduction kernels (72 + 200 + 337 + 63 + 197 + 41), 90 us for
-// this one and 16 for the reduction (100 MB of partial sums); about half of a
-// tile's 37 us is vector-ALU issue (SiLUs and the sums over lanes), the rest
+// gradient and reduction kernels (72 + 200 + 337 + 63 + 197 + 41), 86 us for
+// this one and 16 for the reduction (100 MB of partial sums; 82 with float32 small
+// sums); about half of a tile's 41 us is vector-ALU issue (SiLUs and the sums over lanes), the rest
 // waits of two waves per SIMD at 256 registers.
 constexpr int kTrainThreads = 512;
 constexpr int kTrainPts = 128;
