@@ -698,12 +698,14 @@ __global__ __launch_bounds__(256) void eof_points_kernel(
 // nodes: when their force blocks fit in kStageFloat4, the block copies them
 // to LDS and the SL sums read them there.  pts2 (may be NULL): a second set of n2
 // points in its own cell order, numbered after the first.  Bound by vector ALU
-// issue (77 % busy) and address units (71 %) where the chip is full: 2M points 149
-// us with WAVES = 4 a SIMD (128 registers, 20 B spilled), 155 with three (144);
+// issue (77 % busy) and address units (71 %) where the chip is full: 2M points 131
+// us with FOUR waves a SIMD (128 registers, 20 B spilled), 139 with three (144);
 // fewer points by one wave's own latency, where three are faster
-// (eval_four_waves).
-template <int WAVES>
-__global__ __launch_bounds__(256, WAVES) void field_eval_kernel(
+// (eval_four_waves).  The three-wave build states no number of waves: told three,
+// the compiler takes as many registers in another order of the same instructions,
+// 5 to 9 % slower (200 000 points 33.4 us, untold 31.3; 400 000 47.1 and 43.9).
+template <bool FOUR>
+__global__ __launch_bounds__(256, FOUR ? 4 : 1) void field_eval_kernel(
     const float* __restrict__ px, const float* __restrict__ py, const float* __restrict__ pz,
     int64_t n, const float4* __restrict__ pts, const float4* __restrict__ pts2, int64_t n2,
     FieldTables T, float* fx, float* fy, float* fz, float* pot, float* comp,
@@ -1109,8 +1111,8 @@ static int field_eval_run(Context* c, const FieldTables& T, const float* x, cons
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, s, x, y, z, pts2 ? n1 : n, pts, pts2, n - n1, T,
                        fx, fy, fz, pot, comp, quad, n);
   };
-  if (eval_four_waves(n, (T.flags & BFE_COMPAT_SL_COS_L) != 0)) go(field_eval_kernel<4>);
-  else go(field_eval_kernel<3>);
+  if (eval_four_waves(n, (T.flags & BFE_COMPAT_SL_COS_L) != 0)) go(field_eval_kernel<true>);
+  else go(field_eval_kernel<false>);
   timer_end(c, "field_eval", s);
   BFE_HIP(c, hipGetLastError());
   if (quad) {

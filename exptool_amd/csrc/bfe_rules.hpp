@@ -9,13 +9,14 @@ namespace bfe {
 
 // Builds of field_eval_kernel: 144 registers (three waves a SIMD) or 128 with
 // 20 B spilled (four).  The second pays only where a fourth wave has work, from
-// about eight blocks of 256 a CU.  Three / four, in cell order: 262 144 points
-// 63.5 / 65.8 us at lmax = mmax = 6 and 90.2 / 95.0 at 12, 500 000 90.0 / 91.6 and
-// 128.7 / 130.5, 800 000 115.6 / 113.9 and 173.7 / 168.3, 2M 218 / 214 and 342 /
-// 320; in input order 65 536 points 22.6 / 24.0 and 47.9 / 56.6.  With cos(l phi)
-// factors from three blocks a CU: 196 608 points on, (10, 6) 200 000 84.0 / 78.6, 500 000
-// 128 / 122; 65 536 52.7 / 51.3 and (12, 12) 75.6 / 78.4.
-constexpr int64_t kEvalFourWaves = 524288, kEvalFourWavesCosL = 196608;
+// about nine blocks of 256 a CU on.  Kernel us, three / four, in cell order at
+// (lmax, mmax): 262 144 points (4, 4) 25.6 / 26.8, (6, 6) 32.6 / 34.9, (12, 12) 60.4 /
+// 64.6; 524 288 38.6 / 39.6, 49.5 / 50.7, 88.2 / 90.8; 600 000 43.8 / 43.5, 55.8 /
+// 56.5, 102.5 / 102.6; 800 000 53.4 / 51.5, 67.3 / 66.6, 125.8 / 121.8; 2M 108 / 102,
+// 139 / 131, 260 / 244.  ((10, 6) and (2, 2) cross at 400 000: 58.3 / 56.6 there.)
+// With cos(l phi) factors from six blocks a CU on: (10, 6) 300 000 61.6 / 63.5,
+// 400 000 78.4 / 76.3, 600 000 102 / 98; (12, 12) 84.2 / 90.4, 106.7 / 106.0, 137 / 134.
+constexpr int64_t kEvalFourWaves = 589824, kEvalFourWavesCosL = 393216;
 inline bool eval_four_waves(int64_t n, bool cos_l) {
   return n >= (cos_l ? kEvalFourWavesCosL : kEvalFourWaves);
 }

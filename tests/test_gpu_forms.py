@@ -10,10 +10,10 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("ordered", [False, True])
 def test_three_and_four_wave_builds_agree(system, ordered):  # noqa: F811
-    """524 288 points and more take the four-wave build, slices of them the
+    """589 824 points and more take the four-wave build, slices of them the
     three-wave one; ragged last block."""
     import torch
-    p = _points(524_288 + 77, 8)
+    p = _points(589_824 + 77, 8)
     system.set_tuning("split_eval_max", 0)
     system.set_tuning("order_min", 1 if ordered else 1 << 40)
     whole = system.field_forces(*p.unbind(0), rotpos=0.4)

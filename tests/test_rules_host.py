@@ -60,12 +60,12 @@ def rule(tmp_path_factory):
 def test_four_waves_only_where_the_chip_is_full(rule):
     """Up to three blocks of 256 points a CU (256 CUs) are resident with three
     waves a SIMD, so the four-wave build has nothing to give there; with
-    cos(l phi) factors it gives from there on, without from 524 288 points."""
-    ns = [1, 256, 65_536, 131_072, 196_608, 262_144, 500_000, 1_000_000, 2_000_000]
+    cos(l phi) factors it gives from six, without from nine."""
+    ns = [1, 256, 65_536, 131_072, 196_608, 262_144, 393_216, 500_000, 589_823, 600_000, 2_000_000]
     got = [bool(v[0]) for v in rule("eval_four_waves", [(n,) for n in ns])]
-    assert got == [False] * 7 + [True] * 2
+    assert got == [False] * 9 + [True] * 2
     got = [bool(v[0]) for v in rule("eval_four_waves", [(n, 1) for n in ns])]
-    assert got == [False] * 4 + [True] * 5
+    assert got == [False] * 6 + [True] * 5
 
 
 # us of the one-lane and the split integrators on MI355X at (lmax, mmax), orbits
