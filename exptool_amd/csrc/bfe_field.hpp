@@ -505,14 +505,15 @@ struct FieldGeom {
 __device__ __forceinline__ FieldGeom field_geom(const FieldTables& T, double x, double y,
                                                 double z) {
   FieldGeom q;
-  q.r2 = sqrt(fma(x, x, y * y)) + 1.e-15;
+  const double rho = sqrt(fma(x, x, y * y));
+  q.r2 = rho + 1.e-15;
   q.r3 = sqrt(fma(q.r2, q.r2, z * z)) + 1.e-15;
   // reciprocals once; the force combination multiplies by them
   q.ir2 = 1.0 / q.r2;
   q.ir3 = 1.0 / q.r3;
   q.costh = z * q.ir3;
   double c0, s0;
-  planar_angle(x, y, c0, s0);
+  planar_angle(x, y, rho, c0, s0);
   q.c1 = fma(c0, T.crot, -(s0 * T.srot));
   q.s1 = fma(s0, T.crot, c0 * T.srot);
   return q;

@@ -106,10 +106,10 @@ BFE_HD double z_to_y(double z, double ihscale) {
   return (z / (fabs(z) + 1.e-8)) * asinh_nonneg(fabs(z * ihscale));
 }
 
-// Planar angle of (x, y) as cos/sin, with atan2 semantics: the zero vector
-// goes through atan2 itself so that signed zeros behave as in numpy.arctan2.
-BFE_HD void planar_angle(double x, double y, double& c, double& s) {
-  double rho = sqrt(x * x + y * y);
+// Planar angle of (x, y), rho = |(x, y)|, as cos/sin, with atan2 semantics: the
+// zero vector goes through atan2 itself so that signed zeros behave as in
+// numpy.arctan2.
+BFE_HD void planar_angle(double x, double y, double rho, double& c, double& s) {
   if (rho > 0.0) {
     const double irho = 1.0 / rho;
     c = x * irho;
@@ -119,6 +119,9 @@ BFE_HD void planar_angle(double x, double y, double& c, double& s) {
     c = cos(ph);
     s = sin(ph);
   }
+}
+BFE_HD void planar_angle(double x, double y, double& c, double& s) {
+  planar_angle(x, y, sqrt(x * x + y * y), c, s);
 }
 
 // cos(m phi), sin(m phi) for m = 0..mmax by the Chebyshev recurrence
