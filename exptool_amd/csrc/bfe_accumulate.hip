@@ -1820,6 +1820,18 @@ static int eof_accumulate_mfma_run(Context* c, const float* x, const float* y, c
   return 0;
 }
 
+static size_t eof_dep_lds(const Context* c) {
+  return std::max((size_t)4 * ((2 * c->mmax + 1) * kDepStride + kDepExtra) * sizeof(float),
+                  (size_t)4 * c->eof_K * sizeof(double));
+}
+
+// Whether n disc particles of one snapshot are summed in cell order.
+bool eof_cell_ordered(const Context* c, int64_t n) {
+  return n > 0 && n >= c->order_min &&
+         dep_shape(2 * c->mmax + 1, c->norder, kEofShapes, kEofDepShapes, c->eof_dep_shape).ppt > 0 &&
+         eof_dep_lds(c) <= 64 * 1024;
+}
+
 // beside: another accumulate runs concurrently (selects the deposit kernel).
 // order_out (beside only): receives the particles in cell order as (x, y, z,
 // input index), NULL when they are summed in input order; the masses are then
@@ -1831,10 +1843,9 @@ static int eof_accumulate_run(Context* c, const float* x, const float* y, const 
   const int K = c->eof_K;
   // cell-ordered form: (2 mmax + 1) rows x chunks of radial orders per lane,
   // LDS for the per-wave weights and the float64 wave reduction
-  const size_t dlds = std::max((size_t)4 * ((2 * c->mmax + 1) * kDepStride + kDepExtra) * sizeof(float),
-                               (size_t)4 * K * sizeof(double));
+  const size_t dlds = eof_dep_lds(c);
   const DepShape dsh = dep_shape(2 * c->mmax + 1, c->norder, kEofShapes, kEofDepShapes, c->eof_dep_shape);
-  const bool ordered = n >= c->order_min && n > 0 && dsh.ppt > 0 && dlds <= 64 * 1024;
+  const bool ordered = eof_cell_ordered(c, n);
   AccPlan P = off ? plan_batch(c->eof_acc_blocks, c->eof_seg_tiles, off, nsnap, kTile)
                   : ordered ? plan_single(c->eof_acc_blocks, n, kTile)
                             : plan_input_order(c->eof_acc_blocks, n);
@@ -1888,6 +1899,22 @@ static int eof_accumulate_run(Context* c, const float* x, const float* y, const 
   return 0;
 }
 
+static size_t sl_dep_lds(int R, int K) {
+  return std::max((size_t)4 * sl_dep_rows(R) * kDepStride * sizeof(float), (size_t)4 * K * sizeof(double));
+}
+static bool sl_mfma_ok(const Context* c) {
+  return c->lmax <= 7 && (c->lmax + 1) * ((c->nmax + 15) / 16) <= 4 * kMSlots;
+}
+
+// Whether n halo particles of one snapshot are summed in cell order.
+bool sl_cell_ordered(const Context* c, int64_t n, uint32_t flags) {
+  const int R = (c->lmax + 1) * (c->lmax + 1);
+  if (sl_mfma_ok(c) && ((flags & BFE_ACC_BF16) || c->sl_acc_path == 1)) return false;
+  return n > 0 && n >= c->order_min &&
+         dep_shape(R, c->nmax, kSlShapes, kSlDepShapes, c->sl_dep_shape).ppt > 0 &&
+         sl_dep_lds(R, R * c->nmax) <= 64 * 1024;
+}
+
 // beside: another accumulate runs concurrently (selects the deposit kernel).
 // order_out (beside only): receives the particles in cell order as (x, y, z,
 // input index), NULL when they are summed in input order; the masses are then
@@ -1903,12 +1930,11 @@ static int sl_accumulate_run(Context* c, const float* x, const float* y, const f
   const size_t lds = ((size_t)R * (kSLTile + 1) + (size_t)kSLTile * LN + 3 * kSLTile) * 4;
   if (lds > 64 * 1024) return set_error(c, BFE_ELIMIT, "sl_accumulate: LDS %zu B > 64 KiB", lds);
   const DepShape dsh = dep_shape(R, c->nmax, kSlShapes, kSlDepShapes, c->sl_dep_shape);
-  const size_t dlds = std::max((size_t)4 * sl_dep_rows(R) * kDepStride * sizeof(float),
-                               (size_t)4 * K * sizeof(double));
+  const size_t dlds = sl_dep_lds(R, K);
   const bool bf16_mode = (flags & BFE_ACC_BF16) != 0;
-  const bool mfma_ok = c->lmax <= 7 && (c->lmax + 1) * ((c->nmax + 15) / 16) <= 4 * kMSlots;
+  const bool mfma_ok = sl_mfma_ok(c);
   const bool mfma = n > 0 && mfma_ok && (bf16_mode || c->sl_acc_path == 1);
-  const bool ordered = !mfma && n >= c->order_min && n > 0 && dsh.ppt > 0 && dlds <= 64 * 1024;
+  const bool ordered = sl_cell_ordered(c, n, flags);
   AccPlan P = off ? plan_batch(c->sl_acc_blocks, c->sl_seg_tiles, off, nsnap, kSLTile)
                   : plan_single(beside ? c->sl_acc_blocks_beside : c->sl_acc_blocks, n, kSLTile);
   // cell-ordered segments of up to four tiles leave a wave at most one tile,
@@ -2105,14 +2131,14 @@ static int eof_accumulate_noalloc_run(Context* c, const float* x, const float* y
 int eof_accumulate_one(Context* c, const float* x, const float* y, const float* z,
                        const float* m, int64_t n, double* cos_out, double* sin_out, hipStream_t s,
                        const float4** order_out) {
-  *order_out = nullptr;
+  if (order_out) *order_out = nullptr;
   return eof_accumulate_run(c, x, y, z, m, n, nullptr, 1, cos_out, sin_out, s, true, order_out);
 }
 
 int sl_accumulate_one(Context* c, const float* x, const float* y, const float* z, const float* m,
                       int64_t n, uint32_t flags, double* coef_out, hipStream_t s,
                       const float4** order_out) {
-  *order_out = nullptr;
+  if (order_out) *order_out = nullptr;
   return sl_accumulate_run(c, x, y, z, m, n, nullptr, 1, flags, coef_out, s, true, order_out);
 }
 

@@ -1240,22 +1240,45 @@ extern "C" int bfe_forces_disc_halo(bfe_ctx* h, const float* dx, const float* dy
     rc = fork_begin(c, s, &s1);
     if (rc) return rc;
     const float4 *dpts = nullptr, *hpts = nullptr;
-    // disc: accumulate and fold on the caller's stream, the longer branch first
-    int r0 = eof_accumulate_one(c, dx, dy, dz, dm, nd, cos_out, sin_out, s, &dpts);
-    if (!r0) r0 = eof_fold(c, 1, cos_out, sin_out, mm, nn, 0, 1 << 30, no_odd,
-                           (field_flags & BFE_COMPAT_EOF_MASK) != 0, false, s);
-    // halo: accumulate and fold on the first internal stream
-    swap_work(c);
-    int r1 = sl_accumulate_one(c, hx, hy, hz, hm, nh, acc_flags, coef_out, s1, &hpts);
-    swap_work(c);
-    if (!r1) r1 = sl_fold(c, 1, coef_out, halofac, ll, hn, -(1 << 30), 1 << 30, no_odd, s1);
-    if (dpts && hpts) {
-      // both orders are there: the disc's EOF cells (few SL nodes and EOF cells a
-      // block) and the halo's evaluation cells
+    int r0 = 0, r1 = 0;
+    // disc: accumulate and fold on the caller's stream
+    auto disc = [&](const float4** order) {
+      r0 = eof_accumulate_one(c, dx, dy, dz, dm, nd, cos_out, sin_out, s, order);
+      if (!r0) r0 = eof_fold(c, 1, cos_out, sin_out, mm, nn, 0, 1 << 30, no_odd,
+                             (field_flags & BFE_COMPAT_EOF_MASK) != 0, false, s);
+    };
+    // halo: accumulate and fold on the first internal stream, behind the sort of the
+    // points where it is asked for
+    auto halo = [&](bool sort, const float4** order) {
+      swap_work(c);
+      if (sort) r1 = order_points2(c, G, dx, dy, dz, nd, hx, hy, hz, nh, s1, &pts);
+      if (!r1) r1 = sl_accumulate_one(c, hx, hy, hz, hm, nh, acc_flags, coef_out, s1, order);
+      swap_work(c);
+      if (!r1) r1 = sl_fold(c, 1, coef_out, halofac, ll, hn, -(1 << 30), 1 << 30, no_odd, s1);
+    };
+    const bool halo_sorts = sl_cell_ordered(c, nh, acc_flags);
+    if (!split && halo_sorts && eof_cell_ordered(c, nd)) {
+      // both orders serve the evaluation: the disc's EOF cells (few SL nodes and EOF
+      // cells a block) and the halo's evaluation cells.  The disc's branch is the
+      // longer and goes first
+      disc(&dpts);
+      halo(false, &hpts);
       pts = dpts;
       pts2 = hpts;
-    } else if (!r0 && n > 0 && !split) {
-      r0 = order_points2(c, G, dx, dy, dz, nd, hx, hy, hz, nh, s, &pts);
+    } else if (halo_sorts || split || nd < nh || n == 0) {
+      halo(false, nullptr);
+      disc(nullptr);
+      if (!r0 && n > 0 && !split) r0 = order_points2(c, G, dx, dy, dz, nd, hx, hy, hz, nh, s, &pts);
+    } else {
+      // The points' order takes the buffers that a halo summed in input order leaves
+      // free, on its stream: that kernel's two blocks a CU (216 registers) leave the
+      // disc's sort and deposit little room, so the disc's branch is the longer unless
+      // the halo has more particles.  Order behind the disc's fold / before the halo's
+      // sums, us at disc | halo particles: (6, 6) 300 000 | 30 000 214 / 169; (8, 8)
+      // 300 000 | 300 000 364 / 352, 300 000 | 150 000 283 / 262; (10, 6) 300 000 |
+      // 300 000 367 / 352, 30 000 | 300 000 287 / 311.
+      halo(true, nullptr);
+      disc(nullptr);
     }
     rc = fork_end(c, s);
     if (r0 || r1 || rc) return r0 ? r0 : (r1 ? r1 : rc);

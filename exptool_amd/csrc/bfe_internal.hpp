@@ -294,15 +294,17 @@ int order_particles(Context* c, int kind, const float* x, const float* y, const 
 // Single-snapshot accumulates (bfe_eof_accumulate / bfe_sl_accumulate
 // without the argument checks), enqueued on s with the current buffer set.
 // Both are for callers that run them side by side (they take the deposit
-// kernels sized for sharing the GPU).  order_out receives the particles in
-// cell order as (x, y, z, input index) in the order buffer, NULL when they were
-// summed in input order.
+// kernels sized for sharing the GPU).  order_out (may be NULL) receives the
+// particles in cell order as (x, y, z, input index) in the order buffer, NULL when
+// they were summed in input order.
 int eof_accumulate_one(Context* c, const float* x, const float* y, const float* z,
                        const float* m, int64_t n, double* cos_out, double* sin_out, hipStream_t s,
                        const float4** order_out);
 int sl_accumulate_one(Context* c, const float* x, const float* y, const float* z, const float* m,
                       int64_t n, uint32_t flags, double* coef_out, hipStream_t s,
                       const float4** order_out);
+bool eof_cell_ordered(const Context* c, int64_t n);
+bool sl_cell_ordered(const Context* c, int64_t n, uint32_t flags);
 int accumulate_both_small(Context* c, const float* dx, const float* dy, const float* dz,
                           const float* dm, int64_t nd, const float* hx, const float* hy,
                           const float* hz, const float* hm, int64_t nh, uint32_t flags,

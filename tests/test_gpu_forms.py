@@ -49,6 +49,37 @@ def test_default_form_agrees_with_input_order(system, n):  # noqa: F811
             _same(u, v)
 
 
+@pytest.mark.parametrize("nd,nh", [(9001, 2500), (9001, 9001), (9001, 9000), (2500, 9001), (5001, 0)])
+def test_fused_forces_of_a_halo_in_input_order(system, nd, nh):  # noqa: F811
+    """The fused call with the disc in cell order and a halo that is not (few
+    particles, or the matrix-product form), one side as large as the other or not:
+    the coefficients of the accumulates and the forces in input order, every time."""
+    import torch
+    p = _points(nd + nh, 5)
+    m = torch.linspace(0.5, 1.5, nd + nh, dtype=torch.float32, device="cuda") / (nd + nh)
+    d, h = ([q[k].contiguous() for q in (*p.unbind(0), m)] for k in (slice(0, nd), slice(nd, None)))
+    system.set_tuning("split_eval_max", 0)
+    try:
+        for path in (0, 1):
+            if path and system.sl["lmax"] > 7:
+                continue
+            system.set_tuning("sl_acc_path", path)
+            for _ in range(3):
+                system.set_tuning("order_min", 5000)
+                out = system.forces_disc_halo(d, h, rotpos=0.4, components=True)
+                acc = system.accumulate_disc_halo(d, h)
+                for a, b in zip((out["cos"], out["sin"], out["coef"]), acc):
+                    _same(a, b)
+                system.set_tuning("order_min", 1 << 40)
+                ref = system.field_forces(*p.unbind(0), rotpos=0.4, components=True)
+                for k, v in zip(("fx", "fy", "fz", "pot", "comp"), ref):
+                    _same(out[k], v)
+    finally:
+        system.set_tuning("sl_acc_path", 0)
+        system.set_tuning("split_eval_max", 131072)
+        system.set_tuning("order_min", 65536)
+
+
 @pytest.mark.parametrize("density", [False, True])
 @pytest.mark.parametrize("lmax,numr", [(3, 1638), (3, 1639), (9, 601), (16, 108)])
 def test_sl_fold_of_one_and_two_nodes(lmax, numr, density):
