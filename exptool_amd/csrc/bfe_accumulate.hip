@@ -264,7 +264,7 @@ __global__ void fill_f64_kernel(double* __restrict__ a, int64_t n) {
 // ---------------------------------------------------------------------------
 // SL accumulate
 // ---------------------------------------------------------------------------
-template <int OPT>
+template <int OPT, int UNROLL = 8>
 __device__ __forceinline__ void sl_accumulate_block(
     float* smem, const float* __restrict__ px, const float* __restrict__ py,
     const float* __restrict__ pz, const float* __restrict__ pm, const Segments& S, const SLGeom& g,
@@ -362,7 +362,7 @@ __device__ __forceinline__ void sl_accumulate_block(
     }
     __syncthreads();
     // radial functions phi_ln(r_p) for the tile, coalesced over ln
-#pragma unroll 8
+#pragma unroll UNROLL
     for (int idx = tid; idx < kSLTile * LN; idx += 256) {
       const int q = idx / LN, ln = idx - q * LN;
       const size_t i = (size_t)s_i[q];
@@ -371,7 +371,7 @@ __device__ __forceinline__ void sl_accumulate_block(
     __syncthreads();
     const int64_t left = s1 - t0;
     const int np = left < kSLTile ? (int)left : kSLTile;
-#pragma unroll 8
+#pragma unroll UNROLL
     for (int q = 0; q < np; ++q) {
 #pragma unroll
       for (int o = 0; o < OPT; ++o) acc[o] = fmaf(s_Y[yrow[o] + q], s_phi[q * LN + prow[o]], acc[o]);
@@ -398,13 +398,15 @@ __device__ __forceinline__ void sl_accumulate_block(
   }
 }
 
-template <int OPT>
+// Loads in flight a lane against blocks a CU: UNROLL 8 takes 216 registers at OPT 4
+// (two blocks a CU), 4 takes 167 (three, where their LDS fits).
+template <int OPT, int UNROLL = 8>
 __global__ __launch_bounds__(256) void sl_accumulate_kernel(
     const float* __restrict__ px, const float* __restrict__ py, const float* __restrict__ pz,
     const float* __restrict__ pm, Segments S, SLGeom g, const float* __restrict__ E,
     const double* __restrict__ lmc, int no_odd, double* __restrict__ partials) {
   extern __shared__ float smem[];
-  sl_accumulate_block<OPT>(smem, px, py, pz, pm, S, g, E, lmc, no_odd, partials, blockIdx.x, gridDim.x);
+  sl_accumulate_block<OPT, UNROLL>(smem, px, py, pz, pm, S, g, E, lmc, no_odd, partials, blockIdx.x, gridDim.x);
 }
 
 // The input-order accumulates of a disc and a halo in one launch, the disc's
@@ -2012,6 +2014,8 @@ static int sl_accumulate_run(Context* c, const float* x, const float* y, const f
     hipLaunchKernelGGL(sl_accumulate_kernel<1>, dim3(P.grid), dim3(256), lds, s, x, y, z, m, P.S, g, c->sl_e32, c->sl_lmc, no_odd, partials);
   } else if (opt == 2) {
     hipLaunchKernelGGL(sl_accumulate_kernel<2>, dim3(P.grid), dim3(256), lds, s, x, y, z, m, P.S, g, c->sl_e32, c->sl_lmc, no_odd, partials);
+  } else if (!beside && sl_three_blocks(P.grid, lds)) {
+    hipLaunchKernelGGL((sl_accumulate_kernel<4, 4>), dim3(P.grid), dim3(256), lds, s, x, y, z, m, P.S, g, c->sl_e32, c->sl_lmc, no_odd, partials);
   } else {
     hipLaunchKernelGGL(sl_accumulate_kernel<4>, dim3(P.grid), dim3(256), lds, s, x, y, z, m, P.S, g, c->sl_e32, c->sl_lmc, no_odd, partials);
   }

@@ -98,6 +98,13 @@ inline bool eval_split_two(int64_t n, int lmax, int mmax, bool split_ok, int64_t
   return n <= (split_fixed(lmax, mmax) ? 114688 : 49152);
 }
 
+// Whether an input-order halo sum that has the GPU to itself takes the build of three
+// blocks a CU: from more than two blocks a CU on, where three fit in the LDS.  us with
+// two / three at (lmax, mmax): (6, 6) 30 000 particles (469 blocks) 25.4 / 26.3, 60 000
+// 45.4 / 43.7; (8, 8) 60 000 45.6 / 43.7, 300 000 178.5 / 151.2, 1M 482 / 402; (10, 6),
+// 54 KiB a block, 1M 521 / 532.
+inline bool sl_three_blocks(int64_t blocks, uint64_t lds) { return blocks > 2 * 256 && 3 * lds <= 160 * 1024; }
+
 // Nodes a group of four lanes folds in the whole-table SL fold: one until the lanes
 // of two a group fill 128 blocks, then two, which share rows.  Whole calls, one / two,
 // us at lmax, numr (nmax 20): 0, 2000 7.8 / 8.5; 2, 2000 10.3 / 11.0; 4, 1000 (30 000

@@ -80,6 +80,24 @@ def test_fused_forces_of_a_halo_in_input_order(system, nd, nh):  # noqa: F811
         system.set_tuning("order_min", 65536)
 
 
+@pytest.mark.parametrize("n", [32_769, 40_003])
+def test_halo_sums_of_two_and_three_blocks_a_unit(n):
+    """A halo in input order of more than 512 tiles, with the device to itself and
+    beside a disc: the same segments, the same bits."""
+    import torch
+    from exptool_amd.bfe import BFESystem
+    from exptool_amd.utils import workloads as W
+    st, et = W.disc_halo_tables(seed=2, n_eof_sample=4000, lmax_s=10, nmax_s=8,
+                                eof=dict(mmax=2, norder=4, numx=32, numy=16), sl=dict(lmax=8, nmax=12, numr=300))
+    s = BFESystem(sl=st, eof=et)
+    p = _points(n, 9)
+    m = torch.linspace(0.5, 1.5, n, dtype=torch.float32, device="cuda") / n
+    h = [q.contiguous() for q in (*p.unbind(0), m)]
+    s.set_tuning("order_min", 1 << 40)
+    alone = s.sl_accumulate(*h)
+    _same(alone, s.accumulate_disc_halo([q[:70] for q in h], h)[2])
+
+
 @pytest.mark.parametrize("density", [False, True])
 @pytest.mark.parametrize("lmax,numr", [(3, 1638), (3, 1639), (9, 601), (16, 108)])
 def test_sl_fold_of_one_and_two_nodes(lmax, numr, density):

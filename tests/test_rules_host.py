@@ -26,6 +26,7 @@ int main() {
     else if (!std::strcmp(f, "eval_split_two"))
       std::printf("%d\n", (int)bfe::eval_split_two(a[0], a[1], a[2], a[3] != 0, a[4], a[5]));
     else if (!std::strcmp(f, "sl_fold_rows")) std::printf("%d\n", bfe::sl_fold_rows(a[0], a[1]));
+    else if (!std::strcmp(f, "sl_three_blocks")) std::printf("%d\n", (int)bfe::sl_three_blocks(a[0], a[1]));
     else if (!std::strcmp(f, "mlp_grad_launch")) {
       const bfe::GradLaunch g = bfe::mlp_grad_launch(a[0]);
       std::printf("%d %d %d\n", g.waves, g.per, g.blocks);
@@ -148,6 +149,17 @@ SL_FOLD = [(300, 0, 7.6, 8.3), (300, 8, 21.1, 21.7), (1000, 1, 8.9, 9.6), (1000,
 def test_sl_fold_shares_rows_where_it_is_the_faster(rule):
     for (numr, lmax, *us), (rows,) in zip(SL_FOLD, rule("sl_fold_rows", [v[:2] for v in SL_FOLD])):
         assert us[rows - 1] == min(us), (numr, lmax, rows)
+
+
+# (particles, LDS bytes a block, us with two blocks a CU, us with three)
+SL_ALONE = [(30_000, 49_284, 25.4, 26.3), (60_000, 49_284, 45.4, 43.7), (60_000, 49_476, 45.6, 43.7),
+            (300_000, 49_476, 178.5, 151.2), (1_000_000, 49_476, 481.6, 401.6), (150_000, 54_756, 101.4, 104.1),
+            (1_000_000, 54_756, 521.0, 531.9)]
+
+
+def test_halo_sums_take_three_blocks_where_they_are_the_faster(rule):
+    for (n, lds, *us), (three,) in zip(SL_ALONE, rule("sl_three_blocks", [(-(-n // 64), lds) for n, lds, *_ in SL_ALONE])):
+        assert us[three] == min(us), (n, lds, three)
 
 
 def test_surrogate_inference_fills_the_device(rule):
